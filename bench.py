@@ -591,15 +591,11 @@ def main() -> None:
     gms, gn, gwork = kern["gemm_bx"]
     avg_ms = gms / max(gn, 1)
     if all(min(s[-2:]) <= 64 for s in orth_shapes) and pdtype == torch.bfloat16:
-        # iterates of at most 64 rows run in short.hip: the B X launch streams X in and X'
-        # out (bf16, 4 m n bytes per matrix), HBM-bound; it also forms the next Gram
-        # partials from registers. With the apply fused, the last of the 5 iterations is the
-        # gemm_bx_apply launch (X and the parameters in, the parameters out)
-        plain_iters = 5 - (1 if apply_fused else 0)
-        bx_bytes = sum(plain_iters * 4 * (math.prod(s[:-2]) if len(s) > 2 else 1) * min(s[-2:])
-                       * max(s[-2:]) for s in orth_shapes) * args.steps / max(gn, 1)
-        achieved = bx_bytes / (avg_ms * 1e-3) / 1e9
-        traffic, traffic_src = _measured_traffic("short_bx_kernel<-1>", args.config, args.lp)
+        # iterates of at most 64 rows run in short.hip, HBM-bound: a plain B X launch streams
+        # X in and X' out (bf16, 4 B per element), the gemm_bx_apply launch X and the
+        # parameters in and the parameters out. From 65536 columns on the iterations run on
+        # the Gram matrix and the only product with X is the last one, here with the apply
+        launch, name, per_elem = "gemm_bx", "short_bx_kernel<-1>", 4
         if apply_fused:
             ams, an, _ = kern["gemm_bx_apply"]
             abytes = (2 + 2 * pdtype.itemsize) * numel * args.steps
@@ -607,9 +603,16 @@ def main() -> None:
                 bytes_per_elem=2 + 2 * pdtype.itemsize,
                 gbs=round(abytes / (ams * 1e-3) / 1e9, 1),
                 gbs_frac=round(abytes / (ams * 1e-3) / 1e9 / PEAK_HBM_GBS, 4))
+            if gn == 0:
+                launch, name, per_elem = "gemm_bx_apply", "short_bx_kernel<1, true>", 2 + 2 * pdtype.itemsize
+        lms, ln, _ = kern[launch]
+        avg_ms = lms / max(ln, 1)
+        bx_bytes = per_elem * numel  # one bucket: each launch covers every element
+        achieved = bx_bytes / (avg_ms * 1e-3) / 1e9
+        traffic, traffic_src = _measured_traffic(name, args.config, args.lp)
         roofline = {
             "bound": "hbm",
-            "kernel": "short_bx_kernel<-1> (X' = a X + B X, 64-row iterate)",
+            "kernel": f"{name} (the product with the 64-row iterate)",
             "achieved": round(achieved, 1),
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",

@@ -67,9 +67,12 @@ int muon_launch_short_poly(const OrthLayout& L, float* part, void* bm, int64_t b
 int muon_launch_short_bx(const OrthLayout& L, const void* x, void* xo, const void* bm,
                          float* part, int64_t batch, float alpha, float beta, const float* scale,
                          int first, int gram, hipStream_t s);
-int muon_launch_short_bx_apply(const OrthLayout& L, const void* x, const void* bm,
+int muon_launch_short_bx_apply(const OrthLayout& L, const void* x, const void* bm, float* part,
                                int64_t batch, float alpha, float beta, const float* scale,
                                int first, const MuonApply& ap, hipStream_t s);
+int muon_short_gspace_ok(const OrthLayout& L, const double* coeffs, int steps);
+int muon_launch_short_gspace(const OrthLayout& L, float* part, int64_t batch, const double* coeffs,
+                             int steps, float prescale, float eps, float* scale, hipStream_t s);
 
 enum { MODE_GEMM = 0, MODE_SYRK = 1 };
 
@@ -406,8 +409,10 @@ static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch
   OrthLayout L = muon_orth_layout(ws_dtype, ws_batch, rows, cols);
   hipStream_t s = (hipStream_t)stream;
   char* w = (char*)ws;
-  int rc;
-  {
+  int rc = MUON_OK;
+  // (the iteration on the Gram matrix takes the norm from its trace)
+  const bool gspace = muon_short_gspace_ok(L, coeffs, steps) != 0;
+  if (!gspace) {
     Timed t(MUON_K_OTHER, 0.0, s);
     rc = muon_launch_finalize(L, ws, batch, prescale, eps, s);
   }
@@ -431,6 +436,27 @@ static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch
       rc = muon_launch_short_gram(L, X[0], part, batch, s);
     }
     if (rc != MUON_OK) return rc;
+    const int64_t xs = 64 * L.n_pad * 2, bs = 64 * 64 * 2;  // bytes per matrix
+    if (gspace) {
+      // very wide: every iteration on the Gram matrix, then U = Q X in one product
+      {
+        Timed t(MUON_K_SYRK_AA, bm * steps * md * (md + 1) * md, s);
+        rc = muon_launch_short_gspace(L, part, batch, coeffs, steps, prescale, eps,
+                                      (float*)(w + L.off_scale), s);
+      }
+      if (rc != MUON_OK) return rc;
+      if (ap) {
+        Timed t(MUON_K_GEMM_BX_APPLY, bm * 2.0 * md * md * nd, s);
+        const int64_t ps = L.gparts * SHORT_PART_BYTES / 4;
+        return apply_chunks(*ap, [&](int64_t m0, int64_t cnt, const MuonApply& tab) {
+          return muon_launch_short_bx_apply(L, X[0] + m0 * xs, nullptr, part + m0 * ps, cnt, 1.0f,
+                                            0.0f, scale + m0, 1, tab, s);
+        });
+      }
+      Timed t(MUON_K_GEMM_BX, bm * 2.0 * md * md * nd, s);
+      return muon_launch_short_bx(L, X[0], X[steps & 1], nullptr, part, batch, 1.0f, 0.0f, scale,
+                                  1, 0, s);
+    }
     for (int it = 0; it < steps; ++it) {
       const float a = (float)coeffs[3 * it], b = (float)coeffs[3 * it + 1],
                   c = (float)coeffs[3 * it + 2];
@@ -443,10 +469,9 @@ static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch
       if (rc != MUON_OK) return rc;
       if (ap && !more) {
         Timed t(MUON_K_GEMM_BX_APPLY, bm * 2.0 * md * md * nd, s);
-        const int64_t xs = 64 * L.n_pad * 2, bs = 64 * 64 * 2;  // bytes per matrix
         rc = apply_chunks(*ap, [&](int64_t m0, int64_t cnt, const MuonApply& tab) {
-          return muon_launch_short_bx_apply(L, X[it & 1] + m0 * xs, B + m0 * bs, cnt, 1.0f, a,
-                                            scale + m0, first, tab, s);
+          return muon_launch_short_bx_apply(L, X[it & 1] + m0 * xs, B + m0 * bs, nullptr, cnt,
+                                            1.0f, a, scale + m0, first, tab, s);
         });
       } else {
         Timed t(MUON_K_GEMM_BX, bm * 2.0 * md * md * nd + (more ? bm * md * (md + 1) * nd : 0.0), s);

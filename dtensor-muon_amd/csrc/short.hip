@@ -14,6 +14,8 @@
 //                      partial Gram matrices of the bf16 X' for the next iteration,
 //                      formed from the registers that hold X' (X is read once per
 //                      iteration, X' written once).
+// From 65536 columns on the iterations run on the Gram matrix instead, and X is read once by
+// the Gram product and once by the last one (short_gspace_kernel).
 // The arithmetic is the one of the tiled path (gemm.hip) for the same iteration: fp32
 // accumulation of bf16 products, A and B rounded to bf16 once, X' = alpha (acc + ratio X)
 // rounded once; only the summation order of the Gram sums differs (column ranges).
@@ -51,6 +53,18 @@ struct ShortArgs {
   int gram;            // short_bx_kernel: write the next iteration's partials
   int64_t b0;          // index of this launch's matrix 0 in the bucket (the apply's tensors)
 };
+
+// The whole iteration on the 64 x 64 Gram matrix (short_gspace_kernel).
+constexpr int SG_GSTEPS = 5;
+struct GspaceArgs {
+  float* part;         // Gram partials [matrix][P][SG_PART]; part 0 holds their sum, parts 1-2
+                       // receive Q
+  int P, steps;
+  float prescale, eps;
+  float* scale;        // per-matrix Frobenius prescale s (written)
+  float a[SG_GSTEPS], b[SG_GSTEPS], c[SG_GSTEPS];
+};
+constexpr int SG_QELEMS = SG_ROWS * SG_ROWS;  // bf16 values of one part of Q
 
 // Column range [pb, pe) of panels for range p: balanced, non-empty when P <= panels.
 MUON_DEVICE void short_range(const ShortArgs& a, int p, int& pb, int& pe) {
@@ -190,6 +204,153 @@ __global__ __launch_bounds__(1024) void short_poly_kernel(ShortArgs a) {
   *(uint2*)(a.bm + (int64_t)b * SG_ROWS * SG_ROWS + i * SG_ROWS + j0) = w;
 }
 
+// Sum of the Gram partials of each matrix, into partial 0 as fp32: grid (48, batch), 256
+// threads = 64 elements x 4 groups of partials, each group summed in order in double and the
+// four groups in order. One workgroup per matrix (short_poly_kernel's own sum) reads 3 MB of
+// partials through one CU, 40-45 us; 48 workgroups read them in 7 us.
+__global__ __launch_bounds__(256) void short_reduce_kernel(float* part, int P) {
+  __shared__ double red[256];
+  const int tid = threadIdx.x, e = blockIdx.x * 64 + (tid & 63), grp = tid >> 6;
+  float* base = part + (int64_t)blockIdx.y * P * SG_PART + e;
+  const int p0 = grp * P / 4, p1 = (grp + 1) * P / 4;
+  double s = 0.0;
+#pragma unroll 16
+  for (int p = p0; p < p1; ++p) s += (double)base[(int64_t)p * SG_PART];
+  red[tid] = s;
+  __syncthreads();  // every partial of these 64 elements has been read
+  if (grp == 0) base[0] = (float)(((red[tid] + red[64 + tid]) + red[128 + tid]) + red[192 + tid]);
+}
+
+// All iterations of a very wide short matrix on its Gram matrix: grid (batch), 16 waves.
+// X_{k+1} = P_k X_k with P_k = a I + B_k a polynomial of A_k = X_k X_k^T, so
+// A_{k+1} = P_k A_k P_k^T and X_steps = Q X_0, Q = s P_{steps-1} ... P_0: X is read once by the
+// Gram product and once by the last product (short_bx_kernel with GS) instead of twice and
+// written once per iteration. G (the Gram matrix before rounding), P and Q are fp32; A and B
+// are rounded to bf16 where the streaming iteration rounds them, so the update follows that
+// iteration (its bf16 X' between the iterations is what is not rounded any more). The step on
+// three 64 x 2883584 matrices went from 4.94 to 2.88 ms: gone are four passes of 0.455 ms over
+// X, five launches of short_poly_kernel (45 us each on one CU per matrix) and the norm's own
+// reduction (46 us). Its error against 64 bits, root mean square over 8 inputs each, here and in the streaming iteration:
+// 1.44e-2 and 1.48e-2 for 64 x 131072, 2.15e-2 and 2.11e-2 for 16 x 131072, 2.87e-2 and 2.91e-2
+// for 8 x 2000000. An error e of G grows by a^2 per iteration in the directions X does not
+// reach; the caller bounds that growth (muon_short_gspace_ok).
+// Wave w owns the 16 x 16 tile (w / 4, w % 4) of every product (fp32 MFMA, 16 x 16 x 4).
+// The matrices live in LDS with a row pitch of 65 words. Q goes out as three bf16 parts
+// (24 significant bits) in the order of short_bx_kernel's fragments.
+constexpr int GS_LD = 65;
+constexpr int GS_MAT = SG_ROWS * GS_LD;
+__global__ __launch_bounds__(1024) void short_gspace_kernel(GspaceArgs ga) {
+#pragma clang fp contract(off)
+  __shared__ float lds[4 * GS_MAT];
+  __shared__ double tr[64];
+  float* G = lds;                // Gram matrix
+  float* M = lds + GS_MAT;       // A, then P
+  float* T = lds + 2 * GS_MAT;   // P G
+  float* Q = lds + 3 * GS_MAT;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, b = blockIdx.x;
+  const int ti = (wave >> 2) * 16, tj = (wave & 3) * 16;
+  float* part = ga.part + (int64_t)b * ga.P * SG_PART;
+  {
+    // element r * 64 + l of a block is (8 (r / 4) + 4 (l / 32) + r % 4, l % 32); the diagonal
+    // blocks keep their upper triangle, block (0, 1) goes to both halves
+    const int r = t >> 6, l = t & 63;
+    const int bi = 8 * (r >> 2) + 4 * (l >> 5) + (r & 3), bj = l & 31;
+    const float s0 = part[t], s1 = part[1024 + t], s2 = part[2048 + t];
+    if (bi <= bj) {
+      G[bi * GS_LD + bj] = s0;
+      G[bj * GS_LD + bi] = s0;
+      G[(32 + bi) * GS_LD + 32 + bj] = s2;
+      G[(32 + bj) * GS_LD + 32 + bi] = s2;
+    }
+    G[bi * GS_LD + 32 + bj] = s1;
+    G[(32 + bj) * GS_LD + bi] = s1;
+  }
+  __syncthreads();
+  // s = 1 / (||X||_F prescale + eps), ||X||_F^2 the trace
+  if (t < 64) tr[t] = (double)G[t * GS_LD + t];
+  __syncthreads();
+  double nn = 0.0;
+  for (int k = 0; k < 64; ++k) nn += tr[k];
+  const float norm = (float)sqrt(nn);
+  const float denom = norm * ga.prescale;
+  const float s = 1.0f / (denom + ga.eps);
+  if (t == 0) ga.scale[b] = s;
+  for (int e = t; e < SG_ROWS * SG_ROWS; e += 1024) G[(e >> 6) * GS_LD + (e & 63)] *= s * s;
+  __syncthreads();
+
+  // acc (16 x 16 tile, rows ti + 4 (lane / 16) + r, column tj + lane % 16) of L R, R(k, j) at
+  // R[k * rk + j * rj]
+  const int li = lane & 15, lk = lane >> 4;
+  auto product = [&](const float* L, const float* R, int rk, int rj) -> f32x4 {
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < SG_ROWS; k += 4)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(L[(ti + li) * GS_LD + k + lk],
+                                                 R[(k + lk) * rk + (tj + li) * rj], acc, 0, 0, 0);
+    return acc;
+  };
+  const int row0 = ti + 4 * lk, col = tj + li;
+
+  for (int it = 0; it < ga.steps; ++it) {
+    const float a = ga.a[it], bc = ga.b[it], c = ga.c[it];
+    const bool more = it + 1 < ga.steps;
+    // A = bf16(G), exactly symmetric (G's upper triangle)
+    for (int e = t; e < SG_ROWS * SG_ROWS; e += 1024) {
+      const int i = e >> 6, j = e & 63;
+      M[i * GS_LD + j] = bf16_to_f32(f32_to_bf16(i <= j ? G[i * GS_LD + j] : G[j * GS_LD + i]));
+    }
+    __syncthreads();
+    // B = bf16(c (A A + (b / c) A)), P = a I + B
+    const f32x4 aa = product(M, M, GS_LD, 1);
+    const float ratio = bc != 0.0f ? bc / c : 0.0f;
+    float pv[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float av = M[(row0 + r) * GS_LD + col];
+      const float rv = ratio * av;
+      const float bv = bf16_to_f32(f32_to_bf16(c != 0.0f ? c * (aa[r] + rv) : bc * av));
+      pv[r] = row0 + r == col ? a + bv : bv;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      M[(row0 + r) * GS_LD + col] = pv[r];
+      if (it == 0) Q[(row0 + r) * GS_LD + col] = pv[r];
+    }
+    __syncthreads();
+    f32x4 q = {}, tg = {};
+    if (it > 0) q = product(M, Q, GS_LD, 1);
+    if (more) tg = product(M, G, GS_LD, 1);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (it > 0) Q[(row0 + r) * GS_LD + col] = q[r];
+      if (more) T[(row0 + r) * GS_LD + col] = tg[r];
+    }
+    __syncthreads();
+    if (more) {
+      const f32x4 g = product(T, M, 1, GS_LD);  // T P^T
+#pragma unroll
+      for (int r = 0; r < 4; ++r) G[(row0 + r) * GS_LD + col] = g[r];
+      __syncthreads();
+    }
+  }
+  // Q = hi + mid + lo, each bf16; fragment (fm, ks) of part h: lane l holds
+  // Q(32 fm + l % 32, 16 ks + 8 (l / 32) .. +7)
+  bf16_t* out = (bf16_t*)(part + SG_PART);
+  for (int e = t; e < SG_QELEMS; e += 1024) {
+    const int j = e & 7, l = (e >> 3) & 63, f = e >> 9;  // f = 4 fm + ks
+    const float v = Q[(32 * (f >> 2) + (l & 31)) * GS_LD + 16 * (f & 3) + 8 * (l >> 5) + j];
+    const bf16_t hi = f32_to_bf16(v);
+    const float r1 = v - bf16_to_f32(hi);
+    const bf16_t mid = f32_to_bf16(r1);
+    const float r2 = r1 - bf16_to_f32(mid);
+    out[e] = hi;
+    out[SG_QELEMS + e] = mid;
+    out[2 * SG_QELEMS + e] = f32_to_bf16(r2);
+  }
+}
+
 // 16-byte chunk position of logical chunk c in row `row` of a wave's sub-panel (rows of
 // 128 bytes). Bit 2 (row bit 1) puts the four rows of one transposing read in four
 // different 64-byte bank groups; bits 0-1 (row bits 2-3) spread the 32 rows of one
@@ -214,9 +375,13 @@ MUON_DEVICE int sg_swz(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) &
 // 16-byte piece of it is the update of 8 parameter elements, applied as the post-pass does
 // (apply_bf16x8, form AM) and the parameter written back. The parameter pieces of a panel
 // load before the next panel's X, so waiting for them never waits for that prefetch.
-template <int AM>
+// GS (the one product of an iteration run on the Gram matrix): X' = alpha Q X with Q in three
+// bf16 parts, the two low ones read from LDS (16 KB above the sub-panels) in fragment order;
+// X' may overwrite X (a panel is read before it is written, by the same wave).
+template <int AM, bool GS = false>
 __global__ __launch_bounds__(256) void short_bx_kernel(ShortArgs a, MuonApply ap) {
   __shared__ __align__(16) float red[4 * SG_PART];  // sub-panels (32 KB), then partials
+  static_assert(4 * SG_WAVE_LDS + 2 * SG_QELEMS * 2 <= 4 * SG_PART * 4, "Q parts fit");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int p = blockIdx.x, b = blockIdx.y;
   int pb, pe;
@@ -231,7 +396,17 @@ __global__ __launch_bounds__(256) void short_bx_kernel(ShortArgs a, MuonApply ap
 
   // B fragments: lane l holds B(32 fm + l % 32, 16 ks + 8 (l / 32) .. +7)
   bf16x8_mfma bfr[2][4];
-  {
+  const uint4* qlow = (const uint4*)((uint8_t*)red + 4 * SG_WAVE_LDS) + lane;
+  if constexpr (GS) {
+    const uint4* qp = (const uint4*)(a.part + ((int64_t)b * a.P + 1) * SG_PART);
+#pragma unroll
+    for (int f = 0; f < 8; ++f) bfr[f >> 2][f & 3] = as_frag(qp[f * 64 + lane]);
+    uint4* ql = (uint4*)((uint8_t*)red + 4 * SG_WAVE_LDS);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      ql[k * 256 + threadIdx.x] = qp[SG_QELEMS / 8 + k * 256 + threadIdx.x];
+    __syncthreads();
+  } else {
     const bf16_t* bp = a.bm + (int64_t)b * SG_ROWS * SG_ROWS + (lane & 31) * SG_ROWS + (lane >> 5) * 8;
 #pragma unroll
     for (int fm = 0; fm < 2; ++fm)
@@ -311,6 +486,16 @@ __global__ __launch_bounds__(256) void short_bx_kernel(ShortArgs a, MuonApply ap
         xf[ks] = __builtin_bit_cast(bf16x8_mfma, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
       f32x16 acc[2] = {{}, {}};
+      if constexpr (GS) {
+#pragma unroll
+        for (int h = 1; h >= 0; --h)
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int fm = 0; fm < 2; ++fm)
+              acc[fm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                  xf[ks], as_frag(qlow[h * (SG_QELEMS / 8) + (fm * 4 + ks) * 64]), acc[fm], 0, 0, 0);
+      }
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
@@ -323,6 +508,13 @@ __global__ __launch_bounds__(256) void short_bx_kernel(ShortArgs a, MuonApply ap
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
           uint8_t* pos = reg + row * 128 + (((4 * fn + rg) ^ sg_swz(row)) << 4) + fh * 8;
+          if constexpr (GS) {
+            const f2x v01 = {alpha * acc[fm][rg * 4 + 0], alpha * acc[fm][rg * 4 + 1]};
+            const f2x v23 = {alpha * acc[fm][rg * 4 + 2], alpha * acc[fm][rg * 4 + 3]};
+            *(u32x2*)pos = u32x2{__builtin_bit_cast(uint32_t, __builtin_convertvector(v01, bf2x)),
+                                 __builtin_bit_cast(uint32_t, __builtin_convertvector(v23, bf2x))};
+            continue;
+          }
           const u32x2 xw = *(const u32x2*)pos;
           const f2x v01 = {alpha * (acc[fm][rg * 4 + 0] + ratio * __uint_as_float(xw.x << 16)),
                            alpha * (acc[fm][rg * 4 + 1] + ratio * __uint_as_float(xw.x & 0xffff0000u))};
@@ -333,7 +525,7 @@ __global__ __launch_bounds__(256) void short_bx_kernel(ShortArgs a, MuonApply ap
           *(u32x2*)pos = w[fm][rg];
         }
       }
-      if (AM < 0 && a.gram) {
+      if (AM < 0 && !GS && a.gram) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const bf16x8_mfma h0 = as_frag(uint4{w[0][2 * h].x, w[0][2 * h].y, w[0][2 * h + 1].x, w[0][2 * h + 1].y});
@@ -360,7 +552,7 @@ __global__ __launch_bounds__(256) void short_bx_kernel(ShortArgs a, MuonApply ap
     }
     asm volatile("" ::: "memory");
   }
-  if (AM < 0 && a.gram) short_write_partial(a, red, g00, g01, g11, b, p);
+  if (AM < 0 && !GS && a.gram) short_write_partial(a, red, g00, g01, g11, b, p);
 }
 
 }  // namespace
@@ -408,9 +600,48 @@ int muon_launch_short_poly(const OrthLayout& L, float* part, void* bm, int64_t b
   return MUON_OK;
 }
 
+// The iteration on the Gram matrix (short_gspace_kernel) serves iterates of at least
+// SG_GSPACE_N columns: below that X fits the caches and its passes are launches, not bytes,
+// while the bf16 rounding of A decides more of the result as the Gram sums get shorter. The
+// partials' slots 1 and 2 hold Q, and an error of the Gram matrix may grow 2^18 times (Polar
+// Express 1.8e5, Newton-Schulz 2.0e4 over five iterations), to 2% from fp32's 1e-7.
+constexpr int64_t SG_GSPACE_N = 65536;
+int muon_short_gspace_ok(const OrthLayout& L, const double* coeffs, int steps) {
+  if (!L.short_m || L.n < SG_GSPACE_N || L.gparts < 3 || steps < 2 || steps > SG_GSTEPS) return 0;
+  double growth = 1.0;
+  for (int it = 0; it + 1 < steps; ++it) growth *= coeffs[3 * it] * coeffs[3 * it];
+  return growth <= 262144.0;
+}
+
+// Sum of the partials, the iteration on the Gram matrix, Q into the partials' slots.
+int muon_launch_short_gspace(const OrthLayout& L, float* part, int64_t batch, const double* coeffs,
+                             int steps, float prescale, float eps, float* scale, hipStream_t s) {
+  GspaceArgs a = {};
+  a.P = (int)L.gparts;
+  a.steps = steps;
+  a.prescale = prescale;
+  a.eps = eps;
+  for (int it = 0; it < steps; ++it) {
+    a.a[it] = (float)coeffs[3 * it];
+    a.b[it] = (float)coeffs[3 * it + 1];
+    a.c[it] = (float)coeffs[3 * it + 2];
+  }
+  for (int64_t b0 = 0; b0 < batch; b0 += SG_GRID_Y) {
+    const int64_t nb = std::min<int64_t>(SG_GRID_Y, batch - b0);
+    a.part = part + b0 * a.P * SG_PART;
+    a.scale = scale + b0;
+    hipLaunchKernelGGL(short_reduce_kernel, dim3(SG_PART / 64, (unsigned)nb), dim3(256), 0, s,
+                       a.part, a.P);
+    hipLaunchKernelGGL(short_gspace_kernel, dim3((unsigned)nb), dim3(1024), 0, s, a);
+  }
+  MUON_CHECK_LAUNCH("short_gspace");
+  return MUON_OK;
+}
+
 // X' = alpha B X + beta X of a short iterate (ap == nullptr: into xo, with the next partials
 // when gram), or the last iteration with the apply of a wide bucket of bf16 parameters
 // (ap: X' is not stored, the parameters are updated in place; no partials).
+// bm == nullptr: Q X from the partials' slots (after muon_launch_short_gspace).
 static int launch_short_bx(const OrthLayout& L, const void* x, void* xo, const void* bm,
                            float* part, int64_t batch, float alpha, float beta,
                            const float* scale, int first, int gram, const MuonApply* ap,
@@ -454,17 +685,21 @@ static int launch_short_bx(const OrthLayout& L, const void* x, void* xo, const v
     ShortArgs c = a;
     c.x += b0 * c.mstride;
     if (c.xo) c.xo += b0 * c.mstride;
-    c.bm += b0 * SG_ROWS * SG_ROWS;
+    if (c.bm) c.bm += b0 * SG_ROWS * SG_ROWS;
     if (c.part) c.part += b0 * c.P * SG_PART;
     c.scale = scale ? scale + b0 : nullptr;
     c.b0 = b0;
     const int64_t nb = std::min<int64_t>(SG_GRID_Y, batch - b0);
     const dim3 grid((unsigned)c.P, (unsigned)nb);
+    const bool gs = bm == nullptr;
+    auto launch = [&](auto* kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, c, apv);
+    };
     switch (mode) {
-      case 0: hipLaunchKernelGGL(short_bx_kernel<0>, grid, dim3(256), 0, s, c, apv); break;
-      case 1: hipLaunchKernelGGL(short_bx_kernel<1>, grid, dim3(256), 0, s, c, apv); break;
-      case 2: hipLaunchKernelGGL(short_bx_kernel<2>, grid, dim3(256), 0, s, c, apv); break;
-      default: hipLaunchKernelGGL(short_bx_kernel<-1>, grid, dim3(256), 0, s, c, apv); break;
+      case 0: launch(gs ? short_bx_kernel<0, true> : short_bx_kernel<0>); break;
+      case 1: launch(gs ? short_bx_kernel<1, true> : short_bx_kernel<1>); break;
+      case 2: launch(gs ? short_bx_kernel<2, true> : short_bx_kernel<2>); break;
+      default: launch(gs ? short_bx_kernel<-1, true> : short_bx_kernel<-1>); break;
     }
   }
   MUON_CHECK_LAUNCH("short_bx");
@@ -477,8 +712,8 @@ int muon_launch_short_bx(const OrthLayout& L, const void* x, void* xo, const voi
   return launch_short_bx(L, x, xo, bm, part, batch, alpha, beta, scale, first, gram, nullptr, s);
 }
 
-int muon_launch_short_bx_apply(const OrthLayout& L, const void* x, const void* bm,
+int muon_launch_short_bx_apply(const OrthLayout& L, const void* x, const void* bm, float* part,
                                int64_t batch, float alpha, float beta, const float* scale,
                                int first, const MuonApply& ap, hipStream_t s) {
-  return launch_short_bx(L, x, nullptr, bm, nullptr, batch, alpha, beta, scale, first, 0, &ap, s);
+  return launch_short_bx(L, x, nullptr, bm, part, batch, alpha, beta, scale, first, 0, &ap, s);
 }
