@@ -275,6 +275,12 @@ int muon_gram(const void* x, void* y, int dtype, int64_t batch, int64_t M, int64
     return muon_launch_gemm(dtype, MODE_SYRK, false, batch, M, M, K, x, K, M * K, x, K, M * K,
                             nullptr, 0, 0, y, M, M * M, nullptr, 0, 0, M, M, 1.0f, 0.0f,
                             nullptr, 0, (hipStream_t)stream);
+  if (dtype == MUON_DT_F32 && M % 128 == 0 && K % 64 == 0 && !((uintptr_t)x & 15) &&
+      !((uintptr_t)y & 15))
+    // the same for fp32: whole 128-row tiles and 64-wide steps of K
+    return muon_launch_gemm(dtype, MODE_SYRK, false, batch, M, M, K, x, K, M * K, x, K, M * K,
+                            nullptr, 0, 0, y, M, M * M, nullptr, 0, 0, M, M, 1.0f, 0.0f,
+                            nullptr, 0, (hipStream_t)stream);
   return muon_launch_gemm(dtype, MODE_SYRK, true, batch, M, M, K, x, K,
                           M * K, x, K, M * K, nullptr, 0, 0, y, M, M * M, nullptr, 0, 0, M, M,
                           1.0f, 0.0f, nullptr, 0, (hipStream_t)stream);

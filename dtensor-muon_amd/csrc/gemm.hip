@@ -334,26 +334,22 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_bf16_kernel(GemmArgs g
 }
 
 // ----------------------------------------------------------------------------------
-// fp32: 128 x 128 x 16 tile, 4 wavefronts in 2 x 2, each 64 x 64 (2 x 2 MFMA
-// 32x32x2 f32 blocks). Used for the fp32 iteration mode and fp32 gram_. In GEMM (NN)
-// mode the b panel is staged as rows k of X (pitch F_XP); the MFMA takes one value
-// per lane, so no transpose is needed.
-constexpr int F_BM = 128, F_BN = 128, F_BK = 16, F_LDSP = F_BK + 4, F_XP = F_BN + 4;
-static_assert(F_BK * F_XP <= F_BN * F_LDSP, "fp32 X panel fits the b buffer");
+// fp32 gram_ of caller-owned tensors (any extents, element loads with bounds): 128 x 128 x
+// 16 tile, 4 wavefronts in 2 x 2, each 64 x 64 (2 x 2 MFMA 32x32x2 f32 blocks).
+constexpr int F_BM = 128, F_BK = 16, F_LDSP = F_BK + 4;
 
-template <int MODE, bool MASKED>
-__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs g) {
+__global__ __launch_bounds__(256, 2) void gemm_f32_masked_kernel(GemmArgs g) {
   __shared__ __align__(16) float As[2][F_BM * F_LDSP];
-  __shared__ __align__(16) float Bs[2][F_BN * F_LDSP];
+  __shared__ __align__(16) float Bs[2][F_BM * F_LDSP];
 
   int bidx, tm, tn;
-  map_tile(g, MODE, bidx, tm, tn);
+  map_tile(g, MODE_SYRK, bidx, tm, tn);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
 
   const float* A = (const float*)g.a + (int64_t)bidx * g.sa;
   const float* B = (const float*)g.b + (int64_t)bidx * g.sb;
-  const int64_t arow0 = (int64_t)tm * F_BM, brow0 = (int64_t)tn * F_BN;
+  const int64_t arow0 = (int64_t)tm * F_BM, brow0 = (int64_t)tn * F_BM;
 
   float4 ra[2], rb[2];
   auto gload = [&](int64_t k0) {
@@ -361,24 +357,16 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs g) {
     for (int q = 0; q < 2; ++q) {
       const int c = q * 256 + tid;
       const int r = c >> 2, cc = (c & 3) * 4;
-      if (!MASKED) {
-        ra[q] = *(const float4*)(A + (arow0 + r) * g.lda + k0 + cc);
-        if (MODE == MODE_GEMM)
-          rb[q] = *(const float4*)(B + (k0 + (c >> 5)) * g.ldb + brow0 + (c & 31) * 4);
-        else
-          rb[q] = *(const float4*)(B + (brow0 + r) * g.ldb + k0 + cc);
-      } else {
-        float ta[4], tb[4];
+      float ta[4], tb[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t k = k0 + cc + e;
-          const int64_t ia = arow0 + r, ib = brow0 + r;
-          ta[e] = (ia < g.Mt && k < g.Kt) ? A[ia * g.lda + k] : 0.0f;
-          tb[e] = (ib < g.Nt && k < g.Kt) ? B[ib * g.ldb + k] : 0.0f;
-        }
-        ra[q] = make_float4(ta[0], ta[1], ta[2], ta[3]);
-        rb[q] = make_float4(tb[0], tb[1], tb[2], tb[3]);
+      for (int e = 0; e < 4; ++e) {
+        const int64_t k = k0 + cc + e;
+        const int64_t ia = arow0 + r, ib = brow0 + r;
+        ta[e] = (ia < g.Mt && k < g.Kt) ? A[ia * g.lda + k] : 0.0f;
+        tb[e] = (ib < g.Nt && k < g.Kt) ? B[ib * g.ldb + k] : 0.0f;
       }
+      ra[q] = make_float4(ta[0], ta[1], ta[2], ta[3]);
+      rb[q] = make_float4(tb[0], tb[1], tb[2], tb[3]);
     }
   };
   auto sstore = [&](int buf) {
@@ -387,10 +375,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs g) {
       const int c = q * 256 + tid;
       const int r = c >> 2, cc = (c & 3) * 4;
       *(float4*)(&As[buf][r * F_LDSP + cc]) = ra[q];
-      if (MODE == MODE_GEMM)
-        *(float4*)(&Bs[buf][(c >> 5) * F_XP + (c & 31) * 4]) = rb[q];
-      else
-        *(float4*)(&Bs[buf][r * F_LDSP + cc]) = rb[q];
+      *(float4*)(&Bs[buf][r * F_LDSP + cc]) = rb[q];
     }
   };
 
@@ -416,8 +401,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs g) {
 #pragma unroll
       for (int f = 0; f < 2; ++f) {
         af[f] = As[cur][(wm * 64 + f * 32 + frow) * F_LDSP + ks * 2 + fk];
-        bfr[f] = MODE == MODE_GEMM ? Bs[cur][(ks * 2 + fk) * F_XP + wn * 64 + f * 32 + frow]
-                                   : Bs[cur][(wn * 64 + f * 32 + frow) * F_LDSP + ks * 2 + fk];
+        bfr[f] = Bs[cur][(wn * 64 + f * 32 + frow) * F_LDSP + ks * 2 + fk];
       }
 #pragma unroll
       for (int fm = 0; fm < 2; ++fm)
@@ -429,8 +413,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs g) {
     __syncthreads();
   }
 
-  epilogue<float, 2, 2, MASKED>(g, MODE, bidx, arow0 + wm * 64, brow0 + wn * 64, acc, lane,
-                        MODE == MODE_SYRK && tm == tn);
+  epilogue<float, 2, 2, true>(g, MODE_SYRK, bidx, arow0 + wm * 64, brow0 + wn * 64, acc, lane,
+                              tm == tn);
 }
 
 // ----------------------------------------------------------------------------------
@@ -2758,6 +2742,143 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_s16h_kernel(GemmArgs g) {
     kloop(I2{}, std::true_type{});
 }
 
+// ----------------------------------------------------------------------------------
+// The fp32 iteration (padded workspaces) and fp32 gram_ of whole tiles: 64 x 64 output tiles,
+// 8 waves: two groups of 2 x 2, each wave one 32 x 32 block of 32 x 32 x 2 MFMAs; group 0 sums
+// k 0-15 of every 32, group 1 k 16-31, and group 0 adds the two sums at the end (half the
+// length of the chains: 1.8e-6 from 64 bits after five iterations of 4 x 768 x 2304, 2.7e-6
+// with one chain). Bound by the fp32 matrix rate (64 cycles for each 4 KFLOP MFMA), so the
+// kernel has to keep an MFMA ready on every SIMD also where a launch has one workgroup per CU.
+// Operands stream HBM/L2 -> LDS with `buffer_load_dwordx4 ... lds` into five stages of 32 k
+// (80 KB: two workgroups per CU); a K-tile's fragments are read while the MFMAs of the one
+// before run, and a lane reads 4 consecutive k of its row with one ds_read_b128: MFMA t of a
+// group of 8 k takes k = 8 q + 4 (lane / 32) + t on both operands (a sum may take its k in
+// any order). Panel rows of 32 floats are stored with the 16-byte chunk c of row r at
+// c ^ kswz(r), so the 16 rows of a read phase fall in distinct banks. In GEMM (NN) mode the b
+// panel is 32 rows k of X (one float per lane and MFMA, 32 consecutive columns; the rows of
+// the two half waves are 4 apart, and the XOR of the column's bit 5 with row bit 2 keeps
+// them in different banks).
+// Four matrices of 768 x 2304, one iteration's three products (X X^T, A A, B X): 77, 33 and
+// 106 us, against 265, 101 and 173 us on the 128-row tiles of a register-staged kernel before
+// (84 workgroups for the Gram products on 256 CUs, one wave per SIMD, LDS bank conflicts). This
+// kernel on 128-row tiles was slower at every size: 117 against 126 TFLOP/s over the whole loop
+// on 2 x 4096 x 4096, 83 against 109 on 8 x 1024 x 4096, 54 against 64 on 64 x 256 x 1024.
+constexpr int F_TM = 64, F_KT = 32, F_NS = 5;
+constexpr int F_PANELB = F_TM * F_KT * 4, F_STAGEB = 2 * F_PANELB, F_SMEM = F_NS * F_STAGEB;
+
+MUON_DEVICE void f32_dma(int vo, u32x4 rs, int so, uint32_t m0) {
+  asm volatile("s_mov_b32 m0, %[mz]\n\ts_nop 0\n\tbuffer_load_dwordx4 %[vo], %[rs], %[so] offen lds\n\t"
+               :
+               : [vo] "v"(vo), [rs] "s"(rs), [so] "s"(so), [mz] "s"(m0)
+               : "m0", "memory");
+}
+
+template <int MODE>
+__global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  int bidx, tm, tn;
+  map_tile(g, MODE, bidx, tm, tn);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+  const int64_t row0 = (int64_t)tm * F_TM, col0 = (int64_t)tn * F_TM;
+  const float* A = (const float*)g.a + (int64_t)bidx * g.sa + row0 * g.lda;
+  const float* B = (const float*)g.b + (int64_t)bidx * g.sb + (MODE == MODE_GEMM ? col0 : col0 * g.ldb);
+  const u32x4 rsa = n4_rsrc(A, false), rsb = n4_rsrc(B, false), rs_none = n4_rsrc(A, true);
+  const int lda_b = (int)(g.lda * 4), ldb_b = (int)(g.ldb * 4);
+  // this wave's load of a panel fills 1 KB: 8 rows of 8 chunks (K-contiguous panels), or 4
+  // rows k of 16 chunks (X panel)
+  const int ra = wave * 8 + (lane >> 3);
+  const int voa = ra * lda_b + (((lane & 7) ^ kswz(ra)) << 4);
+  int vob, kstep_b;
+  if constexpr (MODE == MODE_GEMM) {
+    const int rk = wave * 4 + (lane >> 4);
+    vob = rk * ldb_b + (((lane & 15) ^ (((rk >> 2) & 1) << 3)) << 4);
+    kstep_b = F_KT * ldb_b;
+  } else {
+    vob = ra * ldb_b + (((lane & 7) ^ kswz(ra)) << 4);
+    kstep_b = F_KT * 4;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  const int KT = (int)(g.K / F_KT);
+  auto issue = [&](int kt, int st) {
+    const bool on = kt < KT;  // past the last K-tile: the null descriptor reads no memory
+    const int kk = on ? kt : 0;
+    const uint32_t m0 = lds0 + st * F_STAGEB + wave * 1024;
+    f32_dma(voa, on ? rsa : rs_none, kk * F_KT * 4, m0);
+    f32_dma(vob, on ? rsb : rs_none, kk * kstep_b, m0 + F_PANELB);
+  };
+
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  const int fr = lane & 31, fh = lane >> 5;
+  struct Frags {
+    float4 a[2], b[2];  // this group's two groups of 8 k
+  };
+  auto load = [&](Frags& f, int st) {
+    const uint8_t* pa = smem + st * F_STAGEB + (wm * 32 + fr) * (F_KT * 4);
+    const uint8_t* pb = smem + st * F_STAGEB + F_PANELB;
+#pragma unroll
+    for (int q2 = 0; q2 < 2; ++q2) {
+      const int q = 2 * grp + q2;
+      const int cpos = ((2 * q + fh) ^ kswz(fr)) << 4;  // (a row offset by 32 keeps its swizzle)
+      f.a[q2] = *(const float4*)(pa + cpos);
+      if constexpr (MODE == MODE_GEMM) {
+        const float* x = (const float*)pb + (8 * q + 4 * fh) * F_TM + ((wn * 32 + fr) ^ (fh << 5));
+        f.b[q2] = make_float4(x[0], x[F_TM], x[2 * F_TM], x[3 * F_TM]);
+      } else {
+        f.b[q2] = *(const float4*)(pb + (wn * 32 + fr) * (F_KT * 4) + cpos);
+      }
+    }
+  };
+  auto mma = [&](const Frags& f) {
+#pragma unroll
+    for (int q2 = 0; q2 < 2; ++q2)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float*)&f.a[q2])[t],
+                                                   ((const float*)&f.b[q2])[t], acc, 0, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < F_NS - 1; ++t) issue(t, t);
+  // K-tile kt: once K-tile kt + 1 has landed (those up to kt + F_NS - 2 may still be under way,
+  // two loads each) and every wave has read K-tile kt, the load of K-tile kt + F_NS - 1, the
+  // fragments of K-tile kt + 1, and the MFMAs of K-tile kt while those reads complete
+  int st = 0;
+  auto step = [&](int kt, const Frags& cur, Frags& next) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * (F_NS - 3)) : "memory");
+    lds_barrier();
+    issue(kt + F_NS - 1, st == 0 ? F_NS - 1 : st - 1);
+    st = st + 1 == F_NS ? 0 : st + 1;
+    load(next, st);
+    mma(cur);
+  };
+  Frags f0, f1;
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * (F_NS - 2)) : "memory");
+  lds_barrier();
+  load(f0, 0);
+  for (int kt = 0; kt < KT; kt += 2) {  // (K is a multiple of 64)
+    step(kt, f0, f1);
+    step(kt + 1, f1, f0);
+  }
+  wait_vmcnt0();
+  // group 1's sums through LDS (the stages are done with)
+  float* sum = (float*)smem + (wave & 3) * 1024 + lane;
+  lds_barrier();
+  if (grp == 1) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[r * 64] = acc[r];
+  }
+  lds_barrier();
+  if (grp == 1) return;
+  f32x16 accs[1][1];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) accs[0][0][r] = acc[r] + sum[r * 64];
+  epilogue<float, 1, 1, false>(g, MODE, bidx, row0 + wm * 32, col0 + wn * 32, accs, lane,
+                               MODE == MODE_SYRK && tm == tn);
+}
+
 // Wave grid of the register-staged bf16 kernel (gemm_bf16_kernel), which serves the
 // masked gram_ path and SYRKs whose beta term has no alpha to fold into: 4 x 2
 // wavefronts, each 64 x 128, two waves per SIMD.
@@ -2770,9 +2891,9 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_s16h_kernel(GemmArgs g) {
 constexpr int BF_WGM = MUON_BF16_WGM, BF_WGN = MUON_BF16_WGN;
 constexpr int BF_NT = 64 * BF_WGM * BF_WGN;
 
-// The bf16 kernels need more than the default 64 KiB of dynamic LDS; raise the
+// The product kernels need more than the default 64 KiB of dynamic LDS; raise the
 // per-kernel limit once per process for every instantiation.
-int reserve_bf16_lds() {
+int reserve_lds() {
   static int status = -1;
   static std::once_flag once;
   std::call_once(once, [] {
@@ -2803,6 +2924,12 @@ int reserve_bf16_lds() {
         (const void*)gemm_bf16_nn16_kernel<2, 2>};
     for (const void* k : n16)
       if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, N4_SMEM) !=
+          hipSuccess)
+        status = -1;
+    const void* f32[2] = {(const void*)gemm_f32_kernel<MODE_SYRK>,
+                          (const void*)gemm_f32_kernel<MODE_GEMM>};
+    for (const void* k : f32)
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, F_SMEM) !=
           hipSuccess)
         status = -1;
   });
@@ -2893,7 +3020,7 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
   g.store_out = out != nullptr;
   g.store_out_t = out_t != nullptr;
   const int bm = dtype == MUON_DT_BF16 ? BF_BM : F_BM;
-  const int bk = dtype == MUON_DT_BF16 ? BF_BK : F_BK;
+  const int bk = dtype == MUON_DT_BF16 ? BF_BK : (masked ? F_BK : 64);
   g.tiles_m = (int)((M + bm - 1) / bm);
   g.tiles_n = (int)((N + bm - 1) / bm);
   g.K = masked ? round_up(K, bk) : K;
@@ -2925,11 +3052,11 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
     return MUON_ERR_SHAPE;
   }
   dim3 grid((unsigned)blocks), block(256);
+  if (reserve_lds() != 0) {
+    muon_set_error("gemm: cannot reserve %d B of LDS", BF_SMEM);
+    return MUON_ERR_LAUNCH;
+  }
   if (dtype == MUON_DT_BF16) {
-    if (reserve_bf16_lds() != 0) {
-      muon_set_error("gemm: cannot reserve %d B of LDS", BF_SMEM);
-      return MUON_ERR_LAUNCH;
-    }
 #define LAUNCH_BF(MODE_, MASK_)                                                        \
   do {                                                                                 \
     hipLaunchKernelGGL((gemm_bf16_kernel<MODE_, MASK_, BF_WGM, BF_WGN>), grid, dim3(BF_NT), \
@@ -2983,13 +3110,25 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
     }
 #undef LAUNCH_BF
   } else if (dtype == MUON_DT_F32) {
-    if (mode == MODE_SYRK) {
-      if (masked)
-        hipLaunchKernelGGL((gemm_f32_kernel<MODE_SYRK, true>), grid, block, 0, stream, g);
-      else
-        hipLaunchKernelGGL((gemm_f32_kernel<MODE_SYRK, false>), grid, block, 0, stream, g);
+    if (masked) {
+      hipLaunchKernelGGL(gemm_f32_masked_kernel, grid, block, 0, stream, g);
     } else {
-      hipLaunchKernelGGL((gemm_f32_kernel<MODE_GEMM, false>), grid, block, 0, stream, g);
+      GemmArgs gh = g;  // 64-row tiles
+      gh.tiles_m = (int)(M / F_TM);
+      gh.tiles_n = (int)(N / F_TM);
+      gh.tiles_per_batch = mode == MODE_SYRK ? gh.tiles_m * (gh.tiles_m + 1) / 2
+                                             : gh.tiles_m * gh.tiles_n;
+      const int64_t bh = (int64_t)gh.tiles_per_batch * batch;
+      if (bh > 0x7fffffffLL) {
+        muon_set_error("gemm: grid too large (%lld workgroups)", (long long)bh);
+        return MUON_ERR_SHAPE;
+      }
+      if (mode == MODE_SYRK)
+        hipLaunchKernelGGL((gemm_f32_kernel<MODE_SYRK>), dim3((unsigned)bh), dim3(512), F_SMEM,
+                           stream, gh);
+      else
+        hipLaunchKernelGGL((gemm_f32_kernel<MODE_GEMM>), dim3((unsigned)bh), dim3(512), F_SMEM,
+                           stream, gh);
     }
   } else {
     muon_set_error("gemm: unsupported dtype %d", dtype);
@@ -3047,7 +3186,7 @@ int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const
     return MUON_ERR_SHAPE;
   }
   g.tiles_total = (int)blocks;
-  if (reserve_bf16_lds() != 0) {
+  if (reserve_lds() != 0) {
     muon_set_error("gemm_apply: cannot reserve LDS");
     return MUON_ERR_LAUNCH;
   }
