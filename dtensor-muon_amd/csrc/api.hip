@@ -20,7 +20,9 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
 int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const void* a,
                            int64_t lda, int64_t sa, const void* b, int64_t ldb, int64_t sb,
                            int64_t Mv, int64_t Nv, float alpha, float beta, const float* scale,
-                           int scale_mode, const MuonApply& ap, int tall, hipStream_t stream);
+                           int scale_mode, const MuonApply& ap, int pdt, int tall,
+                           hipStream_t stream);
+int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int64_t n, int pdt);
 int muon_launch_prepass(int ntensors, void* const* grads, void* const* bufs, int gdt, int bdt,
                         int64_t nb, int64_t rows, int64_t cols, int64_t s_pitch,
                         int64_t s_mstride, float momentum, int nesterov, int maximize,
@@ -363,13 +365,13 @@ int muon_prepass(int ntensors, void* const* grads, void* const* bufs, int g_dtyp
 
 // The iteration; with `ap` (eligible shapes only, checked by the caller) the last X' is
 // not stored but applied to the parameters in the GEMM's epilogue.
-// The parameters of a fused apply: per tensor a bf16 pointer and lr * lr_ratio, nb matrices
+// The parameters of a fused apply: their type, per tensor a pointer and lr * lr_ratio, nb matrices
 // of prows x pcols each, wd and cautious. The last product's launches take them in chunks of
 // at most MUON_APPLY_MAX tensors (the table a launch carries).
 struct ApplyReq {
   void* const* params;
   const float* adj;
-  int ntensors;
+  int p_dtype, ntensors;
   int64_t nb, prows, pcols;
   float wd;
   int cautious;
@@ -520,7 +522,7 @@ static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch
       rc = apply_chunks(*ap, [&](int64_t m0, int64_t cnt, const MuonApply& tab) {
         return muon_launch_gemm_apply(cnt, mp, np, kq, B + m0 * mp * mp * 2, mp, mp * mp,
                                       Xc + m0 * mp * xp * 2, xp, mp * xp, L.m, L.n, 1.0f, a,
-                                      scale + m0, first ? 1 : 0, tab, L.tall, s);
+                                      scale + m0, first ? 1 : 0, tab, ap->p_dtype, L.tall, s);
       });
     } else {
     Timed t(MUON_K_GEMM_BX, bm * 2.0 * md * md * nd, s);
@@ -544,15 +546,16 @@ int muon_orth_run_apply(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,
                         int64_t cols, const double* coeffs, int steps, float prescale,
                         float eps, int ntensors, void* const* params, int p_dtype, int64_t nb,
                         const float* adjusted_lrs, float wd, int cautious, void* stream) {
-  bool fuse = ws_dtype == MUON_DT_BF16 && p_dtype == MUON_DT_BF16 && steps > 0 && rows > 0 &&
-              cols > 0 && nb > 0 && ntensors > 0 && (int64_t)ntensors * nb == batch && batch <= ws_batch && params && adjusted_lrs &&
-              cols % 8 == 0;
+  bool fuse = ws_dtype == MUON_DT_BF16 && io_dtype_ok(p_dtype) && steps > 0 && rows > 0 &&
+              cols > 0 && nb > 0 && ntensors > 0 && (int64_t)ntensors * nb == batch &&
+              batch <= ws_batch && params && adjusted_lrs && cols % 8 == 0;
   if (fuse) {
     const OrthLayout L = muon_orth_layout(ws_dtype, ws_batch, rows, cols);
     const int64_t kq = std::min(L.m_pad, round_up(L.m, 128));
-    // the tiled path from K = 768; iterates of at most 64 rows when the parameter is wide
-    // (its rows are the iterate's)
-    fuse = L.short_m ? !L.tall : kq >= 768;
+    // the tiled path where it pays; iterates of at most 64 rows when the parameter is bf16 and
+    // wide (its rows are the iterate's)
+    fuse = L.short_m ? !L.tall && p_dtype == MUON_DT_BF16
+                     : muon_apply_fuses(batch, L.m_pad, L.n_pad, kq, L.m, L.n, p_dtype) != 0;
     for (int t = 0; fuse && t < ntensors; ++t) fuse = params[t] && !((uintptr_t)params[t] & 15);
   }
   if (!fuse) {
@@ -562,7 +565,7 @@ int muon_orth_run_apply(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,
     return muon_postpass(ntensors, params, p_dtype, nullptr, 0, ws, ws_dtype, ws_batch, steps,
                          nb, rows, cols, adjusted_lrs, nullptr, wd, cautious, stream);
   }
-  const ApplyReq ap = {params, adjusted_lrs, ntensors, nb, rows, cols, wd, cautious};
+  const ApplyReq ap = {params, adjusted_lrs, p_dtype, ntensors, nb, rows, cols, wd, cautious};
   return orth_run_impl(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps, prescale, eps,
                        &ap, stream);
 }

@@ -47,6 +47,18 @@ struct GemmArgs {
   int tiles_m, tiles_n, tiles_per_batch;
   int tiles_total;             // tiles_per_batch * batch
   int store_out, store_out_t;
+  int t0, nb;                  // tile_bx_kernel's apply: first tensor in the table, matrices per tensor
+};
+
+// One launch over the products of several buckets (GROUP_MAX at most): group i owns the tiles
+// tile0[i] .. tile0[i + 1] - 1 of the launch. The buckets of a model share one side (its
+// width), so their launches of one kind do the same work on different matrices, and each
+// alone may leave most CUs idle.
+constexpr int GROUP_MAX = 8;
+struct GemmTab {
+  int n;
+  int tile0[GROUP_MAX + 1];
+  GemmArgs g[GROUP_MAX];
 };
 
 // Workgroup L of a one-tile-per-workgroup launch of `total` -> tile index. Dispatch
@@ -67,8 +79,8 @@ MUON_DEVICE int64_t xcd_tile(int64_t L, int64_t total, int tiles_per_batch) {
                    : 8 * nfull + x * rq + std::min<int64_t>(x, rr) + (i - nfull);
 }
 
-MUON_DEVICE void map_tile(const GemmArgs& g, int mode, int& bidx, int& tm, int& tn) {
-  const int64_t L = xcd_tile(blockIdx.x, (int64_t)gridDim.x, g.tiles_per_batch);
+// Tile t of a group -> matrix, tile row and column.
+MUON_DEVICE void tile_at(const GemmArgs& g, int mode, int64_t L, int& bidx, int& tm, int& tn) {
   bidx = (int)(L / g.tiles_per_batch);
   int t = (int)(L % g.tiles_per_batch);
   if (mode == MODE_SYRK) {
@@ -89,6 +101,24 @@ MUON_DEVICE void map_tile(const GemmArgs& g, int mode, int& bidx, int& tm, int& 
     tm = first + local % gsz;
     tn = local / gsz;
   }
+}
+
+MUON_DEVICE void map_tile(const GemmArgs& g, int mode, int& bidx, int& tm, int& tn) {
+  tile_at(g, mode, xcd_tile(blockIdx.x, (int64_t)gridDim.x, g.tiles_per_batch), bidx, tm, tn);
+}
+
+// This workgroup's arguments and tile. Of a launch over one bucket: its own; of several: the
+// launch's tiles in one contiguous range per XCD.
+MUON_DEVICE const GemmArgs& args_of(const GemmArgs& g, int mode, int& bidx, int& tm, int& tn) {
+  map_tile(g, mode, bidx, tm, tn);
+  return g;
+}
+MUON_DEVICE const GemmArgs& args_of(const GemmTab& tab, int mode, int& bidx, int& tm, int& tn) {
+  const int64_t L = xcd_tile(blockIdx.x, (int64_t)gridDim.x, 1);
+  int gi = 0;
+  while (gi + 1 < tab.n && L >= tab.tile0[gi + 1]) ++gi;
+  tile_at(tab.g[gi], mode, L - tab.tile0[gi], bidx, tm, tn);
+  return tab.g[gi];
 }
 
 template <typename OutT>
@@ -792,8 +822,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_v2_kernel(GemmArgs g) {
     if (kt + 1 < KT) issue_b(kt + 1, cs ^ 1);
     substep(a0, b0, a1, b1, aaddr(cs, 1), baddr(cs, 1));
     substep(a1, b1, a0, b0, aaddr(cs, 2), baddr(cs, 2));
-    substep(a0, b0, a1, b1, aaddr(cs, 3), baddr(cs, 3));
     if (MC != 2 && kt == kdiag) {
+      // after the first 32 k, where the other SYRK kernels add it: same bits from each
       // cin(i, j) = b(j, i): row j of the b panel, k offset i - kt*BK (4 consecutive
       // rows i of one accumulator group are 8 contiguous bytes of that row)
       mfma_to_valu_wait();
@@ -815,6 +845,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_v2_kernel(GemmArgs g) {
           }
       valu_to_mfma_wait();
     }
+    substep(a0, b0, a1, b1, aaddr(cs, 3), baddr(cs, 3));
     wait_vmcnt0();
     lds_barrier();
     if (kt + 2 < KT) issue_a(kt + 2, cs);
@@ -1007,11 +1038,9 @@ MUON_DEVICE void nn_join(bf16x8_mfma (&cx)[4], const i16x4 (&lo)[4], const i16x4
 // Persistent bf16 X' = alpha * (B X + ratio * X): 4 wavefronts (2 x 2), each owning a
 // 128 x 128 block of the 256 x 256 tile, accumulators in AGPRs (256 per lane).
 //
-// Against 8 waves of 64 x 128 (measured 2-8% slower on the same box) a wave reads 8 KB of
-// fragments from LDS per 16 MFMAs instead of 6 KB per 8, and with one wave per SIMD the DMA of
-// K-tile k + 2 is issued from inside the MFMA stream of K-tile k (B panel) and k + 1 (X panel),
-// one buffer_load ... lds after each of a substep's first 8 MFMAs, M0 stepping through the
-// destination slabs. The grid is one workgroup per CU; each walks a list of tiles with
+// Against 8 waves of 64 x 128 (measured 2-8% slower on the same box) a wave reads fewer LDS
+// bytes per MFMA, and with one wave per SIMD the DMA of K-tile k + 2 is issued from inside the
+// MFMA stream of K-tile k. The grid is one workgroup per CU; each walks a list of tiles with
 // the operand pipeline running across tile boundaries: the last two K-tiles of a tile
 // prefetch the first two of the next, so a tile's epilogue overlaps the next tile's loads.
 //
@@ -1023,11 +1052,13 @@ MUON_DEVICE void nn_join(bf16x8_mfma (&cx)[4], const i16x4 (&lo)[4], const i16x4
 // product runs 5-8% faster.
 //
 // Tiles are dealt to the 8 XCDs (workgroup b runs on XCD b % 8) in stripes of 64
-// consecutive tiles: the workgroups of one XCD share its L2 across neighbouring tiles
-// (GM = 8 tile rows per column group, as map_tile), and all XCDs work on the same
-// matrices at a time. The beta term reads the staged X panel during the
-// two K-tiles whose k range covers the wave's output rows, holds the values in 128
-// VGPRs (bf16 pairs) and adds them in the epilogue.
+// consecutive tiles: XCD x's list is stripes x, x + 8, x + 16, ... while whole rounds of 8
+// stripes remain, then an equal share of the rest, and its workgroups take every gx-th
+// tile of it. The workgroups of one XCD thus share its L2 across neighbouring tiles (GM = 8
+// tile rows per column group, as map_tile), and all XCDs work on the same matrices at a
+// time, so the operand panels their L2s miss on come from one matrix's worth of data (which
+// the Infinity Cache holds) rather than from 8 matrices (contiguous ranges per XCD: 4%
+// slower on the 4096 x 14336 bucket).
 constexpr int N4_EPB = 32 * 256;                 // epilogue staging per wave: 32 rows
 constexpr int N4_STRIPE = 64;                    // tiles per XCD stripe
 constexpr int N4_SMEM = 2 * NN_STAGEB + 4 * N4_EPB;  // 160 KiB
@@ -1038,194 +1069,6 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 MUON_DEVICE u32x4 n4_rsrc(const void* base, bool none) {
   const uint64_t a = (uint64_t)base;
   return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, none ? 0u : 0x7fffffffu, 0x00020000u};
-}
-
-#define MF(C, X, B) "v_mfma_f32_32x32x16_bf16 %[" #C "], %[" #X "], %[" #B "], %[" #C "]\n\t"
-#define TRL(D, XA, O) "ds_read_b64_tr_b16 %[" #D "], %[" #XA "] offset:%[" #O "]\n\t"
-#define N4_ACC_OUT                                                                          \
-  [c00] "+a"(acc[0][0]), [c01] "+a"(acc[0][1]), [c02] "+a"(acc[0][2]), [c03] "+a"(acc[0][3]), \
-  [c10] "+a"(acc[1][0]), [c11] "+a"(acc[1][1]), [c12] "+a"(acc[1][2]), [c13] "+a"(acc[1][3]), \
-  [c20] "+a"(acc[2][0]), [c21] "+a"(acc[2][1]), [c22] "+a"(acc[2][2]), [c23] "+a"(acc[2][3]), \
-  [c30] "+a"(acc[3][0]), [c31] "+a"(acc[3][1]), [c32] "+a"(acc[3][2]), [c33] "+a"(acc[3][3]), \
-  [nb0] "=&v"(nb[0]), [nb1] "=&v"(nb[1]), [nb2] "=&v"(nb[2]), [nb3] "=&v"(nb[3]),              \
-  [l0] "=&v"(nxl[0]), [h0] "=&v"(nxh[0]), [l1] "=&v"(nxl[1]), [h1] "=&v"(nxh[1]),              \
-  [l2] "=&v"(nxl[2]), [h2] "=&v"(nxh[2]), [l3] "=&v"(nxl[3]), [h3] "=&v"(nxh[3])
-#define N4_FRAG_IN                                                                          \
-  [cb0] "v"(cb[0]), [cb1] "v"(cb[1]), [cb2] "v"(cb[2]), [cb3] "v"(cb[3]), [cx0] "v"(cx[0]),    \
-  [cx1] "v"(cx[1]), [cx2] "v"(cx[2]), [cx3] "v"(cx[3]), [ba] "v"(ba), [x0] "v"(xa[0]),         \
-  [x1] "v"(xa[1]), [x2] "v"(xa[2]), [x3] "v"(xa[3]), [o0] "i"(XO), [o1] "i"(XO + 4 * NN_XROWB)
-
-// One k-substep of the 128 x 128 wave tile: 16 MFMAs (accumulator (fm, fn) takes X
-// fragment fn as srcA and B fragment fm as srcB) interleaved with the 12 LDS reads of
-// the next substep's fragments (X: two tr reads per fragment at xa[f] + XO and + 2 KB;
-// B: b128 at ba + 4 KB * fm), complete when the block ends.
-template <int XO>
-MUON_DEVICE void nn4_substep(f32x16 (&acc)[4][4], const bf16x8_mfma (&cb)[4],
-                             const bf16x8_mfma (&cx)[4], bf16x8_mfma (&nb)[4], i16x4 (&nxl)[4],
-                             i16x4 (&nxh)[4], uint32_t ba, const uint32_t (&xa)[4]) {
-  asm volatile(
-      TRL(l0, x0, o0) MF(c00, cx0, cb0)
-      TRL(h0, x0, o1) MF(c01, cx1, cb0)
-      TRL(l1, x1, o0) MF(c02, cx2, cb0)
-      TRL(h1, x1, o1) MF(c03, cx3, cb0)
-      TRL(l2, x2, o0) MF(c10, cx0, cb1)
-      TRL(h2, x2, o1) MF(c11, cx1, cb1)
-      TRL(l3, x3, o0) MF(c12, cx2, cb1)
-      TRL(h3, x3, o1) MF(c13, cx3, cb1)
-      "ds_read_b128 %[nb0], %[ba]\n\t" MF(c20, cx0, cb2)
-      "ds_read_b128 %[nb1], %[ba] offset:4096\n\t" MF(c21, cx1, cb2)
-      "ds_read_b128 %[nb2], %[ba] offset:8192\n\t" MF(c22, cx2, cb2)
-      "ds_read_b128 %[nb3], %[ba] offset:12288\n\t" MF(c23, cx3, cb2)
-      MF(c30, cx0, cb3) MF(c31, cx1, cb3) MF(c32, cx2, cb3) MF(c33, cx3, cb3)
-      "s_waitcnt lgkmcnt(0)"
-      : N4_ACC_OUT
-      : N4_FRAG_IN);
-}
-
-// nn4_substep plus the DMA of half a K-tile into one stage: this wave's 8 slabs of one
-// operand panel (B panel: rows 32 q + 8 wave .. +7; X panel: rows 8 q + 2 wave, +1; LDS
-// slab 4 q + wave of that panel), one buffer_load ... lds after each of the first 8
-// MFMAs. M0 holds the LDS destination; each M0 write is separated from its load by an
-// MFMA (the one wait state the hardware needs). t steps the scalar byte offset by one
-// slab group (st).
-//
-// A K-tile's two halves go out in two different substeps (the B panel of K-tile k + 2
-// right after the barrier, the X panel of K-tile k + 2 in the next substep): the 64
-// loads of one K-tile per CU, issued in one substep, queued in the load path and held
-// up the MFMAs behind them (about 37 issue cycles per load); in halves the main loop
-// takes 7-8% fewer cycles.
-#define DL "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-#define DN "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\t"
-template <int XO>
-MUON_DEVICE void nn4_substep_dma(f32x16 (&acc)[4][4], const bf16x8_mfma (&cb)[4],
-                                 const bf16x8_mfma (&cx)[4], bf16x8_mfma (&nb)[4],
-                                 i16x4 (&nxl)[4], i16x4 (&nxh)[4], uint32_t ba,
-                                 const uint32_t (&xa)[4], int vo, u32x4 rs, int so, int st,
-                                 uint32_t m0) {
-  int t;
-  asm volatile(
-      "s_mov_b32 m0, %[m0]\n\ts_mov_b32 %[t], %[so]\n\t"
-      TRL(l0, x0, o0) MF(c00, cx0, cb0) DL
-      DN TRL(h0, x0, o1) MF(c01, cx1, cb0) DL
-      DN TRL(l1, x1, o0) MF(c02, cx2, cb0) DL
-      DN TRL(h1, x1, o1) MF(c03, cx3, cb0) DL
-      DN TRL(l2, x2, o0) MF(c10, cx0, cb1) DL
-      DN TRL(h2, x2, o1) MF(c11, cx1, cb1) DL
-      DN TRL(l3, x3, o0) MF(c12, cx2, cb1) DL
-      DN TRL(h3, x3, o1) MF(c13, cx3, cb1) DL
-      "ds_read_b128 %[nb0], %[ba]\n\t" MF(c20, cx0, cb2)
-      "ds_read_b128 %[nb1], %[ba] offset:4096\n\t" MF(c21, cx1, cb2)
-      "ds_read_b128 %[nb2], %[ba] offset:8192\n\t" MF(c22, cx2, cb2)
-      "ds_read_b128 %[nb3], %[ba] offset:12288\n\t" MF(c23, cx3, cb2)
-      MF(c30, cx0, cb3) MF(c31, cx1, cb3) MF(c32, cx2, cb3) MF(c33, cx3, cb3)
-      "s_waitcnt lgkmcnt(0)"
-      : N4_ACC_OUT, [t] "=&s"(t)
-      : N4_FRAG_IN, [vo] "v"(vo), [rs] "s"(rs), [so] "s"(so), [st] "s"(st), [m0] "s"(m0)
-      : "m0", "scc", "memory");
-}
-#undef DL
-#undef DN
-
-// The B panel half of a K-tile without MFMAs (pipeline start).
-MUON_DEVICE void nn4_dma_half(int vo, u32x4 rs, int so, int st, uint32_t m0) {
-  int t;
-  asm volatile(
-      "s_mov_b32 m0, %[m0]\n\ts_mov_b32 %[t], %[so]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[t], %[t], %[st]\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %[vo], %[rs], %[t] offen lds\n\t"
-      : [t] "=&s"(t)
-      : [vo] "v"(vo), [rs] "s"(rs), [so] "s"(so), [st] "s"(st), [m0] "s"(m0)
-      : "m0", "scc", "memory");
-}
-
-#define DA "buffer_load_dwordx4 %[voa], %[rsa], %[ta] offen lds\n\t"
-#define DX "buffer_load_dwordx4 %[vox], %[rsx], %[tx] offen lds\n\t"
-#define NA "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[ta], %[ta], %[sta]\n\t"
-#define NX "s_add_u32 m0, m0, 0x1000\n\ts_add_u32 %[tx], %[tx], %[stx]\n\t"
-// The DMA of one K-tile without MFMAs (pipeline start).
-MUON_DEVICE void nn4_dma(int voa, int vox, u32x4 rsa, u32x4 rsx, int soa, int sox, int sta,
-                         int stx, uint32_t m0a, uint32_t m0x) {
-  int ta, tx;
-  asm volatile(
-      "s_mov_b32 m0, %[m0a]\n\ts_mov_b32 %[ta], %[soa]\n\ts_nop 0\n\t"
-      DA NA "s_nop 0\n\t" DA NA "s_nop 0\n\t" DA NA "s_nop 0\n\t" DA
-      NA "s_nop 0\n\t" DA NA "s_nop 0\n\t" DA NA "s_nop 0\n\t" DA NA "s_nop 0\n\t" DA
-      "s_mov_b32 m0, %[m0x]\n\ts_mov_b32 %[tx], %[sox]\n\ts_nop 0\n\t"
-      DX NX "s_nop 0\n\t" DX NX "s_nop 0\n\t" DX NX "s_nop 0\n\t" DX
-      NX "s_nop 0\n\t" DX NX "s_nop 0\n\t" DX NX "s_nop 0\n\t" DX NX "s_nop 0\n\t" DX
-      : [ta] "=&s"(ta), [tx] "=&s"(tx)
-      : [voa] "v"(voa), [vox] "v"(vox), [rsa] "s"(rsa), [rsx] "s"(rsx), [soa] "s"(soa),
-        [sox] "s"(sox), [sta] "s"(sta), [stx] "s"(stx), [m0a] "s"(m0a), [m0x] "s"(m0x)
-      : "m0", "scc", "memory");
-}
-#undef DA
-#undef DX
-#undef NA
-#undef NX
-
-template <int XO>
-MUON_DEVICE void nn4_frag_load(bf16x8_mfma (&nb)[4], i16x4 (&nxl)[4], i16x4 (&nxh)[4], uint32_t ba,
-                               const uint32_t (&xa)[4]) {
-  asm volatile(
-      TRL(l0, x0, o0) TRL(h0, x0, o1) TRL(l1, x1, o0) TRL(h1, x1, o1)
-      TRL(l2, x2, o0) TRL(h2, x2, o1) TRL(l3, x3, o0) TRL(h3, x3, o1)
-      "ds_read_b128 %[nb0], %[ba]\n\t"
-      "ds_read_b128 %[nb1], %[ba] offset:4096\n\t"
-      "ds_read_b128 %[nb2], %[ba] offset:8192\n\t"
-      "ds_read_b128 %[nb3], %[ba] offset:12288\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : [nb0] "=&v"(nb[0]), [nb1] "=&v"(nb[1]), [nb2] "=&v"(nb[2]), [nb3] "=&v"(nb[3]),
-        [l0] "=&v"(nxl[0]), [h0] "=&v"(nxh[0]), [l1] "=&v"(nxl[1]), [h1] "=&v"(nxh[1]),
-        [l2] "=&v"(nxl[2]), [h2] "=&v"(nxh[2]), [l3] "=&v"(nxl[3]), [h3] "=&v"(nxh[3])
-      : [ba] "v"(ba), [x0] "v"(xa[0]), [x1] "v"(xa[1]), [x2] "v"(xa[2]), [x3] "v"(xa[3]),
-        [o0] "i"(XO), [o1] "i"(XO + 4 * NN_XROWB));
-}
-#undef MF
-#undef TRL
-#undef N4_ACC_OUT
-#undef N4_FRAG_IN
-
-// X(i, j .. j+3) for the accumulators of rows H0, H0 + 1 (panel row k = h*32 + lane%32,
-// columns 128 wn + 32 fn + 8 rg + 4 (lane/32)) from the staged X panel at sx, as bf16
-// pairs. The LDS base is laundered so the lane addresses are formed here and not kept
-// live across the main loop.
-template <int H0>
-MUON_DEVICE void nn4_beta_rows(u32x2 (&xb)[4][4][4], uint32_t sx, int wn, int fr, int fh) {
-  asm volatile("" : "+v"(sx));
-  const uint32_t base = sx + fr * NN_XROWB + wn * 256 + fh * 8;
-#pragma unroll
-  for (int fn = 0; fn < 4; ++fn) {
-    // logical 16-byte chunk 16 wn + 4 fn + rg sits at position ^ ((k & 3) << 2)
-    const uint32_t b2 = base + (((fn ^ (fr & 3)) << 2) << 4);
-    asm volatile(
-        "ds_read_b64 %0, %8 offset:0\n\t"
-        "ds_read_b64 %1, %8 offset:16\n\t"
-        "ds_read_b64 %2, %8 offset:32\n\t"
-        "ds_read_b64 %3, %8 offset:48\n\t"
-        "ds_read_b64 %4, %8 offset:%9\n\t"
-        "ds_read_b64 %5, %8 offset:%10\n\t"
-        "ds_read_b64 %6, %8 offset:%11\n\t"
-        "ds_read_b64 %7, %8 offset:%12\n\t"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(xb[H0][fn][0]), "=&v"(xb[H0][fn][1]), "=&v"(xb[H0][fn][2]),
-          "=&v"(xb[H0][fn][3]), "=&v"(xb[H0 + 1][fn][0]), "=&v"(xb[H0 + 1][fn][1]),
-          "=&v"(xb[H0 + 1][fn][2]), "=&v"(xb[H0 + 1][fn][3])
-        : "v"(b2), "i"(32 * NN_XROWB), "i"(32 * NN_XROWB + 16), "i"(32 * NN_XROWB + 32),
-          "i"(32 * NN_XROWB + 48));
-  }
 }
 
 // Tile t of the launch -> (matrix, row origin, column origin); GM tile rows per column
@@ -1242,247 +1085,20 @@ MUON_DEVICE void nn4_tile(const GemmArgs& g, int t, int& bidx, int64_t& arow0, i
   bcol0 = (int64_t)(local / gsz) * 256;
 }
 
-__global__ __launch_bounds__(256, 1) void gemm_bf16_nn4_kernel(GemmArgs g) {
-  constexpr int FM = 4, FN = 4, WM = 128, WN = 128;
-  extern __shared__ __align__(16) uint8_t smem[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-
-  // this workgroup's tiles: XCD x's list holds tcount tiles and its gx workgroups take
-  // every gx-th one starting at their index l within the XCD. The list: stripes x, x + 8,
-  // x + 16, ... of N4_STRIPE consecutive tiles while whole rounds of 8 stripes remain,
-  // then an equal share of the rest. All XCDs thus work on the same matrices at a time,
-  // so the operand panels their L2s miss on come from one matrix's worth of data (which
-  // the Infinity Cache holds) rather than from 8 matrices (contiguous ranges per XCD:
-  // 4% slower on the 4096 x 14336 bucket).
-  const int G = gridDim.x, T = g.tiles_total;
-  const int x = blockIdx.x & 7, l = blockIdx.x >> 3;
-  const int gx = (G >> 3) + (x < (G & 7) ? 1 : 0);
-  const int nfull = T / (8 * N4_STRIPE) * N4_STRIPE;  // tiles per XCD in whole rounds
-  const int rq = (T - 8 * nfull) >> 3, rr = (T - 8 * nfull) & 7;
-  const int tcount = nfull + rq + (x < rr ? 1 : 0);
-  auto tile_of = [&](int i) {
-    return i < nfull ? ((i / N4_STRIPE) * 8 + x) * N4_STRIPE + i % N4_STRIPE
-                     : 8 * nfull + x * rq + min(x, rr) + (i - nfull);
-  };
-  int li = l;
-  if (li >= tcount) return;
-
-  const int lda_b = (int)(g.lda * 2), ldx_b = (int)(g.ldb * 2);
-  // DMA lanes: B panel row 8 wave + lane/8 (+ 32 q), logical chunk (lane%8) ^ kswz(row);
-  // X panel row 2 wave + lane/32 (+ 8 q), chunk (lane%32) ^ ((row & 3) << 2)
-  const int ra_in = wave * 8 + (lane >> 3);
-  const int voa = ra_in * lda_b + (((lane & 7) ^ kswz(ra_in)) << 4);
-  const int rx_in = wave * 2 + (lane >> 5);
-  const int vox = rx_in * ldx_b + (((lane & 31) ^ ((rx_in & 3) << 2)) << 4);
-  const int sta = 32 * lda_b, stx = 8 * ldx_b;
-  const bf16_t* const A0 = (const bf16_t*)g.a;
-  const bf16_t* const X0 = (const bf16_t*)g.b;
-
-  // B fragment rows (k contiguous, as gemm_bf16_v2_kernel) and X fragment tr-read offsets:
-  // group g = lane/16, r = lane%16 points at panel row 8 (g/2) + r/4 (+ 16 ks, + 4 for
-  // the high half), column 128 wn + 32 f + 16 (g%2) + 4 (r%4)
-  const int fr = lane & 31, fh = lane >> 5;
-  int foff[4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) foff[ks] = fr * V2_ROWB + (((ks * 2 + fh) ^ kswz(fr)) << 4);
-  const int abase = wm * WM * V2_ROWB;
-  const int tg = lane >> 4, trr = lane & 15, ts = trr >> 2;
-  uint32_t xoff[4];
-#pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    const int chunk = wn * 16 + ((f ^ ts) << 2) + (tg & 1) * 2 + ((trr & 3) >> 1);
-    xoff[f] = NN_ATILEB + (8 * (tg >> 1) + ts) * NN_XROWB + chunk * 16 + (trr & 1) * 8;
-  }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  auto baddr = [&](int st, int ks) -> uint32_t { return lds0 + st * NN_STAGEB + abase + foff[ks]; };
-  uint32_t xa[4];
-  auto set_xa = [&](int st) {
-#pragma unroll
-    for (int f = 0; f < 4; ++f) xa[f] = lds0 + st * NN_STAGEB + xoff[f];
-  };
-  const uint32_t m0w = lds0 + wave * 1024;
-  // even: the last two K-tiles of a tile prefetch the next tile's first two into stages
-  // (KT - 2) & 1 and (KT - 1) & 1, and every tile starts reading stage 0
-  const int KT = (int)(g.K / V2_BK);
-
-  // current tile and its descriptors; the next tile's (num_records 0 if none)
-  int bidx;
-  int64_t arow0, bcol0;
-  nn4_tile(g, tile_of(li), bidx, arow0, bcol0);
-  u32x4 rsa = n4_rsrc(A0 + (int64_t)bidx * g.sa + arow0 * g.lda, false);
-  u32x4 rsx = n4_rsrc(X0 + (int64_t)bidx * g.sb + bcol0, false);
-
-  bf16x8_mfma b0[FM], b1[FM], x0[FN], x1[FN];
-  i16x4 xl[FN], xh[FN];
-  nn4_dma(voa, vox, rsa, rsx, 0, 0, sta, stx, m0w, m0w + NN_ATILEB);
-  wait_vmcnt0();
-  lds_barrier();
-  // K-tile 1: the B panel now, the X panel with the first substep of K-tile 0
-  nn4_dma_half(voa, rsa, V2_ROWB, sta, m0w + NN_STAGEB);
-  set_xa(0);
-  nn4_frag_load<0>(b0, xl, xh, baddr(0, 0), xa);
-  nn_join(x0, xl, xh);
-
-  f32x16 acc[FM][FN];
-  for (;;) {
-    const int lnext = li + gx;
-    const bool has_next = lnext < tcount;
-    int nbidx = 0;
-    int64_t narow0 = 0, nbcol0 = 0;
-    if (has_next) nn4_tile(g, tile_of(lnext), nbidx, narow0, nbcol0);
-    const u32x4 rsa_n = n4_rsrc(A0 + (int64_t)nbidx * g.sa + narow0 * g.lda, !has_next);
-    const u32x4 rsx_n = n4_rsrc(X0 + (int64_t)nbidx * g.sb + nbcol0, !has_next);
-
-    float alpha = g.alpha, beta = g.beta;
-    if (g.scale_mode == 1) {
-      const float sc = g.scale[bidx];
-      alpha *= sc;
-      beta *= sc;
-    }
-    const float ratio = beta != 0.0f ? beta / alpha : 0.0f;
-    // the wave's 128 output rows are the k rows of K-tiles kd0 and kd0 + 1
-    const int kd0 = ratio != 0.0f ? (int)((arow0 + wm * WM) / V2_BK) : -8;
-
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    u32x2 xb[FM][FN][4];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) xb[i][j][r] = u32x2{0u, 0u};
-
-    int kt = 0;
-    do {
-      const int cs = kt & 1;
-      set_xa(cs);
-      // the X panel of K-tile kt + 1 of this tile (or K-tile 0 of the next) into stage
-      // cs ^ 1; its B panel went out with the previous DMA substep
-      const bool c1 = kt + 1 < KT;
-      const int k1 = c1 ? kt + 1 : kt + 1 - KT;
-      nn4_substep_dma<1 * 16 * NN_XROWB>(acc, b0, x0, b1, xl, xh, baddr(cs, 1), xa, vox,
-                                         c1 ? rsx : rsx_n, k1 * V2_BK * ldx_b, stx,
-                                         m0w + (cs ^ 1) * NN_STAGEB + NN_ATILEB);
-      nn_join(x1, xl, xh);
-      nn4_substep<2 * 16 * NN_XROWB>(acc, b1, x1, b0, xl, xh, baddr(cs, 2), xa);
-      nn_join(x0, xl, xh);
-      nn4_substep<3 * 16 * NN_XROWB>(acc, b0, x0, b1, xl, xh, baddr(cs, 3), xa);
-      nn_join(x1, xl, xh);
-      if (kt == kd0) nn4_beta_rows<0>(xb, lds0 + cs * NN_STAGEB + NN_ATILEB, wn, fr, fh);
-      if (kt == kd0 + 1) nn4_beta_rows<2>(xb, lds0 + cs * NN_STAGEB + NN_ATILEB, wn, fr, fh);
-      wait_vmcnt0();
-      lds_barrier();
-      // the B panel of K-tile kt + 2 of this tile, or K-tile kt + 2 - KT of the next,
-      // into stage cs
-      const bool c2 = kt + 2 < KT;
-      const int k2 = c2 ? kt + 2 : kt + 2 - KT;
-      set_xa(cs ^ 1);
-      nn4_substep_dma<0>(acc, b1, x1, b0, xl, xh, baddr(cs ^ 1, 0), xa, voa, c2 ? rsa : rsa_n,
-                         k2 * V2_ROWB, sta, m0w + cs * NN_STAGEB);
-      nn_join(x0, xl, xh);
-    } while (++kt < KT);
-    mfma_to_valu_wait();
-
-    // epilogue: accumulator (fm, fn) element 4 rg + q is X'(i, j + q) with
-    // i = 128 wm + 32 fm + lane%32, j = 128 wn + 32 fn + 8 rg + 4 (lane/32). Each 32-row
-    // block fm goes through the wave's LDS staging rows (16-byte chunk k of row r kept at
-    // chunk k ^ (r & 15), so both the 8-byte writes and the 16-byte reads are free of
-    // bank conflicts), then out as 4 whole rows of 256 bytes per non-temporal store.
-    // The staging rows are the wave's own and LDS serves one wave's accesses in order.
-    bf16_t* outw = (bf16_t*)g.out + (int64_t)bidx * g.so + (arow0 + wm * WM) * g.ldo + bcol0 + wn * WN;
-    const __amdgpu_buffer_rsrc_t rso =
-        __builtin_amdgcn_make_buffer_rsrc((void*)outw, 0, 0x7fffffff, 0x00020000);
-    const int ldo_b = (int)(g.ldo * 2);
-    const uint32_t ep = lds0 + 2 * NN_STAGEB + wave * N4_EPB;
-    const uint32_t epw = ep + fr * 256 + fh * 8;   // row fr, this lane's 8-byte half
-    const uint32_t epr = ep + (lane >> 4) * 256;  // rows lane/16 + 4 i
-    const int vor = (lane >> 4) * ldo_b + (lane & 15) * 16;
-    // valid extents from this lane's first row / column (zeros are stored beyond);
-    // most tiles lie inside both and take the unmasked path
-    const bool full = arow0 + 256 <= g.Mv && bcol0 + 256 <= g.Nv;
-    const int rem_i = (int)g.Mv - (int)(arow0 + wm * WM + fr);
-    const int rem_j = (int)g.Nv - (int)(bcol0 + wn * WN + fh * 4);
-    auto emit = [&](auto masked) {
-#pragma unroll
-      for (int fm = 0; fm < FM; ++fm) {
-#pragma unroll
-        for (int fn = 0; fn < FN; ++fn) {
-          // one accumulator at a time out of the AGPRs
-          f32x16 av;
-          asm volatile("" : "=v"(av) : "0"(acc[fm][fn]));
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            const u32x2 xw = xb[fm][fn][rg];
-            f2x v01 = {alpha * (av[rg * 4 + 0] + ratio * __uint_as_float(xw.x << 16)),
-                       alpha * (av[rg * 4 + 1] + ratio * __uint_as_float(xw.x & 0xffff0000u))};
-            f2x v23 = {alpha * (av[rg * 4 + 2] + ratio * __uint_as_float(xw.y << 16)),
-                       alpha * (av[rg * 4 + 3] + ratio * __uint_as_float(xw.y & 0xffff0000u))};
-            if (decltype(masked)::value) {
-              const int jq = fn * 32 + rg * 8;
-              const bool vi = fm * 32 < rem_i;
-              v01.x = vi && jq + 0 < rem_j ? v01.x : 0.0f;
-              v01.y = vi && jq + 1 < rem_j ? v01.y : 0.0f;
-              v23.x = vi && jq + 2 < rem_j ? v23.x : 0.0f;
-              v23.y = vi && jq + 3 < rem_j ? v23.y : 0.0f;
-            }
-            const u32x2 w = {__builtin_bit_cast(uint32_t, __builtin_convertvector(v01, bf2x)),
-                             __builtin_bit_cast(uint32_t, __builtin_convertvector(v23, bf2x))};
-            // addresses are formed here rather than hoisted into registers for the loop
-            uint32_t ea = epw, fx = fr & 15;
-            asm volatile("" : "+v"(ea), "+v"(fx));
-            *(u32x2 __attribute__((address_space(3)))*)(ea + (((4 * fn + rg) ^ fx) << 4)) = w;
-          }
-        }
-        uint32_t ra = epr, lc = lane & 15, lr = lane >> 4;
-        int vs = vor;
-        asm volatile("" : "+v"(ra), "+v"(vs), "+v"(lc), "+v"(lr));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const uint32_t c = lc ^ ((4 * i + lr) & 15);
-          const u32x4 q4 = *(const u32x4 __attribute__((address_space(3)))*)(ra + i * 1024 + (c << 4));
-          // aux 2: non-temporal
-          __builtin_amdgcn_raw_buffer_store_b128(q4, rso, vs + i * 4 * ldo_b, fm * 32 * ldo_b, 2);
-        }
-      }
-    };
-    if (full)
-      emit(std::false_type{});
-    else
-      emit(std::true_type{});
-    if (!has_next) break;
-    li = lnext;
-    bidx = nbidx;
-    arow0 = narow0;
-    bcol0 = nbcol0;
-    rsa = rsa_n;
-    rsx = rsx_n;
-  }
-}
-
-// ----------------------------------------------------------------------------------
-// The persistent B X kernel on 16 x 16 x 32 MFMAs, for K of at least 768.
-//
-// Same tiling, waves, LDS layout, tile order and epilogue staging as gemm_bf16_nn4_kernel;
-// the wave's 128 x 128 block is 8 x 8 accumulators of 16 x 16 (AGPRs) and a K-tile is two
-// 32-k substeps of 64 MFMAs. A single wave issues v_mfma_f32_32x32x16_bf16 at most every 32
-// cycles and each 16-byte fragment read between them costs it issue time; with
+// The kernel: the wave's 128 x 128 block is 8 x 8 accumulators of 16 x 16 (AGPRs) and a K-tile
+// is two 32-k substeps of 64 MFMAs. A single wave issues v_mfma_f32_32x32x16_bf16 at most
+// every 32 cycles and each 16-byte fragment read between them costs it issue time; with
 // v_mfma_f32_16x16x32_bf16 the same LDS bytes per FLOP ride along at almost no cost: a
 // probe loop with this kernel's reads, DMA and barrier took 35.7 cycles per
-// 32 x 32 x 16-equivalent against about 48 for the 32 x 32 x 16 loop.
+// 32 x 32 x 16-equivalent against about 48 for the 32 x 32 x 16 loop. (On 32 x 32 x 16 MFMAs
+// B X of 256 matrices of 512 x 1024 took 178 us against 167, of 200 of 640 x 2560 590 against
+// 549, of 512 of 128 x 1024 96 against 93.)
 //
 // Fragments (lane l, r = l % 16, g = l / 16): srcA is X^T, 8 consecutive k (two tr reads)
 // of column 16 fj + r; srcB is B, 8 consecutive k (one b128) of row 16 fi + r; the
 // accumulator register q of block (fi, fj) is X'(16 fi + r, 16 fj + 4 g + q).
 //
-// The X panel's chunk swizzle adds row bit 3 to gemm_bf16_nn4_kernel's: chunk c of row k sits
-// at c ^ ((k & 3) << 2) ^ (((k >> 3) & 1) << 1). A transposing read serves 32 lanes at a time,
+// The X panel's chunk swizzle has row bit 3 in it: chunk c of row k sits at c ^ ((k & 3) << 2) ^ (((k >> 3) & 1) << 1). A transposing read serves 32 lanes at a time,
 // lanes 0-15 from rows 8 g' .. +3 and lanes 16-31 from rows 8 g' + 8 .. +11 (g' even); with
 // the low-bit swizzle alone both groups hit the same 32 banks (35% of LDS-active cycles were
 // bank conflicts), with bit 3 they use the other 32. The DMA takes the row parity of each X
@@ -1491,8 +1107,7 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_nn4_kernel(GemmArgs g) {
 // The beta term is added during the two K-tiles whose k range is the wave's rows (no
 // registers hold X values through the loop, which the double-buffered fragments need), by
 // 32 more MFMAs per substep (n16_beta), so the accumulators never leave their AGPRs; those
-// two K-tiles are peeled off the loop. It takes its own K-loop structure and per-tile work,
-// so below K = 768 (where that work weighs more) gemm_bf16_nn4_kernel is used instead.
+// two K-tiles are peeled off the loop.
 #define M16(C, X, B) "v_mfma_f32_16x16x32_bf16 %[" #C "], %[" #X "], %[" #B "], %[" #C "]\n\t"
 #define N16_OUT(ACC)                                                                      \
   [c0] "+a"(ACC[0]), [c1] "+a"(ACC[1]), [c2] "+a"(ACC[2]), [c3] "+a"(ACC[3]),               \
@@ -1692,10 +1307,7 @@ MUON_DEVICE void n16_substep_dma(f32x4 (&acc)[8][8], const bf16x8_mfma (&cb)[8],
 // MFMAs, whose latency it does not see, and the moves raced their results: B X then differed
 // by an ulp from run to run.) db[par][part]: lane l (r = l%16, g = l/16) holds B(k, n) for
 // k = 8 g .. 8 g + 7, n = r: part at k = 16 par + r, else zero.
-MUON_DEVICE void n16_beta_frags(float ratio, int lane, bf16x8_mfma (&db)[2][2]) {
-  const float hi = bf16_to_f32(f32_to_bf16(ratio));
-  const float lo = ratio - hi;
-  const uint32_t parts[2] = {(uint32_t)f32_to_bf16(hi), (uint32_t)f32_to_bf16(lo)};
+MUON_DEVICE void n16_diag_frags(const uint32_t (&parts)[2], int lane, bf16x8_mfma (&db)[2][2]) {
   const int r = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int par = 0; par < 2; ++par)
@@ -1708,6 +1320,22 @@ MUON_DEVICE void n16_beta_frags(float ratio, int lane, bf16x8_mfma (&db)[2][2]) 
         w[d] = (e == 2 * d ? parts[pt] : 0u) | (e == 2 * d + 1 ? parts[pt] << 16 : 0u);
       db[par][pt] = __builtin_bit_cast(bf16x8_mfma, u32x4{w[0], w[1], w[2], w[3]});
     }
+}
+MUON_DEVICE void n16_beta_frags(float ratio, int lane, bf16x8_mfma (&db)[2][2]) {
+  const float hi = bf16_to_f32(f32_to_bf16(ratio));
+  const uint32_t parts[2] = {(uint32_t)f32_to_bf16(hi), (uint32_t)f32_to_bf16(ratio - hi)};
+  n16_diag_frags(parts, lane, db);
+}
+// The third part of ratio (and zero): hi + lo + third is the fp32 value. Products of K below
+// BETA3_K take it too: at two parts the coefficient's 2^-17 error changes the rounding of enough
+// elements of X' that the update of a 256 x 512 matrix ends 9.1e-3 to 9.6e-3 from the iteration
+// with the exact coefficient instead of 7.3e-3 to 8.2e-3 (768 x 2304: 7.1e-3 against 5.9e-3).
+constexpr int BETA3_K = 768;
+MUON_DEVICE void n16_beta_third(float ratio, int lane, bf16x8_mfma (&db)[2][2]) {
+  const float hi = bf16_to_f32(f32_to_bf16(ratio));
+  const float lo = bf16_to_f32(f32_to_bf16(ratio - hi));
+  const uint32_t parts[2] = {(uint32_t)f32_to_bf16((ratio - hi) - lo), 0u};
+  n16_diag_frags(parts, lane, db);
 }
 
 #define M16(C, X, B) "v_mfma_f32_16x16x32_bf16 %[" #C "], %[" #X "], %[" #B "], %[" #C "]\n\t"
@@ -1751,7 +1379,8 @@ MUON_DEVICE void n16_beta(f32x4 (&acc)[8][8], const bf16x8_mfma (&cx)[8],
 // (parameter row j = X' column j), computed with swapped MFMA operands so the accumulators
 // hold parameter rows.
 // MODE (APPLY 1, 2): the form of the apply, from the uniform wd and cautious (below).
-template <int APPLY, int MODE = 0>
+// B3: K below BETA3_K, the beta term in three parts.
+template <int APPLY, int MODE = 0, bool B3 = false>
 __global__ __launch_bounds__(256, 1) void gemm_bf16_nn16_kernel(GemmArgs g, MuonApply ap) {
   constexpr int WM = 128, WN = 128;
   constexpr bool SW = APPLY == 2;
@@ -1871,6 +1500,10 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_nn16_kernel(GemmArgs g, Muon
         bf16x8_mfma db[2][2];
         n16_beta_frags(ratio, lane, db);
         n16_beta<FB, SW>(acc, x0, db);
+        if constexpr (B3) {
+          n16_beta_third(ratio, lane, db);
+          n16_beta<FB, SW>(acc, x0, db);
+        }
       }
       n16_join(x1, xl, xh);
       wait_vmcnt0();
@@ -1886,6 +1519,10 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_nn16_kernel(GemmArgs g, Muon
         bf16x8_mfma db[2][2];
         n16_beta_frags(ratio, lane, db);
         n16_beta<FB + 2, SW>(acc, x1, db);
+        if constexpr (B3) {
+          n16_beta_third(ratio, lane, db);
+          n16_beta<FB + 2, SW>(acc, x1, db);
+        }
       }
       n16_join(x0, xl, xh);
     };
@@ -2553,12 +2190,13 @@ MUON_DEVICE void h16_frag_load(h16_frags& n, uint32_t aa, uint32_t ba) {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
-__global__ __launch_bounds__(256, 2) void gemm_bf16_s16h_kernel(GemmArgs g) {
+template <typename Args>
+__global__ __launch_bounds__(256, 2) void gemm_bf16_s16h_kernel(Args args) {
   constexpr int NW = 4, WM = 64, WN = 64;
   extern __shared__ __align__(16) uint8_t smem[];
 
   int bidx, tm, tn;
-  map_tile(g, MODE_SYRK, bidx, tm, tn);
+  const GemmArgs& g = args_of(args, MODE_SYRK, bidx, tm, tn);
   const int64_t arow0 = (int64_t)tm * 128, brow0 = (int64_t)tn * 128;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2879,6 +2517,389 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
                                MODE == MODE_SYRK && tm == tn);
 }
 
+// ----------------------------------------------------------------------------------
+// Products of small and medium launches on TM x TM tiles (TM = 128 or 64), several buckets per
+// launch (GemmTab): four waves of (TM / 2) x (TM / 2), 16 x 16 x 32 MFMAs. With 256-row tiles and
+// one workgroup per CU such a launch fills a fraction of the CUs (a 256 x 512 matrix: one
+// workgroup for X X^T, two for B X) and its time is that of one workgroup's K loop and
+// epilogue: 9.7 us for X X^T and 14.6 us for B X of that matrix.
+// A K-tile is 64 k. TM = 128: two stages of 32 KB, two workgroups per CU. TM = 64: four stages of
+// 16 KB, two workgroups per CU: the loads of K-tiles k + 1 .. k + 3 are under way while K-tile k
+// is multiplied, since a launch of one small workgroup per CU has nothing else to hide their
+// latency with. Operands stream to LDS by `buffer_load_dwordx4 ... lds`, rows of K-contiguous
+// panels swizzled with kswz.
+// (A 128-row tile_syrk_kernel took 169 us against gemm_bf16_s16h_kernel's 155 for A A of two
+// matrices of 4096 rows and 17 against 18 for a dozen of 768: the SYRK's 128-row tiles stay
+// that kernel's.)
+// Each output element sees the MFMAs of gemm_bf16_s16_kernel / gemm_bf16_nn16_kernel in the same
+// order, the beta term at the same place, so its bits do not depend on the kernel that
+// serves a launch.
+template <int TM>
+struct TileK {
+  static constexpr int NS = TM == 64 ? 4 : 2;
+  static constexpr int PANELB = TM * V2_ROWB;  // either operand's panel of one K-tile
+  static constexpr int STAGEB = 2 * PANELB;
+  static constexpr int SMEM = NS * STAGEB;
+  static constexpr int F = TM / 32;            // 16-row blocks per wave and side
+  static constexpr int LOADS = TM / 32;        // 1 KB loads per wave and panel
+  static constexpr int PITCH = TM + 8;         // epilogue staging row (elements)
+  static_assert(TM * PITCH * 2 <= SMEM, "the staging tile fits the stages");
+};
+
+MUON_DEVICE void tile_dma(int vo, u32x4 rs, int so, uint32_t m0) {
+  asm volatile("s_mov_b32 m0, %[mz]\n\ts_nop 0\n\tbuffer_load_dwordx4 %[vo], %[rs], %[so] offen lds\n\t"
+               :
+               : [vo] "v"(vo), [rs] "s"(rs), [so] "s"(so), [mz] "s"(m0)
+               : "m0", "memory");
+}
+
+// A = alpha X X^T (K = n) or B = alpha (A A + ratio A): upper-triangle tiles, mirrored.
+template <int TM, typename Args>
+__global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
+  typedef TileK<TM> C;
+  constexpr int F = C::F, WM = TM / 2;
+  extern __shared__ __align__(16) uint8_t smem[];
+  int bidx, tm, tn;
+  const GemmArgs& g = args_of(args, MODE_SYRK, bidx, tm, tn);
+  const int row0 = tm * TM, col0 = tn * TM;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const bool diag = tm == tn;  // one panel serves both operands
+  const bf16_t* A = (const bf16_t*)g.a + (int64_t)bidx * g.sa;
+  const u32x4 rsa = n4_rsrc(A + (int64_t)row0 * g.lda, false);
+  const u32x4 rsb = n4_rsrc(A + (int64_t)col0 * g.lda, diag);
+  const u32x4 rs_none = n4_rsrc(A, true);
+  const int lda_b = (int)(g.lda * 2);
+  // load q of this wave: rows (4 q + wave) * 8 + lane / 8 of the panel, 16-byte chunk lane % 8
+  const int r_in = wave * 8 + (lane >> 3);
+  const int vo = r_in * lda_b + (((lane & 7) ^ kswz(r_in)) << 4);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  const int KT = (int)(g.K / V2_BK);
+  auto issue = [&](int kt, int st) {
+    const bool on = kt < KT;
+    const int kb = on ? kt * V2_ROWB : 0;
+    const uint32_t m0 = lds0 + st * C::STAGEB + wave * 1024;
+    const u32x4 pa = on ? rsa : rs_none, pb = on ? rsb : rs_none;
+#pragma unroll
+    for (int q = 0; q < C::LOADS; ++q) {
+      tile_dma(vo, pa, kb + q * 32 * lda_b, m0 + q * 4096);
+      tile_dma(vo, pb, kb + q * 32 * lda_b, m0 + C::PANELB + q * 4096);
+    }
+  };
+  float alpha = g.alpha, beta = g.beta;
+  if (g.scale_mode == 2) {
+    const float s = g.scale[bidx];
+    alpha *= s * s;
+  }
+  const float ratio = beta != 0.0f ? beta / alpha : 0.0f;
+  // K-tile whose k range holds this wave's output rows (of a 64-row wave exactly, of a 32-row
+  // one a half of it)
+  const int kdiag = ratio != 0.0f ? (row0 + wm * WM) / V2_BK : -1;
+  const int koff = (row0 + wm * WM) & 63;  // the rows' place in it
+
+  f32x4 acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int fr = lane & 15, fg = lane >> 4;
+  const int abase = wm * WM * V2_ROWB, bbase = (diag ? 0 : C::PANELB) + wn * WM * V2_ROWB;
+#pragma unroll
+  for (int t = 0; t < C::NS - 1; ++t) issue(t, t);
+  int st = 0;
+  for (int kt = 0; kt < KT; ++kt) {
+    // 2 LOADS loads per K-tile: those of K-tiles kt + 1 .. kt + NS - 2 may still be under way
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * C::LOADS * (C::NS - 2)) : "memory");
+    lds_barrier();
+    issue(kt + C::NS - 1, st == 0 ? C::NS - 1 : st - 1);
+    const uint8_t* sp = smem + st * C::STAGEB;
+    bf16x8_mfma a[2][F], b[2][F];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int off = fr * V2_ROWB + (((ks * 4 + fg) ^ kswz(fr)) << 4);
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        a[ks][f] = __builtin_bit_cast(bf16x8_mfma, *(const uint4*)(sp + abase + f * 16 * V2_ROWB + off));
+        b[ks][f] = __builtin_bit_cast(bf16x8_mfma, *(const uint4*)(sp + bbase + f * 16 * V2_ROWB + off));
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][i], b[ks][j], acc[i][j], 0, 0, 0);
+      if (ks == 0 && kt == kdiag) {
+        // cin(i, j) = b(j, i): row j of the b panel, k offset of row i
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+          for (int j = 0; j < F; ++j) {
+            const int k = koff + i * 16 + fg * 4;
+            const uint2 w = *(const uint2*)(sp + bbase + (j * 16 + fr) * V2_ROWB +
+                                            (((k >> 3) ^ kswz(fr)) << 4) + (k & 7) * 2);
+            acc[i][j][0] += ratio * __uint_as_float(w.x << 16);
+            acc[i][j][1] += ratio * __uint_as_float(w.x & 0xffff0000u);
+            acc[i][j][2] += ratio * __uint_as_float(w.y << 16);
+            acc[i][j][3] += ratio * __uint_as_float(w.y & 0xffff0000u);
+          }
+      }
+    }
+    st = st + 1 == C::NS ? 0 : st + 1;
+  }
+  wait_vmcnt0();
+  lds_barrier();
+
+  // epilogue: accumulator (i, j) element q is C(16 i + 4 fg + q, 16 j + fr) of the wave's block.
+  // The tile goes through LDS transposed (the mirror half, whole rows of the output; 4
+  // consecutive rows of one column per lane) and then row-major.
+  bf16_t* T = (bf16_t*)smem;
+  bf16_t* out = (bf16_t*)g.out + (int64_t)bidx * g.so;
+  const int mv = (int)g.Mv;
+  uint32_t hv[F][F][2];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int r = row0 + wm * WM + i * 16 + fg * 4 + 2 * h, c = col0 + wn * WM + j * 16 + fr;
+        const f2x v = {alpha * acc[i][j][2 * h], alpha * acc[i][j][2 * h + 1]};
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf2x));
+        // zeros outside the valid extent, so that the padding stays zero
+        hv[i][j][h] = w & ((c < mv && r < mv ? 0x0000ffffu : 0u) | (c < mv && r + 1 < mv ? 0xffff0000u : 0u));
+      }
+  constexpr int CH = TM / 8, ROWS = 256 / CH;  // 16-byte chunks per row, rows per store
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+      *(uint2*)(T + (wn * WM + j * 16 + fr) * C::PITCH + wm * WM + i * 16 + fg * 4) =
+          make_uint2(hv[i][j][0], hv[i][j][1]);
+  lds_barrier();
+  if (!diag) {
+#pragma unroll
+    for (int it = 0; it < TM / ROWS; ++it) {
+      const int jl = it * ROWS + tid / CH, c = tid % CH * 8;
+      *(uint4*)(out + (int64_t)(col0 + jl) * g.ldo + row0 + c) = *(const uint4*)(T + jl * C::PITCH + c);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+      for (int j = 0; j < F; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          T[(wm * WM + i * 16 + fg * 4 + q) * C::PITCH + wn * WM + j * 16 + fr] =
+              (bf16_t)(hv[i][j][q >> 1] >> (16 * (q & 1)));
+    lds_barrier();
+  }
+  // (a diagonal tile stays transposed: row il of the output takes, at column c, the upper
+  // element, (min, max) of its indices, which the stage holds at [max][min])
+#pragma unroll
+  for (int it = 0; it < TM / ROWS; ++it) {
+    const int il = it * ROWS + tid / CH, c = tid % CH * 8;
+    uint4 w;
+    if (!diag) {
+      w = *(const uint4*)(T + il * C::PITCH + c);
+    } else {
+      uint16_t e[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        e[q] = c + q > il ? T[(c + q) * C::PITCH + il] : T[il * C::PITCH + c + q];
+      __builtin_memcpy(&w, e, 16);
+    }
+    *(uint4*)(out + (int64_t)(row0 + il) * g.ldo + col0 + c) = w;
+  }
+}
+
+// X' = alpha (B X + ratio X). PDT < 0: X' stored. PDT >= 0 (the last iteration): each element of
+// X', rounded to bf16, is the update of one parameter element of type PDT, applied as the
+// post-pass does (apply_elem) and the parameter written back; SW (tall parameters: their rows
+// are columns of X') swaps the MFMA operands, so that the staged tile is the parameter's.
+// Accumulator (i, j) element q is X'(16 i + fr, 16 j + 4 fg + q) of the wave's block, with SW
+// X'(16 i + 4 fg + q, 16 j + fr).
+template <int TM, int PDT, bool SW, typename Args>
+__global__ __launch_bounds__(256, 2) void tile_bx_kernel(Args args, MuonApply ap) {
+  typedef TileK<TM> C;
+  constexpr int F = C::F, WM = TM / 2, XR = TM * 2, XCH = XR / 16;  // X panel: 64 rows of XR bytes
+  extern __shared__ __align__(16) uint8_t smem[];
+  int bidx, tm, tn;
+  const GemmArgs& g = args_of(args, MODE_GEMM, bidx, tm, tn);
+  const int row0 = tm * TM, col0 = tn * TM;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const bf16_t* A = (const bf16_t*)g.a + (int64_t)bidx * g.sa + (int64_t)row0 * g.lda;
+  const bf16_t* X = (const bf16_t*)g.b + (int64_t)bidx * g.sb + col0;
+  const u32x4 rsa = n4_rsrc(A, false), rsx = n4_rsrc(X, false), rs_none = n4_rsrc(A, true);
+  const int lda_b = (int)(g.lda * 2), ldx_b = (int)(g.ldb * 2);
+  const int r_in = wave * 8 + (lane >> 3);
+  const int voa = r_in * lda_b + (((lane & 7) ^ kswz(r_in)) << 4);
+  // X panel rows k: chunk c of row k at c ^ xsw(k). A transposing read takes 4 rows of 32 bytes for
+  // 16 lanes, and the next 16 lanes 4 rows eight further: xsw puts the eight in different
+  // 32-byte groups of the 64 banks.
+  auto xsw = [](int k) {
+    return TM == 128 ? ((k & 3) << 2) | (((k >> 3) & 1) << 1) : (((k >> 1) & 1) | (((k >> 3) & 1) << 1)) << 1;
+  };
+  const int x_in = wave * (1024 / XR) + lane / XCH;
+  const int vox = x_in * ldx_b + (((lane % XCH) ^ xsw(x_in)) << 4);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  const int KT = (int)(g.K / V2_BK);
+  auto issue = [&](int kt, int st) {
+    const bool on = kt < KT;
+    const int kk = on ? kt : 0;
+    const uint32_t m0 = lds0 + st * C::STAGEB + wave * 1024;
+    const u32x4 pa = on ? rsa : rs_none, px = on ? rsx : rs_none;
+#pragma unroll
+    for (int q = 0; q < C::LOADS; ++q) {
+      tile_dma(voa, pa, kk * V2_ROWB + q * 32 * lda_b, m0 + q * 4096);
+      tile_dma(vox, px, (kk * V2_BK + q * (4096 / XR)) * ldx_b, m0 + C::PANELB + q * 4096);
+    }
+  };
+  float alpha = g.alpha, beta = g.beta;
+  if (g.scale_mode == 1) {
+    const float s = g.scale[bidx];
+    alpha *= s;
+    beta *= s;
+  }
+  const float ratio = beta != 0.0f ? beta / alpha : 0.0f;
+  // 32-k step whose rows of X are this wave's output rows (F / 2 of them from here on)
+  const int sdiag = ratio != 0.0f ? (row0 + wm * WM) / 32 : -2 * F;
+
+  f32x4 acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int fr = lane & 15, fg = lane >> 4;
+  auto mma = [&](const bf16x8_mfma& b, const bf16x8_mfma& x, f32x4& c) {
+    c = SW ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, x, c, 0, 0, 0)
+           : __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b, c, 0, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < C::NS - 1; ++t) issue(t, t);
+  int st = 0;
+  for (int kt = 0; kt < KT; ++kt) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * C::LOADS * (C::NS - 2)) : "memory");
+    lds_barrier();
+    issue(kt + C::NS - 1, st == 0 ? C::NS - 1 : st - 1);
+    const uint8_t* sp = smem + st * C::STAGEB;
+    uint8_t* xp = smem + st * C::STAGEB + C::PANELB;
+    bf16x8_mfma b[2][F], x[2][F];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int off = (wm * WM + fr) * V2_ROWB + (((ks * 4 + fg) ^ kswz(fr)) << 4);
+      const int k = 32 * ks + 8 * fg + (fr >> 2);
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        b[ks][f] = __builtin_bit_cast(bf16x8_mfma, *(const uint4*)(sp + f * 16 * V2_ROWB + off));
+        const int c = (wn * WM + f * 16) / 8 + ((fr & 3) >> 1);
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) i16x4*)(xp + k * XR + ((c ^ xsw(k)) << 4) + (fr & 1) * 8));
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) i16x4*)(xp + (k + 4) * XR + ((c ^ xsw(k + 4)) << 4) + (fr & 1) * 8));
+        x[ks][f] = __builtin_bit_cast(bf16x8_mfma, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) mma(b[ks][i], x[ks][j], acc[i][j]);
+      const int sd = 2 * kt + ks - sdiag;
+      if (sd >= 0 && sd < F / 2) {
+        bf16x8_mfma db[2][2], d3[2][2];
+        n16_beta_frags(ratio, lane, db);
+        n16_beta_third(ratio, lane, d3);
+#pragma unroll
+        for (int f = 0; f < F / 2; ++f)
+          if (sd == f) {
+#pragma unroll
+            for (int part = 0; part < 2; ++part)
+#pragma unroll
+              for (int par = 0; par < 2; ++par)
+#pragma unroll
+                for (int j = 0; j < F; ++j) mma(db[par][part], x[ks][j], acc[2 * f + par][j]);
+            if (g.K < BETA3_K) {
+#pragma unroll
+              for (int par = 0; par < 2; ++par)
+#pragma unroll
+                for (int j = 0; j < F; ++j) mma(d3[par][0], x[ks][j], acc[2 * f + par][j]);
+            }
+          }
+      }
+    }
+    st = st + 1 == C::NS ? 0 : st + 1;
+  }
+  wait_vmcnt0();
+  lds_barrier();
+
+  // epilogue: rows of the staged tile are X' rows (SW: X' columns), 4 consecutive elements of
+  // one row per lane
+  bf16_t* T = (bf16_t*)smem;
+  const int mv = (int)g.Mv, nv = (int)g.Nv;
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const f2x v01 = {alpha * acc[i][j][0], alpha * acc[i][j][1]};
+      const f2x v23 = {alpha * acc[i][j][2], alpha * acc[i][j][3]};
+      uint32_t w0 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v01, bf2x));
+      uint32_t w1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v23, bf2x));
+      const int ri = wm * WM + i * 16, cj = wn * WM + j * 16;
+      if constexpr (PDT < 0) {
+        // zeros outside the valid extent, so that the padding stays zero
+        const int r = row0 + ri + fr, c = col0 + cj + 4 * fg;
+        w0 &= (r < mv && c < nv ? 0x0000ffffu : 0u) | (r < mv && c + 1 < nv ? 0xffff0000u : 0u);
+        w1 &= (r < mv && c + 2 < nv ? 0x0000ffffu : 0u) | (r < mv && c + 3 < nv ? 0xffff0000u : 0u);
+      }
+      bf16_t* pos = SW ? T + (cj + fr) * C::PITCH + ri + 4 * fg : T + (ri + fr) * C::PITCH + cj + 4 * fg;
+      *(uint2*)pos = make_uint2(w0, w1);
+    }
+  lds_barrier();
+  constexpr int CH = TM / 8, ROWS = 256 / CH;
+  if constexpr (PDT < 0) {
+    bf16_t* out = (bf16_t*)g.out + (int64_t)bidx * g.so;
+#pragma unroll
+    for (int it = 0; it < TM / ROWS; ++it) {
+      const int il = it * ROWS + tid / CH, c = tid % CH * 8;
+      *(uint4*)(out + (int64_t)(row0 + il) * g.ldo + col0 + c) = *(const uint4*)(T + il * C::PITCH + c);
+    }
+  } else {
+    // matrix bidx of the group is matrix bidx % nb of its tensor t0 + bidx / nb
+    const int t = g.t0 + bidx / g.nb;
+    const int64_t mb = bidx % g.nb;
+    const float adj = ap.adj[t];
+    const int prows = SW ? nv : mv, pcols = SW ? mv : nv;
+    const int pr0 = SW ? col0 : row0, pc0 = SW ? row0 : col0;
+    void* prm = ap.params[t];
+    const int64_t base = mb * (int64_t)prows * pcols;
+    Raw8<PDT> pv[TM / ROWS];
+#pragma unroll
+    for (int it = 0; it < TM / ROWS; ++it) {
+      const int r = pr0 + it * ROWS + tid / CH, c = pc0 + tid % CH * 8;
+      if (r < prows && c < pcols) pv[it].load(prm, base + (int64_t)r * pcols + c);
+    }
+#pragma unroll
+    for (int it = 0; it < TM / ROWS; ++it) {
+      const int il = it * ROWS + tid / CH, cl = tid % CH * 8;
+      const int r = pr0 + il, c = pc0 + cl;
+      if (r >= prows || c >= pcols) continue;
+      float p[8], u[8];
+      pv[it].unpack(p);
+      Vec8<MUON_DT_BF16>::load(T + il * C::PITCH + cl, 0, u);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = apply_elem<PDT, MUON_DT_BF16>(p[e], u[e], ap.wd, ap.cautious, adj);
+      pv[it].pack(p);
+      pv[it].store(prm, base + (int64_t)r * pcols + c);
+    }
+  }
+}
+
 // Wave grid of the register-staged bf16 kernel (gemm_bf16_kernel), which serves the
 // masked gram_ path and SYRKs whose beta term has no alpha to fold into: 4 x 2
 // wavefronts, each 64 x 128, two waves per SIMD.
@@ -2911,17 +2932,18 @@ int reserve_lds() {
     if (hipFuncSetAttribute((const void*)gemm_bf16_s16_kernel,
                             hipFuncAttributeMaxDynamicSharedMemorySize, V2_SMEM) != hipSuccess)
       status = -1;
-    if (hipFuncSetAttribute((const void*)gemm_bf16_s16h_kernel,
+    if (hipFuncSetAttribute((const void*)gemm_bf16_s16h_kernel<GemmArgs>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, H_SMEM) != hipSuccess)
       status = -1;
-    if (hipFuncSetAttribute((const void*)gemm_bf16_nn4_kernel,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, N4_SMEM) != hipSuccess)
-      status = -1;
-    const void* n16[7] = {
-        (const void*)gemm_bf16_nn16_kernel<0>,    (const void*)gemm_bf16_nn16_kernel<1, 0>,
-        (const void*)gemm_bf16_nn16_kernel<1, 1>, (const void*)gemm_bf16_nn16_kernel<1, 2>,
-        (const void*)gemm_bf16_nn16_kernel<2, 0>, (const void*)gemm_bf16_nn16_kernel<2, 1>,
-        (const void*)gemm_bf16_nn16_kernel<2, 2>};
+    const void* n16[14] = {
+#define N16_ALL(B3)                                                                           \
+  (const void*)gemm_bf16_nn16_kernel<0, 0, B3>, (const void*)gemm_bf16_nn16_kernel<1, 0, B3>, \
+      (const void*)gemm_bf16_nn16_kernel<1, 1, B3>, (const void*)gemm_bf16_nn16_kernel<1, 2, B3>, \
+      (const void*)gemm_bf16_nn16_kernel<2, 0, B3>, (const void*)gemm_bf16_nn16_kernel<2, 1, B3>, \
+      (const void*)gemm_bf16_nn16_kernel<2, 2, B3>
+        N16_ALL(false), N16_ALL(true)
+#undef N16_ALL
+    };
     for (const void* k : n16)
       if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, N4_SMEM) !=
           hipSuccess)
@@ -2956,26 +2978,65 @@ int device_cus() {
 // CU needs, with the tiles spread evenly over them (a launch of a few hundred tiles leaves
 // the CUs it does not need to kernels on other streams instead of idling them in its last
 // round). Unchanged when the tile count is a multiple of the CU count.
-// Whether a full-tile SYRK launch of `blocks` 256-row tiles (tiles_m per side, `batch`
-// matrices) takes gemm_bf16_s16h_kernel's 128-row tiles instead: when it has at most two
-// rounds of 256-row tiles (one workgroup per CU) and the 128-row tiles, two workgroups per
-// CU with a quarter of the work each, need fewer rounds, counting a 128-row round as half
-// a 256-row one at 85% of its efficiency (72 workgroups of 12 matrices of 768 rows: one
-// round against one half-round; 320 of 32 matrices of 1024 rows: two rounds against three
-// half-rounds; 200 would be one round against two half-rounds, and stays).
-static bool use_h128(int tiles_m, int64_t batch, int64_t blocks) {
-  const int64_t cus = device_cus();
-  const int64_t th = 2 * (int64_t)tiles_m;
-  const int64_t bh = th * (th + 1) / 2 * batch;
-  const int64_t rounds = (blocks + cus - 1) / cus, rounds_h = (bh + 2 * cus - 1) / (2 * cus);
-  return blocks <= 2 * cus && 20 * rounds_h <= 34 * rounds;
-}
-
 static int persistent_wgs(int64_t blocks) {
   const int64_t cus = device_cus();
   if (blocks <= cus) return (int)blocks;
   const int64_t rounds = (blocks + cus - 1) / cus;
   return (int)((blocks + rounds - 1) / rounds);
+}
+
+// Tile size of a SYRK (256, 128 or 64 rows) and of a B X launch, by the time each would take: the
+// kernels give the same bits. Microseconds of one launch, fitted to launches of 1 to 1000 matrices of
+// 128 to 4096 rows (K from 128 to 14336; within about 20%, the choice within 10% of the best
+// of the three measured ones). A launch on 256-row tiles is rounds of one workgroup per CU, each
+// its prologue and epilogue plus a time per k; on 128-row tiles two workgroups share a CU, and
+// once the CUs are full the time goes by the operand bytes (half the reuse of 256-row tiles);
+// 64-row tiles have the shortest chain and again half the reuse. blocks: tiles of the size at
+// hand; the padding beyond round_up(m, 128) rows is only computed by 256-row tiles.
+// Measured (us, 256 / 128 / 64): X X^T of 1 x 256 x 512 12.4 / 13.3 / 7.7 and of 1 x 1024 x 4096 52.9 / 45.4
+// / 20.7, of 64 x 512 x 2048 65 / 80 / 79; A A of 1408 rows 45.5 / 22.0 / 11.5; B X of 4 x 512 x 512
+// 22.0 / 12.1 / 9.3, of 2 x 1024 x 4096 30.2 / 24.3 / 39.4, of 12 x 768 x 3072 47.5 / 56 / 99.
+static double per_cu(int64_t blocks) {
+  const double w = (double)blocks / device_cus();
+  return w <= 1.0 ? 1.0 : w + 0.5;
+}
+static int64_t rounds_of(int64_t blocks) { return (blocks + device_cus() - 1) / device_cus(); }
+
+static int syrk_tile(int64_t batch, int64_t m, int64_t M, int64_t K, int64_t blocks256) {
+  const int64_t t1 = round_up(m, 128) / 128, t2 = 2 * t1;
+  const int64_t n128 = t1 * (t1 + 1) / 2 * batch, n64 = t2 * (t2 + 1) / 2 * batch;
+  const double k = (double)K;
+  const double c256 = rounds_of(blocks256) * (17.0 + 0.0212 * k);
+  const double c128 = n128 <= device_cus() ? 9.0 + 0.0089 * k : 9.0 + per_cu(n128) * (1.7 + 0.0092 * k);
+  const double c64 = 5.0 + rounds_of(n64) * (0.6 + 0.0037 * k);
+  if (c64 < c128 && c64 < c256) return 64;
+  return c128 < c256 ? 128 : 256;
+}
+
+static int bx_tile(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m) {
+  const int64_t me = round_up(m, 128);
+  const int64_t n256 = (M / 256) * (N / 256) * batch, n128 = (me / 128) * (N / 128) * batch;
+  const int64_t n64 = 4 * n128;
+  const double k = (double)K;
+  const double c256 = rounds_of(n256) * (9.0 + 0.0215 * k);
+  const double c128 = n128 <= device_cus()       ? 5.5 + 0.0122 * k
+                      : n128 <= 2 * device_cus() ? 6.0 + 0.0185 * k
+                                                 : 6.0 + per_cu(n128) * (0.8 + 0.0098 * k);
+  const double c64 = n64 <= device_cus() ? 4.5 + 0.0078 * k : 4.5 + per_cu(n64) * (0.5 + 0.0038 * k);
+  if (c64 < c128 && c64 < c256) return 64;
+  // (128-row tiles read twice the operand bytes: near the line the step on a dozen matrices each
+  // of four shapes, whose launches run beside each other, was 0.5% slower with them)
+  return c128 < 0.6 * c256 ? 128 : 256;
+}
+
+// `g` on TM-row tiles covering round_up(m, 128) rows (of a SYRK, columns too).
+static GemmArgs on_tiles(const GemmArgs& g, int mode, int TM, int64_t m, int64_t N, int64_t batch) {
+  GemmArgs t = g;
+  t.tiles_m = (int)(round_up(m, 128) / TM);
+  t.tiles_n = (int)(mode == MODE_SYRK ? t.tiles_m : N / TM);
+  t.tiles_per_batch = mode == MODE_SYRK ? t.tiles_m * (t.tiles_m + 1) / 2 : t.tiles_m * t.tiles_n;
+  t.tiles_total = (int)(t.tiles_per_batch * batch);
+  return t;
 }
 
 }  // namespace
@@ -3071,36 +3132,48 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
         muon_set_error("gemm: bf16 NN products take K a multiple of 128 and no transposed output");
         return MUON_ERR_ARG;
       }
-      // persistent: at most one workgroup per CU walks the tile list
-      const int wgs = persistent_wgs(blocks);
-      if (K >= 768) {
-        MuonApply none;
-        none.nb = 1;
-        hipLaunchKernelGGL(gemm_bf16_nn16_kernel<0>, dim3((unsigned)wgs), dim3(256), N4_SMEM,
-                           stream, g, none);
+      MuonApply none;
+      none.nb = 1;
+      const int TM = bx_tile(batch, M, N, K, Mv);
+      if (TM == 256) {
+        // persistent: at most one workgroup per CU walks the tile list
+        const dim3 pg((unsigned)persistent_wgs(blocks));
+        if (K < BETA3_K)
+          hipLaunchKernelGGL((gemm_bf16_nn16_kernel<0, 0, true>), pg, dim3(256), N4_SMEM, stream, g, none);
+        else
+          hipLaunchKernelGGL(gemm_bf16_nn16_kernel<0>, pg, dim3(256), N4_SMEM, stream, g, none);
+      } else {
+        const GemmArgs gt = on_tiles(g, mode, TM, Mv, N, batch);
+        const dim3 tg((unsigned)gt.tiles_total);
+        if (TM == 128)
+          hipLaunchKernelGGL((tile_bx_kernel<128, -1, false, GemmArgs>), tg, dim3(256),
+                             TileK<128>::SMEM, stream, gt, none);
+        else
+          hipLaunchKernelGGL((tile_bx_kernel<64, -1, false, GemmArgs>), tg, dim3(256),
+                             TileK<64>::SMEM, stream, gt, none);
       }
-      else
-        hipLaunchKernelGGL(gemm_bf16_nn4_kernel, dim3((unsigned)wgs), dim3(256), N4_SMEM, stream, g);
     } else if (!masked && (alpha != 0.0f || beta == 0.0f)) {
       // the last 128 rows padding only: the last tile column's real unit in packed tiles,
       // in the same launch as the full tiles
       const int T = g.tiles_m;
-      if (T >= 2 && Mv <= M - 128 && Nv == Mv) {
-        GemmArgs gp = g;
+      GemmArgs gp = g;
+      const bool packed = T >= 2 && Mv <= M - 128 && Nv == Mv;
+      if (packed) {
         gp.tiles_per_batch = (T - 1) * T / 2 + (2 * T - 1 + 3) / 4;
         gp.tiles_total = gp.tiles_per_batch * (int)batch;
+      }
+      const int TM = syrk_tile(batch, Mv, M, K, gp.tiles_total);
+      if (TM != 256) {
+        const GemmArgs gt = on_tiles(g, mode, TM, Mv, N, batch);
+        const dim3 tg((unsigned)gt.tiles_total);
+        if (TM == 128)
+          hipLaunchKernelGGL((gemm_bf16_s16h_kernel<GemmArgs>), tg, dim3(256), H_SMEM, stream, gt);
+        else
+          hipLaunchKernelGGL((tile_syrk_kernel<64, GemmArgs>), tg, dim3(256), TileK<64>::SMEM, stream,
+                             gt);
+      } else if (packed) {
         hipLaunchKernelGGL((gemm_bf16_v2_kernel<MODE_SYRK, true>),
-                           dim3((unsigned)(gp.tiles_per_batch * batch)), dim3(512),
-                           v2_smem(true), stream, gp);
-      } else if (use_h128(g.tiles_m, batch, blocks)) {
-        // at most two rounds of 256-row tiles, the CUs idle for much of them (72 workgroups,
-        // or 320 in two rounds of 256 and 64): 128-row tiles, two workgroups per CU
-        GemmArgs gh = g;
-        gh.tiles_m = 2 * g.tiles_m;
-        gh.tiles_per_batch = gh.tiles_m * (gh.tiles_m + 1) / 2;
-        gh.tiles_total = gh.tiles_per_batch * (int)batch;
-        hipLaunchKernelGGL(gemm_bf16_s16h_kernel, dim3((unsigned)gh.tiles_total), dim3(256),
-                           H_SMEM, stream, gh);
+                           dim3((unsigned)gp.tiles_total), dim3(512), v2_smem(true), stream, gp);
       } else {
         // full tiles only: the 16 x 16 x 32 MFMA kernel
         hipLaunchKernelGGL(gemm_bf16_s16_kernel, grid, dim3(512), V2_SMEM, stream, g);
@@ -3138,17 +3211,34 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
   return MUON_OK;
 }
 
-// The last iteration's X' = a X + B X with the post-pass applied in its epilogue (bf16
-// parameters, K >= 768: the 16 x 16 x 32 GEMM); extents and operands as muon_launch_gemm's
-// GEMM mode, X' is not stored. tall: the parameter is the transpose of the iterate (its
-// rows are the columns of X'). Parameter rows of whole 8-element chunks (pcols % 8 == 0) and
-// 16-byte aligned tensors are the caller's to check.
+// Whether the apply of `batch` matrices' last B X is fused for parameters of type pdt: bf16 ones
+// always (the 256-row kernel has the epilogue), others where the launch on 128- or 64-row
+// tiles costs less than the 256-row one and a post-pass (which reads U and the parameters
+// and writes the parameters, about 5 TB/s). Six fp32
+// matrices of 768 x 3072: 26 us and 29 us of post-pass against 45 us.
+int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int64_t n, int pdt) {
+  if (pdt == MUON_DT_BF16) return 1;
+  const int pes = pdt == MUON_DT_F32 ? 4 : 2;
+  const double post = 6.0 + (double)batch * m * n * (2 + 2 * pes) / 5.0e6;
+  const int64_t n256 = (M / 256) * (N / 256) * batch, n128 = round_up(m, 128) / 128 * (N / 128) * batch;
+  const double c256 = rounds_of(n256) * (9.0 + 0.0215 * (double)K);
+  const double c128 = 6.0 + per_cu(n128) * (0.8 + 0.0098 * (double)K);
+  return bx_tile(batch, M, N, K, m) != 256 || c128 < c256 + 0.5 * post;
+}
+
+// The last iteration's X' = a X + B X with the post-pass applied in its epilogue: extents and
+// operands as muon_launch_gemm's GEMM mode, X' is not stored. tall: the parameter is the
+// transpose of the iterate (its rows are the columns of X'). Parameter rows of whole 8-element
+// chunks (pcols % 8 == 0), 16-byte aligned tensors and muon_apply_fuses are the caller's to
+// check.
 int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const void* a,
                            int64_t lda, int64_t sa, const void* b, int64_t ldb, int64_t sb,
                            int64_t Mv, int64_t Nv, float alpha, float beta, const float* scale,
-                           int scale_mode, const MuonApply& ap, int tall, hipStream_t stream) {
-  if (K < 768 || K % 128 || M % BF_BM || N % BF_BM || alpha == 0.0f || ap.nb <= 0 ||
-      (batch + ap.nb - 1) / ap.nb > MUON_APPLY_MAX || ap.pcols % 8) {
+                           int scale_mode, const MuonApply& ap, int pdt, int tall,
+                           hipStream_t stream) {
+  if (K % 128 || M % BF_BM || N % BF_BM || alpha == 0.0f || ap.nb <= 0 ||
+      (batch + ap.nb - 1) / ap.nb > MUON_APPLY_MAX || ap.pcols % 8 ||
+      ap.prows != (tall ? Nv : Mv) || ap.pcols != (tall ? Mv : Nv)) {
     muon_set_error("gemm_apply: unsupported launch (K %lld, batch %lld)", (long long)K,
                    (long long)batch);
     return MUON_ERR_ARG;
@@ -3181,7 +3271,7 @@ int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const
   g.tiles_per_batch = g.tiles_m * g.tiles_n;
   const int64_t blocks = (int64_t)g.tiles_per_batch * batch;
   if (blocks == 0) return MUON_OK;
-  if (blocks > 0x7fffffffLL) {
+  if (blocks > 0x7fffffffLL / 16) {
     muon_set_error("gemm_apply: grid too large (%lld tiles)", (long long)blocks);
     return MUON_ERR_SHAPE;
   }
@@ -3190,16 +3280,44 @@ int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const
     muon_set_error("gemm_apply: cannot reserve LDS");
     return MUON_ERR_LAUNCH;
   }
-  const int wgs = persistent_wgs(blocks);
-  const int mode = ap.wd == 0.0f ? 0 : (ap.cautious ? 1 : 2);
-#define LAUNCH_APPLY(A, M) \
-  hipLaunchKernelGGL((gemm_bf16_nn16_kernel<A, M>), dim3((unsigned)wgs), dim3(256), N4_SMEM, stream, g, ap)
-  if (tall) {
-    if (mode == 0) LAUNCH_APPLY(2, 0); else if (mode == 1) LAUNCH_APPLY(2, 1); else LAUNCH_APPLY(2, 2);
-  } else {
-    if (mode == 0) LAUNCH_APPLY(1, 0); else if (mode == 1) LAUNCH_APPLY(1, 1); else LAUNCH_APPLY(1, 2);
-  }
+  int TM = bx_tile(batch, M, N, K, Mv);
+  if (TM == 256 && pdt != MUON_DT_BF16) TM = 128;
+  if (TM == 256) {
+    const int wgs = persistent_wgs(blocks);
+    const int mode = ap.wd == 0.0f ? 0 : (ap.cautious ? 1 : 2);
+#define LAUNCH_APPLY(A, M)                                                                         \
+  do {                                                                                           \
+    if (K < BETA3_K)                                                                             \
+      hipLaunchKernelGGL((gemm_bf16_nn16_kernel<A, M, true>), dim3((unsigned)wgs), dim3(256), N4_SMEM, stream, g, ap); \
+    else                                                                                         \
+      hipLaunchKernelGGL((gemm_bf16_nn16_kernel<A, M>), dim3((unsigned)wgs), dim3(256), N4_SMEM, stream, g, ap); \
+  } while (0)
+    if (tall) {
+      if (mode == 0) LAUNCH_APPLY(2, 0); else if (mode == 1) LAUNCH_APPLY(2, 1); else LAUNCH_APPLY(2, 2);
+    } else {
+      if (mode == 0) LAUNCH_APPLY(1, 0); else if (mode == 1) LAUNCH_APPLY(1, 1); else LAUNCH_APPLY(1, 2);
+    }
 #undef LAUNCH_APPLY
+  } else {
+    GemmArgs gt = on_tiles(g, MODE_GEMM, TM, Mv, N, batch);
+    gt.t0 = 0;
+    gt.nb = (int)ap.nb;
+#define LAUNCH_TILE(TM_, P_, SW_)                                                               \
+  hipLaunchKernelGGL((tile_bx_kernel<TM_, P_, SW_, GemmArgs>), dim3((unsigned)gt.tiles_total), \
+                     dim3(256), TileK<TM_>::SMEM, stream, gt, ap)
+#define LAUNCH_TILE_P(TM_, P_) \
+  do { if (tall) LAUNCH_TILE(TM_, P_, true); else LAUNCH_TILE(TM_, P_, false); } while (0)
+#define LAUNCH_TILE_T(TM_)                                              \
+  do {                                                                  \
+    if (pdt == MUON_DT_BF16) LAUNCH_TILE_P(TM_, MUON_DT_BF16);          \
+    else if (pdt == MUON_DT_F16) LAUNCH_TILE_P(TM_, MUON_DT_F16);       \
+    else LAUNCH_TILE_P(TM_, MUON_DT_F32);                               \
+  } while (0)
+    if (TM == 128) LAUNCH_TILE_T(128); else LAUNCH_TILE_T(64);
+#undef LAUNCH_TILE_T
+#undef LAUNCH_TILE_P
+#undef LAUNCH_TILE
+  }
   MUON_CHECK_LAUNCH("gemm_apply");
   return MUON_OK;
 }
