@@ -16,13 +16,14 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
                      int64_t ldb, int64_t sb, const void* cin, int64_t ldc, int64_t sc,
                      void* out, int64_t ldo, int64_t so, void* out_t, int64_t ldt, int64_t st,
                      int64_t Mv, int64_t Nv, float alpha, float beta, const float* scale,
-                     int scale_mode, hipStream_t stream);
+                     int scale_mode, int beside, hipStream_t stream);
 int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const void* a,
                            int64_t lda, int64_t sa, const void* b, int64_t ldb, int64_t sb,
                            int64_t Mv, int64_t Nv, float alpha, float beta, const float* scale,
-                           int scale_mode, const MuonApply& ap, int pdt, int tall,
+                           int scale_mode, const MuonApply& ap, int pdt, int tall, int beside,
                            hipStream_t stream);
-int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int64_t n, int pdt);
+int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int64_t n, int pdt,
+                     int beside);
 int muon_launch_prepass(int ntensors, void* const* grads, void* const* bufs, int gdt, int bdt,
                         int64_t nb, int64_t rows, int64_t cols, int64_t s_pitch,
                         int64_t s_mstride, float momentum, int nesterov, int maximize,
@@ -276,16 +277,16 @@ int muon_gram(const void* x, void* y, int dtype, int64_t batch, int64_t M, int64
     // operands in place
     return muon_launch_gemm(dtype, MODE_SYRK, false, batch, M, M, K, x, K, M * K, x, K, M * K,
                             nullptr, 0, 0, y, M, M * M, nullptr, 0, 0, M, M, 1.0f, 0.0f,
-                            nullptr, 0, (hipStream_t)stream);
+                            nullptr, 0, 0, (hipStream_t)stream);
   if (dtype == MUON_DT_F32 && M % 128 == 0 && K % 64 == 0 && !((uintptr_t)x & 15) &&
       !((uintptr_t)y & 15))
     // the same for fp32: whole 128-row tiles and 64-wide steps of K
     return muon_launch_gemm(dtype, MODE_SYRK, false, batch, M, M, K, x, K, M * K, x, K, M * K,
                             nullptr, 0, 0, y, M, M * M, nullptr, 0, 0, M, M, 1.0f, 0.0f,
-                            nullptr, 0, (hipStream_t)stream);
+                            nullptr, 0, 0, (hipStream_t)stream);
   return muon_launch_gemm(dtype, MODE_SYRK, true, batch, M, M, K, x, K,
                           M * K, x, K, M * K, nullptr, 0, 0, y, M, M * M, nullptr, 0, 0, M, M,
-                          1.0f, 0.0f, nullptr, 0, (hipStream_t)stream);
+                          1.0f, 0.0f, nullptr, 0, 0, (hipStream_t)stream);
 }
 
 int64_t muon_orth_workspace_bytes(int dtype, int64_t batch, int64_t rows, int64_t cols) {
@@ -402,7 +403,7 @@ static int apply_chunks(const ApplyReq& r, F&& launch) {
 
 static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch, int64_t rows,
                          int64_t cols, const double* coeffs, int steps, float prescale,
-                         float eps, const ApplyReq* ap, void* stream) {
+                         float eps, const ApplyReq* ap, int beside, void* stream) {
   if (!iter_dtype_ok(ws_dtype)) {
     muon_set_error("orth_run: unsupported dtype %d", ws_dtype);
     return MUON_ERR_DTYPE;
@@ -504,7 +505,7 @@ static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch
     Timed t(MUON_K_SYRK_XX, bm * md * (md + 1) * nd, s);
     rc = muon_launch_gemm(ws_dtype, MODE_SYRK, false, batch, mp, mp, np, Xc, xp, mp * xp, Xc, xp,
                           mp * xp, nullptr, 0, 0, A, mp, mp * mp, nullptr, 0, 0, L.m, L.m, 1.0f,
-                          0.0f, scale, first ? 2 : 0, s);
+                          0.0f, scale, first ? 2 : 0, beside, s);
     }
     if (rc != MUON_OK) return rc;
     // B = b*A + c*(A A)
@@ -512,7 +513,7 @@ static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch
     Timed t(MUON_K_SYRK_AA, bm * md * (md + 1) * md, s);
     rc = muon_launch_gemm(ws_dtype, MODE_SYRK, false, batch, mp, mp, kq, A, mp, mp * mp, A, mp,
                           mp * mp, A, mp, mp * mp, B, mp, mp * mp, nullptr, 0, 0, L.m, L.m, c, b,
-                          nullptr, 0, s);
+                          nullptr, 0, beside, s);
     }
     if (rc != MUON_OK) return rc;
     // X' = a*X + B X into the other buffer (every tile reads whole columns of X); the
@@ -522,13 +523,13 @@ static int orth_run_impl(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch
       rc = apply_chunks(*ap, [&](int64_t m0, int64_t cnt, const MuonApply& tab) {
         return muon_launch_gemm_apply(cnt, mp, np, kq, B + m0 * mp * mp * 2, mp, mp * mp,
                                       Xc + m0 * mp * xp * 2, xp, mp * xp, L.m, L.n, 1.0f, a,
-                                      scale + m0, first ? 1 : 0, tab, ap->p_dtype, L.tall, s);
+                                      scale + m0, first ? 1 : 0, tab, ap->p_dtype, L.tall, beside, s);
       });
     } else {
     Timed t(MUON_K_GEMM_BX, bm * 2.0 * md * md * nd, s);
     rc = muon_launch_gemm(ws_dtype, MODE_GEMM, false, batch, mp, np, kq, B, mp, mp * mp, Xc, xp,
                           mp * xp, Xc, xp, mp * xp, Xn, xp, mp * xp, nullptr, 0, 0, L.m, L.n,
-                          1.0f, a, scale, first ? 1 : 0, s);
+                          1.0f, a, scale, first ? 1 : 0, beside, s);
     }
     if (rc != MUON_OK) return rc;
   }
@@ -539,13 +540,30 @@ int muon_orth_run(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch, int64
                   int64_t cols, const double* coeffs, int steps, float prescale, float eps,
                   void* stream) {
   return orth_run_impl(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps, prescale, eps,
-                       nullptr, stream);
+                       nullptr, 0, stream);
 }
 
 int muon_orth_run_apply(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch, int64_t rows,
                         int64_t cols, const double* coeffs, int steps, float prescale,
                         float eps, int ntensors, void* const* params, int p_dtype, int64_t nb,
                         const float* adjusted_lrs, float wd, int cautious, void* stream) {
+  return muon_orth_run_apply_beside(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps,
+                                    prescale, eps, ntensors, params, p_dtype, nb, adjusted_lrs,
+                                    wd, cautious, 0, stream);
+}
+
+int muon_orth_run_beside(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch, int64_t rows,
+                         int64_t cols, const double* coeffs, int steps, float prescale, float eps,
+                         int beside, void* stream) {
+  return orth_run_impl(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps, prescale, eps,
+                       nullptr, beside, stream);
+}
+
+int muon_orth_run_apply_beside(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,
+                               int64_t rows, int64_t cols, const double* coeffs, int steps,
+                               float prescale, float eps, int ntensors, void* const* params,
+                               int p_dtype, int64_t nb, const float* adjusted_lrs, float wd,
+                               int cautious, int beside, void* stream) {
   bool fuse = ws_dtype == MUON_DT_BF16 && io_dtype_ok(p_dtype) && steps > 0 && rows > 0 &&
               cols > 0 && nb > 0 && ntensors > 0 && (int64_t)ntensors * nb == batch &&
               batch <= ws_batch && params && adjusted_lrs && cols % 8 == 0;
@@ -555,19 +573,19 @@ int muon_orth_run_apply(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,
     // the tiled path where it pays; iterates of at most 64 rows when the parameter is bf16 and
     // wide (its rows are the iterate's)
     fuse = L.short_m ? !L.tall && p_dtype == MUON_DT_BF16
-                     : muon_apply_fuses(batch, L.m_pad, L.n_pad, kq, L.m, L.n, p_dtype) != 0;
+                     : muon_apply_fuses(batch, L.m_pad, L.n_pad, kq, L.m, L.n, p_dtype, beside) != 0;
     for (int t = 0; fuse && t < ntensors; ++t) fuse = params[t] && !((uintptr_t)params[t] & 15);
   }
   if (!fuse) {
-    int rc = muon_orth_run(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps, prescale,
-                           eps, stream);
+    int rc = orth_run_impl(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps, prescale,
+                           eps, nullptr, beside, stream);
     if (rc != MUON_OK) return rc;
     return muon_postpass(ntensors, params, p_dtype, nullptr, 0, ws, ws_dtype, ws_batch, steps,
                          nb, rows, cols, adjusted_lrs, nullptr, wd, cautious, stream);
   }
   const ApplyReq ap = {params, adjusted_lrs, p_dtype, ntensors, nb, rows, cols, wd, cautious};
   return orth_run_impl(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps, prescale, eps,
-                       &ap, stream);
+                       &ap, beside, stream);
 }
 
 int muon_orth_extract(const void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,

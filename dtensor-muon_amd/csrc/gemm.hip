@@ -2993,6 +2993,11 @@ static int persistent_wgs(int64_t blocks) {
 // once the CUs are full the time goes by the operand bytes (half the reuse of 256-row tiles);
 // 64-row tiles have the shortest chain and again half the reuse. blocks: tiles of the size at
 // hand; the padding beyond round_up(m, 128) rows is only computed by 256-row tiles.
+// beside: the launch shares the device with other streams' (a step's small buckets). Near the lines
+// the larger tiles then win, since what the launch takes from its neighbours counts, not its own
+// time: 24 fp32 matrices of four shapes with 8-bit momentum, on four streams, took 0.95 ms a
+// step with the factors below and 1.11 without; a dozen matrices each of four shapes 0.5% more
+// with 0.8 in place of 0.6.
 // Measured (us, 256 / 128 / 64): X X^T of 1 x 256 x 512 12.4 / 13.3 / 7.7 and of 1 x 1024 x 4096 52.9 / 45.4
 // / 20.7, of 64 x 512 x 2048 65 / 80 / 79; A A of 1408 rows 45.5 / 22.0 / 11.5; B X of 4 x 512 x 512
 // 22.0 / 12.1 / 9.3, of 2 x 1024 x 4096 30.2 / 24.3 / 39.4, of 12 x 768 x 3072 47.5 / 56 / 99.
@@ -3002,18 +3007,18 @@ static double per_cu(int64_t blocks) {
 }
 static int64_t rounds_of(int64_t blocks) { return (blocks + device_cus() - 1) / device_cus(); }
 
-static int syrk_tile(int64_t batch, int64_t m, int64_t M, int64_t K, int64_t blocks256) {
+static int syrk_tile(int64_t batch, int64_t m, int64_t K, int64_t blocks256, int beside) {
   const int64_t t1 = round_up(m, 128) / 128, t2 = 2 * t1;
   const int64_t n128 = t1 * (t1 + 1) / 2 * batch, n64 = t2 * (t2 + 1) / 2 * batch;
   const double k = (double)K;
   const double c256 = rounds_of(blocks256) * (17.0 + 0.0212 * k);
   const double c128 = n128 <= device_cus() ? 9.0 + 0.0089 * k : 9.0 + per_cu(n128) * (1.7 + 0.0092 * k);
   const double c64 = 5.0 + rounds_of(n64) * (0.6 + 0.0037 * k);
-  if (c64 < c128 && c64 < c256) return 64;
+  if (c64 < (beside ? 0.75 : 1.0) * c128 && c64 < c256) return 64;
   return c128 < c256 ? 128 : 256;
 }
 
-static int bx_tile(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m) {
+static int bx_tile(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int beside) {
   const int64_t me = round_up(m, 128);
   const int64_t n256 = (M / 256) * (N / 256) * batch, n128 = (me / 128) * (N / 128) * batch;
   const int64_t n64 = 4 * n128;
@@ -3024,9 +3029,7 @@ static int bx_tile(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m) {
                                                  : 6.0 + per_cu(n128) * (0.8 + 0.0098 * k);
   const double c64 = n64 <= device_cus() ? 4.5 + 0.0078 * k : 4.5 + per_cu(n64) * (0.5 + 0.0038 * k);
   if (c64 < c128 && c64 < c256) return 64;
-  // (128-row tiles read twice the operand bytes: near the line the step on a dozen matrices each
-  // of four shapes, whose launches run beside each other, was 0.5% slower with them)
-  return c128 < 0.6 * c256 ? 128 : 256;
+  return c128 < (beside ? 0.6 : 0.9) * c256 ? 128 : 256;
 }
 
 // `g` on TM-row tiles covering round_up(m, 128) rows (of a SYRK, columns too).
@@ -3052,7 +3055,7 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
                      int64_t ldb, int64_t sb, const void* cin, int64_t ldc, int64_t sc,
                      void* out, int64_t ldo, int64_t so, void* out_t, int64_t ldt, int64_t st,
                      int64_t Mv, int64_t Nv, float alpha, float beta, const float* scale,
-                     int scale_mode, hipStream_t stream) {
+                     int scale_mode, int beside, hipStream_t stream) {
   GemmArgs g;
   g.a = a;
   g.b = b;
@@ -3134,7 +3137,7 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
       }
       MuonApply none;
       none.nb = 1;
-      const int TM = bx_tile(batch, M, N, K, Mv);
+      const int TM = bx_tile(batch, M, N, K, Mv, beside);
       if (TM == 256) {
         // persistent: at most one workgroup per CU walks the tile list
         const dim3 pg((unsigned)persistent_wgs(blocks));
@@ -3162,7 +3165,7 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
         gp.tiles_per_batch = (T - 1) * T / 2 + (2 * T - 1 + 3) / 4;
         gp.tiles_total = gp.tiles_per_batch * (int)batch;
       }
-      const int TM = syrk_tile(batch, Mv, M, K, gp.tiles_total);
+      const int TM = syrk_tile(batch, Mv, K, gp.tiles_total, beside);
       if (TM != 256) {
         const GemmArgs gt = on_tiles(g, mode, TM, Mv, N, batch);
         const dim3 tg((unsigned)gt.tiles_total);
@@ -3216,14 +3219,15 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
 // tiles costs less than the 256-row one and a post-pass (which reads U and the parameters
 // and writes the parameters, about 5 TB/s). Six fp32
 // matrices of 768 x 3072: 26 us and 29 us of post-pass against 45 us.
-int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int64_t n, int pdt) {
+int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int64_t n, int pdt,
+                     int beside) {
   if (pdt == MUON_DT_BF16) return 1;
   const int pes = pdt == MUON_DT_F32 ? 4 : 2;
   const double post = 6.0 + (double)batch * m * n * (2 + 2 * pes) / 5.0e6;
   const int64_t n256 = (M / 256) * (N / 256) * batch, n128 = round_up(m, 128) / 128 * (N / 128) * batch;
   const double c256 = rounds_of(n256) * (9.0 + 0.0215 * (double)K);
   const double c128 = 6.0 + per_cu(n128) * (0.8 + 0.0098 * (double)K);
-  return bx_tile(batch, M, N, K, m) != 256 || c128 < c256 + 0.5 * post;
+  return bx_tile(batch, M, N, K, m, beside) != 256 || c128 < c256 + 0.5 * post;
 }
 
 // The last iteration's X' = a X + B X with the post-pass applied in its epilogue: extents and
@@ -3234,7 +3238,7 @@ int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, 
 int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const void* a,
                            int64_t lda, int64_t sa, const void* b, int64_t ldb, int64_t sb,
                            int64_t Mv, int64_t Nv, float alpha, float beta, const float* scale,
-                           int scale_mode, const MuonApply& ap, int pdt, int tall,
+                           int scale_mode, const MuonApply& ap, int pdt, int tall, int beside,
                            hipStream_t stream) {
   if (K % 128 || M % BF_BM || N % BF_BM || alpha == 0.0f || ap.nb <= 0 ||
       (batch + ap.nb - 1) / ap.nb > MUON_APPLY_MAX || ap.pcols % 8 ||
@@ -3280,7 +3284,7 @@ int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const
     muon_set_error("gemm_apply: cannot reserve LDS");
     return MUON_ERR_LAUNCH;
   }
-  int TM = bx_tile(batch, M, N, K, Mv);
+  int TM = bx_tile(batch, M, N, K, Mv, beside);
   if (TM == 256 && pdt != MUON_DT_BF16) TM = 128;
   if (TM == 256) {
     const int wgs = persistent_wgs(blocks);

@@ -54,6 +54,17 @@ _SIGNATURES = {
          _c_f32, _c_f32, _c_int, _pp, _c_int, _c_i64, ctypes.POINTER(_c_f32), _c_f32, _c_int,
          _vp],
     ),
+    "muon_orth_run_beside": (
+        _c_int,
+        [_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(ctypes.c_double), _c_int,
+         _c_f32, _c_f32, _c_int, _vp],
+    ),
+    "muon_orth_run_apply_beside": (
+        _c_int,
+        [_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(ctypes.c_double), _c_int,
+         _c_f32, _c_f32, _c_int, _pp, _c_int, _c_i64, ctypes.POINTER(_c_f32), _c_f32, _c_int,
+         _c_int, _vp],
+    ),
     "muon_orth_extract": (
         _c_int, [_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_int, _vp]
     ),

@@ -74,6 +74,31 @@ def release_workspaces() -> None:
 
 
 # ---------------------------------------------------------------------------------
+# Calls made while a step's other buckets run on other streams say so to the library, which then
+# weighs what a launch takes from its neighbours (the results are the same). Per thread.
+
+_neighbours = threading.local()
+
+
+class beside_others:
+    """Context of calls whose launches run beside other streams' (``on`` False: no effect)."""
+
+    def __init__(self, on: bool = True):
+        self.on = on
+
+    def __enter__(self):
+        self.before = getattr(_neighbours, "on", False)
+        _neighbours.on = self.on or self.before
+
+    def __exit__(self, *exc):
+        _neighbours.on = self.before
+
+
+def _beside() -> int:
+    return int(getattr(_neighbours, "on", False))
+
+
+# ---------------------------------------------------------------------------------
 # shape helpers
 
 
@@ -316,17 +341,17 @@ def _fused_step_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Tenso
         # the iteration and the apply in one call: the library fuses the apply into the last
         # X' = a X + B X where the shapes allow it, else runs the post-pass after it
         _lib.check(
-            lib.muon_orth_run_apply(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                                    _flat_coeffs(coeffs), steps, prescale, eps, count,
-                                    _lib.ptr_array(params), _lib.dtype_code(params[0].dtype), nb,
-                                    _lib.f32_array(lrs), float(weight_decay), int(cautious_wd),
-                                    s),
+            lib.muon_orth_run_apply_beside(
+                ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols, _flat_coeffs(coeffs),
+                steps, prescale, eps, count, _lib.ptr_array(params),
+                _lib.dtype_code(params[0].dtype), nb, _lib.f32_array(lrs), float(weight_decay),
+                int(cautious_wd), _beside(), s),
             "muon_orth_run_apply",
         )
         return
     _lib.check(
-        lib.muon_orth_run(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                          _flat_coeffs(coeffs), steps, prescale, eps, s),
+        lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
+                                 _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
         "muon_orth_run",
     )
     _lib.check(
@@ -402,8 +427,8 @@ def _fused_normuon_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Te
         "muon_prepass",
     )
     _lib.check(
-        lib.muon_orth_run(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                          _flat_coeffs(coeffs), steps, prescale, eps, s),
+        lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
+                                 _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
         "muon_orth_run",
     )
     _lib.check(
@@ -523,10 +548,10 @@ def _fused_lp_impl(params: list[Tensor], grads: list[Tensor], codes: list[Tensor
     )
     # the iteration and the apply (fused into the last B X where the shapes allow)
     _lib.check(
-        lib.muon_orth_run_apply(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                                _flat_coeffs(coeffs), steps, prescale, eps, count,
-                                _lib.ptr_array(params), _lib.dtype_code(params[0].dtype), nb,
-                                _lib.f32_array(lrs), float(weight_decay), int(cautious_wd), s),
+        lib.muon_orth_run_apply_beside(
+            ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols, _flat_coeffs(coeffs), steps,
+            prescale, eps, count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype), nb,
+            _lib.f32_array(lrs), float(weight_decay), int(cautious_wd), _beside(), s),
         "muon_orth_run_apply",
     )
 

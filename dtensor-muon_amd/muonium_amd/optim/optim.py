@@ -9,9 +9,9 @@ driver — there is no tracing compiler on this path.
 
 from __future__ import annotations
 
-import contextlib
 import functools
 import math
+import threading
 from typing import cast
 
 import torch
@@ -23,6 +23,7 @@ from torch.optim.optimizer import (
     _use_grad_for_differentiable,
 )
 
+from muonium_amd._ops import beside_others
 from muonium_amd.orthogonalize import OrthogonalizationStrategy
 from muonium_amd.utils import group_tensors_by_shape, move_tensors_to_device
 from muonium_amd.utils.offload import pipeline_supported, run_offloaded
@@ -84,13 +85,16 @@ def _per_tensor_runs(algorithm: MuonAlgorithm, params, grads, state, split_sizes
 # GPU_MAX_HW_QUEUES is 4 by default: with the caller's stream, one hardware queue each (a
 # fourth side stream shared a queue with the third, which serialized their buckets)
 _MAX_SIDE_STREAMS = 3
-_side_streams: dict[tuple[int, int], torch.cuda.Stream] = {}
+# Side streams, and the events of their forks and joins, each of one thread (its identifier is part
+# of the key): workspaces are cached by stream, so threads stepping at the same time must not
+# share a side stream, nor an event between one's record and its wait.
+_side_streams: dict[tuple[int, int, int], torch.cuda.Stream] = {}
 
 
 def _side_stream(device: torch.device, slot: int) -> torch.cuda.Stream:
-    """Side stream `slot` of `device` (default priority), created once per process."""
+    """Side stream `slot` of `device` (default priority), created once per thread."""
     index = device.index if device.index is not None else torch.cuda.current_device()
-    key = (index, slot)
+    key = (threading.get_ident(), index, slot)
     stream = _side_streams.get(key)
     if stream is None:
         stream = _side_streams[key] = torch.cuda.Stream(device=index)
@@ -101,9 +105,10 @@ _sync_events: dict[tuple, torch.cuda.Event] = {}
 
 
 def _wait(waiter: torch.cuda.Stream, producer: torch.cuda.Stream, key: tuple) -> None:
-    """``waiter.wait_stream(producer)`` with an event kept per (device, slot, direction):
-    recording an event again is legal (a wait already issued keeps the state it saw), and
-    it saves creating one per fork and join."""
+    """``waiter.wait_stream(producer)`` with an event kept per (thread, device, slot,
+    direction): recording an event again is legal (a wait already issued keeps the state it
+    saw), and it saves creating one per fork and join."""
+    key = (threading.get_ident(), *key)
     ev = _sync_events.get(key)
     if ev is None:
         ev = _sync_events[key] = torch.cuda.Event()
@@ -150,6 +155,26 @@ def _concurrent_plan(buckets, algorithm: MuonAlgorithm,
     side = ranked[:-1] if len(work) == len(buckets) else ranked
     slots = {bi: k % _MAX_SIDE_STREAMS for k, bi in enumerate(side)}
     return slots, side + [bi for bi in natural if bi not in slots]
+
+
+def _run_on_streams(slots: dict[int, int], order: list[int], device_of, run) -> None:
+    """``run(i)`` for every i of ``order``; those with a slot on that side stream of their
+    device, forked from the caller's stream at first use and joined back into it at the end."""
+    forked: dict[tuple[torch.device, int], torch.cuda.Stream] = {}
+    with beside_others(bool(slots)):
+        for i in order:
+            if i not in slots:
+                run(i)
+                continue
+            key = (device_of(i), slots[i])
+            side = _side_stream(*key)
+            if key not in forked:
+                _wait(side, torch.cuda.current_stream(key[0]), (*key, 0))
+                forked[key] = side
+            with torch.cuda.stream(side):
+                run(i)
+    for key, side in forked.items():
+        _wait(torch.cuda.current_stream(key[0]), side, (*key, 1))
 
 
 class Muon(torch.optim.Optimizer):
@@ -494,7 +519,9 @@ class Muon(torch.optim.Optimizer):
             **opts,
         )
         if not foreach:
-            for idx in _per_tensor_runs(algorithm, params, grads, state, split_sizes):
+            runs = _per_tensor_runs(algorithm, params, grads, state, split_sizes)
+
+            def update(idx) -> None:
                 if len(idx) == 1:
                     i = idx[0]
                     algorithm.update(params[i], grads[i], {k: b[i] for k, b in state.items()},
@@ -504,26 +531,29 @@ class Muon(torch.optim.Optimizer):
                         [params[i] for i in idx], [grads[i] for i in idx],
                         {k: [b[i] for i in idx] for k, b in state.items()},
                         [lr_ratios[i] for i in idx], **hp)
+
+            # runs that are one fused launch sequence each go side by side as the foreach
+            # driver's buckets do; anything else in the reference's order, one after the other
+            if len(runs) > 1 and getattr(algorithm, "batches_per_tensor",
+                                         lambda s: False)(split_sizes):
+                views = [(params[idx[0]].device, None, [grads[i] for i in idx], None, None)
+                         for idx in runs]
+                slots, order = _concurrent_plan(views, algorithm, None)
+            else:
+                slots, order = {}, list(range(len(runs)))
+            _run_on_streams(slots, order, lambda ri: params[runs[ri][0]].device,
+                            lambda ri: update(runs[ri]))
             return
 
         buckets = _group_muon_tensors(params, grads, state, lr_ratios)
         slots, order = _concurrent_plan(buckets, algorithm, self.batch_size)
-        forked: dict[tuple[torch.device, int], torch.cuda.Stream] = {}
-        for bi in order:
+
+        def bucket(bi) -> None:
             device, dev_p, dev_g, dev_state, dev_lr = buckets[bi]
-            if bi in slots:
-                side = _side_stream(device, slots[bi])
-                if (device, slots[bi]) not in forked:
-                    _wait(side, torch.cuda.current_stream(device), (device, slots[bi], 0))
-                    forked[(device, slots[bi])] = side
-                ctx = torch.cuda.stream(side)
-            else:
-                ctx = contextlib.nullcontext()
-            with ctx:
-                self._muon_bucket(algorithm, hp, nesterov, maximize, device, dev_p, dev_g,
-                                  dev_state, dev_lr)
-        for (device, slot), side in forked.items():
-            _wait(torch.cuda.current_stream(device), side, (device, slot, 1))
+            self._muon_bucket(algorithm, hp, nesterov, maximize, device, dev_p, dev_g,
+                              dev_state, dev_lr)
+
+        _run_on_streams(slots, order, lambda bi: buckets[bi][0], bucket)
 
     def _muon_bucket(self, algorithm, hp, nesterov, maximize, device, dev_p, dev_g, dev_state,
                      dev_lr) -> None:

@@ -116,11 +116,11 @@ int muon_orth_run(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch, int64
 
 /* muon_orth_run followed by muon_postpass of its result (u = NULL, the same arguments),
  * with the post-pass fused into the last iteration's X = a*X + B X where the shapes allow
- * (bf16 workspace and parameters; on the iterate's short side either at least 768 valid
- * rows after padding to 128, or at most 64 rows with the parameter stored wide;
- * ntensors * nb == batch, parameter rows a multiple of 8 elements in the stored
- * orientation, 16-byte aligned parameters; the last product launches once per 128 tensors):
- * each bf16 element of the last X' is applied to its parameter element
+ * (bf16 workspace; bf16 parameters, or fp32 / fp16 ones in launches small enough that the
+ * fused form is the faster one; on the iterate's short side more than 64 rows, or at most 64
+ * with bf16 parameters stored wide; ntensors * nb == batch, parameter rows a multiple of 8
+ * elements in the stored orientation, 16-byte aligned parameters; the last product launches
+ * once per 128 tensors): each bf16 element of the last X' is applied to its parameter element
  * (cautious weight decay and the shape-scaled step, exactly as muon_postpass) and X' is
  * not stored, so the workspace does not hold U afterwards. Otherwise the two calls run
  * one after the other. Replaces the orthogonalize-then-apply sequence of
@@ -129,6 +129,19 @@ int muon_orth_run_apply(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,
                         int64_t cols, const double* coeffs, int steps, float prescale,
                         float eps, int ntensors, void* const* params, int p_dtype, int64_t nb,
                         const float* adjusted_lrs, float wd, int cautious, void* stream);
+
+/* muon_orth_run / muon_orth_run_apply for calls whose launches may run beside other calls'
+ * launches on other streams (beside != 0): where two tile sizes of a product take about as
+ * long, the one that leaves more of the device to the others. The results are bit for bit
+ * the same. */
+int muon_orth_run_beside(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch, int64_t rows,
+                         int64_t cols, const double* coeffs, int steps, float prescale, float eps,
+                         int beside, void* stream);
+int muon_orth_run_apply_beside(void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,
+                               int64_t rows, int64_t cols, const double* coeffs, int steps,
+                               float prescale, float eps, int ntensors, void* const* params,
+                               int p_dtype, int64_t nb, const float* adjusted_lrs, float wd,
+                               int cautious, int beside, void* stream);
 
 /* Copy U (first `batch` matrices, stored layout) out of the workspace into a
  * contiguous (batch, rows, cols) tensor of out_dtype. Replaces the return/unbind of
