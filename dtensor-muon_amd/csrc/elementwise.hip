@@ -4,6 +4,8 @@
 // pre-pass can emit both the stored layout and its transpose (through LDS) in one
 // read of the gradient and momentum, and reduce the Frobenius-norm partials of each
 // tile in a fixed order (deterministic, no atomics).
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -547,11 +549,13 @@ __global__ __launch_bounds__(256) void postpass_slab_kernel(PostArgs a) {
 }
 
 // ---- NorMuon ---------------------------------------------------------------------------
-// ss[r] = sum over the columns of stored row r of U^2 (fp32, fixed order), for the 64
-// stored rows r0 .. r0+63 of one matrix per workgroup. TRANS: U is the wide iterate of a
-// tall matrix, stored row r = its column r (lanes over r, coalesced; the 4 waves split the
-// columns and are combined in order). Otherwise lanes stride over the columns of a row
-// (VEC consecutive values each) and a butterfly sums them.
+// ss[r] = sum over the columns of stored row r of U^2 (fp32, fixed order). TRANS: U is the wide
+// iterate of a tall matrix, stored row r = its column r; 64 rows per workgroup (lanes over r,
+// coalesced; the 4 waves split the columns and are combined in order). Otherwise 16 rows per
+// workgroup: each wave strides over the columns of four rows at a time (VEC consecutive
+// values per lane and row) and a butterfly sums them. A row is one latency chain of loads, so
+// the rows in flight decide the time of a small launch: with 16 rows one after the other per
+// wave a dozen 1000 x 1000 matrices took 27 us (24 MB, 5 us of traffic), 9 us so.
 struct RowSsArgs {
   const void* u;  // matrix 0 of this launch
   int64_t u_pitch, u_mstride, rows, cols;
@@ -584,79 +588,110 @@ __global__ __launch_bounds__(256) void row_sumsq_kernel(RowSsArgs a) {
     __syncthreads();
     if (wave == 0 && r < a.rows) ss[r] = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
   } else {
-    for (int i = 0; i < 16; ++i) {
-      const int64_t r = r0 + wave * 16 + i;
-      if (r >= a.rows) break;
-      float s = 0.0f;
-      if constexpr (VEC == 8) {
-        for (int64_t c = (int64_t)lane * 8; c < a.cols; c += 512) {
-          float v[8];
-          Vec8<UDT>::load(a.u, base + r * a.u_pitch + c, v);
-          if (a.has_uscale) {
+    const int64_t rw = (int64_t)blockIdx.x * 16 + wave * 4;
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // rows past the end read the last one (not stored)
+    int64_t row[4];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = Elem<UDT>::round(v[e] * us);
+    for (int i = 0; i < 4; ++i) row[i] = base + std::min<int64_t>(rw + i, a.rows - 1) * a.u_pitch;
+    if constexpr (VEC == 8) {
+      for (int64_t c = (int64_t)lane * 8; c < a.cols; c += 512) {
+        float v[4][8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Vec8<UDT>::load(a.u, row[i] + c, v[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float x = a.has_uscale ? Elem<UDT>::round(v[i][e] * us) : v[i][e];
+            s[i] += x * x;
           }
+      }
+    } else {
+      for (int64_t c = lane; c < a.cols; c += 64) {
+        float v[4];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) s += v[e] * v[e];
-        }
-      } else {
-        for (int64_t c = lane; c < a.cols; c += 64) {
-          float v = Elem<UDT>::load(a.u, base + r * a.u_pitch + c);
-          if (a.has_uscale) v = Elem<UDT>::round(v * us);
-          s += v * v;
+        for (int i = 0; i < 4; ++i) v[i] = Elem<UDT>::load(a.u, row[i] + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float x = a.has_uscale ? Elem<UDT>::round(v[i] * us) : v[i];
+          s[i] += x * x;
         }
       }
-      s = warp_sum(s);
-      if (lane == 0) ss[r] = s;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[i] = warp_sum(s[i]);
+      if (lane == 0 && rw + i < a.rows) ss[rw + i] = s[i];
     }
   }
 }
 
-// The transposed case with 16-byte loads: row r of the update is column r of the stored
-// result (tall matrices), so a lane takes 8 consecutive rows (8 consecutive elements of a
-// stored row) and a workgroup 512 rows; wave w sums stored rows w, w + 4, ... with four
-// loads in flight. The same sums in the same order as row_sumsq_kernel<UDT, 1, true>.
-// Needs rows % 8 == 0 and 16-byte aligned stored rows.
-template <int UDT>
-__global__ __launch_bounds__(256) void row_sumsq_t8_kernel(RowSsArgs a) {
+// R consecutive elements as raw bits (R = 8: Raw8; R = 2: one 4- or 8-byte load).
+template <int DT, int R>
+struct RawR : Raw8<DT> {};
+template <int DT>
+struct RawR<DT, 2> {
+  typename std::conditional<DT == MUON_DT_F32, uint64_t, uint32_t>::type w;
+  MUON_DEVICE void load(const void* p, int64_t i) {
+    w = *(const decltype(w)*)((const char*)p + i * (DT == MUON_DT_F32 ? 4 : 2));
+  }
+  MUON_DEVICE void unpack(float (&v)[2]) const {
+    v[0] = Elem<DT>::load(&w, 0);
+    v[1] = Elem<DT>::load(&w, 1);
+  }
+};
+
+// The transposed case with wide loads: row r of the update is column r of the stored result (tall
+// matrices), so a lane takes R consecutive rows (R consecutive elements of a stored row) and a
+// workgroup 64 R rows; wave w sums stored rows w, w + 4, ... with DEPTH loads in flight. The same
+// sums in the same order as row_sumsq_kernel<UDT, 1, true>. Needs rows % R == 0 and stored rows
+// aligned to R elements. R = 8 (16-byte loads) streams at the rate of the device where the launch
+// fills it; a small one waits for a lane's chain over the columns, and R = 2 gives it four times
+// the waves: four 2720 x 1000 matrices took 82 us with R = 8 and four loads in flight, 57 with
+// 16, 27 to 33 with R = 2 and 32.
+template <int UDT, int R>
+__global__ __launch_bounds__(256) void row_sumsq_t_kernel(RowSsArgs a) {
 #pragma clang fp contract(off)
-  __shared__ float part[4][512];
+  constexpr int DEPTH = R == 2 ? 32 : UDT == MUON_DT_F32 ? 8 : 16;
+  __shared__ float part[4][64 * R];
   const int mat = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t rb = (int64_t)blockIdx.x * 512;
-  const int64_t r = rb + lane * 8;
+  const int64_t rb = (int64_t)blockIdx.x * (64 * R);
+  const int64_t r = rb + lane * R;
   const int64_t base = (int64_t)mat * a.u_mstride;
   float* ss = a.ss + (int64_t)mat * a.ss_mstride;
   const float us = a.uscale[mat / a.nb];
-  float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  float s[R];
+#pragma unroll
+  for (int e = 0; e < R; ++e) s[e] = 0.0f;
+  auto add = [&](const RawR<UDT, R>& w) {
+    float v[R];
+    w.unpack(v);
+#pragma unroll
+    for (int e = 0; e < R; ++e) {
+      const float x = a.has_uscale ? Elem<UDT>::round(v[e] * us) : v[e];
+      s[e] += x * x;
+    }
+  };
   if (r < a.rows) {
     int64_t c = wave;
-    for (; c + 12 < a.cols; c += 16) {
-      float v[4][8];
+    for (; c + 4 * (DEPTH - 1) < a.cols; c += 4 * DEPTH) {
+      RawR<UDT, R> w[DEPTH];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) Vec8<UDT>::load(a.u, base + (c + 4 * q) * a.u_pitch + r, v[q]);
+      for (int q = 0; q < DEPTH; ++q) w[q].load(a.u, base + (c + 4 * q) * a.u_pitch + r);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = a.has_uscale ? Elem<UDT>::round(v[q][e] * us) : v[q][e];
-          s[e] += x * x;
-        }
-      }
+      for (int q = 0; q < DEPTH; ++q) add(w[q]);
     }
     for (; c < a.cols; c += 4) {
-      float v[8];
-      Vec8<UDT>::load(a.u, base + c * a.u_pitch + r, v);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float x = a.has_uscale ? Elem<UDT>::round(v[e] * us) : v[e];
-        s[e] += x * x;
-      }
+      RawR<UDT, R> w;
+      w.load(a.u, base + c * a.u_pitch + r);
+      add(w);
     }
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) part[wave][lane * 8 + e] = s[e];
+  for (int e = 0; e < R; ++e) part[wave][lane * R + e] = s[e];
   __syncthreads();
-  for (int k = tid; k < 512; k += 256) {
+  for (int k = tid; k < 64 * R; k += 256) {
     if (rb + k < a.rows) ss[rb + k] = ((part[0][k] + part[1][k]) + part[2][k]) + part[3][k];
   }
 }
@@ -1101,22 +1136,30 @@ int muon_launch_normuon_stats(int ntensors, void* const* vars, int vdt, const vo
   ra.cols = cols;
   ra.ss = ss;
   ra.ss_mstride = ss_mstride;
-  dim3 grid((unsigned)((rows + 63) / 64), (unsigned)nmat);
+  const dim3 grid64((unsigned)((rows + 63) / 64), (unsigned)nmat);
+  const dim3 grid16((unsigned)((rows + 15) / 16), (unsigned)nmat);
   const bool vec8 = !u_trans && (cols % 8) == 0 && (u_pitch % 8) == 0 && (u_mstride % 8) == 0 &&
                     !((uintptr_t)u & 15);
-  const bool t8 = u_trans && (rows % 8) == 0 && (u_pitch % 8) == 0 && (u_mstride % 8) == 0 &&
-                  !((uintptr_t)u & 15);
+  // 8 rows per lane where that fills the device (two workgroups per CU), else 2
+  const int64_t wg8 = (rows + 511) / 512 * nmat;
+  const bool t8 = u_trans && wg8 >= 512 && (rows % 8) == 0 && (u_pitch % 8) == 0 &&
+                  (u_mstride % 8) == 0 && !((uintptr_t)u & 15);
+  const bool t2 = u_trans && (rows % 2) == 0 && (u_pitch % 2) == 0 && (u_mstride % 2) == 0 &&
+                  !((uintptr_t)u & 7);
   const dim3 grid8((unsigned)((rows + 511) / 512), (unsigned)nmat);
+  const dim3 grid2((unsigned)((rows + 127) / 128), (unsigned)nmat);
 #define ROWSS(UDT_)                                                                        \
   do {                                                                                     \
     if (t8)                                                                                \
-      hipLaunchKernelGGL((row_sumsq_t8_kernel<UDT_>), grid8, dim3(256), 0, s, ra);          \
+      hipLaunchKernelGGL((row_sumsq_t_kernel<UDT_, 8>), grid8, dim3(256), 0, s, ra);        \
+    else if (t2)                                                                           \
+      hipLaunchKernelGGL((row_sumsq_t_kernel<UDT_, 2>), grid2, dim3(256), 0, s, ra);        \
     else if (u_trans)                                                                      \
-      hipLaunchKernelGGL((row_sumsq_kernel<UDT_, 1, true>), grid, dim3(256), 0, s, ra);     \
+      hipLaunchKernelGGL((row_sumsq_kernel<UDT_, 1, true>), grid64, dim3(256), 0, s, ra);   \
     else if (vec8)                                                                         \
-      hipLaunchKernelGGL((row_sumsq_kernel<UDT_, 8, false>), grid, dim3(256), 0, s, ra);    \
+      hipLaunchKernelGGL((row_sumsq_kernel<UDT_, 8, false>), grid16, dim3(256), 0, s, ra);  \
     else                                                                                   \
-      hipLaunchKernelGGL((row_sumsq_kernel<UDT_, 1, false>), grid, dim3(256), 0, s, ra);    \
+      hipLaunchKernelGGL((row_sumsq_kernel<UDT_, 1, false>), grid16, dim3(256), 0, s, ra);  \
   } while (0)
   switch (udt) {
     case MUON_DT_F32: ROWSS(MUON_DT_F32); break;
