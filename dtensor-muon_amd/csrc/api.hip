@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "common.h"
@@ -76,6 +77,12 @@ int muon_launch_short_bx_apply(const OrthLayout& L, const void* x, const void* b
 int muon_short_gspace_ok(const OrthLayout& L, const double* coeffs, int steps);
 int muon_launch_short_gspace(const OrthLayout& L, float* part, int64_t batch, const double* coeffs,
                              int steps, float prescale, float eps, float* scale, hipStream_t s);
+
+int muon_launch_products(int mode, int n, const MuonProduct* items, float alpha, float beta,
+                         int scale_mode, const MuonApply* ap, int pdt, int tall,
+                         hipStream_t stream);
+int muon_launch_finalize_group(int n, const OrthLayout* L, char* const* ws, const int64_t* batch,
+                               float prescale, float eps, hipStream_t s);
 
 enum { MODE_GEMM = 0, MODE_SYRK = 1 };
 
@@ -586,6 +593,199 @@ int muon_orth_run_apply_beside(void* ws, int ws_dtype, int64_t ws_batch, int64_t
   const ApplyReq ap = {params, adjusted_lrs, p_dtype, ntensors, nb, rows, cols, wd, cautious};
   return orth_run_impl(ws, ws_dtype, ws_batch, batch, rows, cols, coeffs, steps, prescale, eps,
                        &ap, beside, stream);
+}
+
+static int orth_run_group(int nbuckets, const MuonBucket* buckets, const double* coeffs,
+                          int steps, float prescale, float eps, float wd, int cautious,
+                          void* stream) {
+  if (nbuckets < 0 || (nbuckets > 0 && !buckets) || steps < 0 || (steps > 0 && !coeffs)) {
+    muon_set_error("orth_run_group: bad arguments (%d buckets, %d steps)", nbuckets, steps);
+    return MUON_ERR_ARG;
+  }
+  std::vector<OrthLayout> L;
+  std::vector<char*> ws;
+  std::vector<int64_t> batch;
+  std::vector<const MuonBucket*> own;  // in common launches
+  for (int i = 0; i < nbuckets; ++i) {
+    const MuonBucket& b = buckets[i];
+    if (!b.ws || b.batch < 0 || b.batch > b.ws_batch || b.rows <= 0 || b.cols <= 0 ||
+        (b.ntensors > 0 && (!b.params || !b.adjusted_lrs || b.nb <= 0 || !io_dtype_ok(b.p_dtype)))) {
+      muon_set_error("orth_run_group: bad bucket %d", i);
+      return MUON_ERR_ARG;
+    }
+    if (b.batch == 0) continue;
+    const OrthLayout l = muon_orth_layout(MUON_DT_BF16, b.ws_batch, b.rows, b.cols);
+    // iterates of at most 64 rows have products of their own
+    if (l.short_m || steps == 0) {
+      int rc = b.ntensors > 0
+                   ? muon_orth_run_apply(b.ws, MUON_DT_BF16, b.ws_batch, b.batch, b.rows, b.cols,
+                                         coeffs, steps, prescale, eps, b.ntensors, b.params,
+                                         b.p_dtype, b.nb, b.adjusted_lrs, wd, cautious, stream)
+                   : muon_orth_run(b.ws, MUON_DT_BF16, b.ws_batch, b.batch, b.rows, b.cols, coeffs,
+                                   steps, prescale, eps, stream);
+      if (rc != MUON_OK) return rc;
+      continue;
+    }
+    L.push_back(l);
+    ws.push_back((char*)b.ws);
+    batch.push_back(b.batch);
+    own.push_back(&b);
+  }
+  const int n = (int)own.size();
+  if (n == 0) return MUON_OK;
+  hipStream_t s = (hipStream_t)stream;
+  double xx = 0.0, aa = 0.0, bx = 0.0;
+  for (int i = 0; i < n; ++i) {
+    const double bm = (double)batch[i], md = (double)L[i].m, nd = (double)L[i].n;
+    xx += bm * md * (md + 1) * nd;
+    aa += bm * md * (md + 1) * md;
+    bx += bm * 2.0 * md * md * nd;
+  }
+  int rc;
+  {
+    Timed t(MUON_K_OTHER, 0.0, s);
+    rc = muon_launch_finalize_group(n, L.data(), ws.data(), batch.data(), prescale, eps, s);
+  }
+  if (rc != MUON_OK) return rc;
+  // longest sums first: their tiles start first
+  std::vector<int> order(n);
+  for (int i = 0; i < n; ++i) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int p, int q) { return L[p].n_pad > L[q].n_pad; });
+  // the fused apply of a bucket, where its shape allows
+  std::vector<char> fuse(n, 0);
+  for (int i = 0; i < n; ++i) {
+    const MuonBucket& b = *own[i];
+    fuse[i] = b.ntensors > 0 && (int64_t)b.ntensors * b.nb == b.batch && b.cols % 8 == 0 &&
+              b.ntensors <= MUON_APPLY_MAX;
+    for (int t = 0; fuse[i] && t < b.ntensors; ++t)
+      fuse[i] = b.params[t] && !((uintptr_t)b.params[t] & 15);
+  }
+  std::vector<MuonProduct> items(n);
+  for (int it = 0; it < steps; ++it) {
+    const float a = (float)coeffs[3 * it], pb = (float)coeffs[3 * it + 1],
+                c = (float)coeffs[3 * it + 2];
+    const bool first = it == 0, last = it + 1 == steps;
+    auto fill = [&](int i, int kind, MuonProduct& p) {
+      const OrthLayout& l = L[i];
+      char* w = ws[i];
+      char* X[2] = {w + l.off_x0, w + l.off_x1};
+      const int64_t kq = std::min(l.m_pad, round_up(l.m, 128));
+      memset(&p, 0, sizeof(p));
+      p.batch = batch[i];
+      p.m = l.m;
+      p.nv = l.n;
+      p.scale = (const float*)(w + l.off_scale);
+      if (kind == 0) {  // A = X X^T
+        p.a = X[it & 1];
+        p.lda = l.x_pitch;
+        p.sa = l.m_pad * l.x_pitch;
+        p.out = w + l.off_a;
+        p.K = l.n_pad;
+        p.N = l.m_pad;
+      } else if (kind == 1) {  // B = c A A + b A
+        p.a = w + l.off_a;
+        p.lda = l.m_pad;
+        p.sa = l.m_pad * l.m_pad;
+        p.out = w + l.off_b;
+        p.K = kq;
+        p.N = l.m_pad;
+      } else {  // X' = a X + B X
+        p.a = w + l.off_b;
+        p.lda = l.m_pad;
+        p.sa = l.m_pad * l.m_pad;
+        p.b = X[it & 1];
+        p.ldb = l.x_pitch;
+        p.sb = l.m_pad * l.x_pitch;
+        p.out = X[(it + 1) & 1];
+        p.K = kq;
+        p.N = l.n_pad;
+      }
+      p.ldo = kind == 2 ? l.x_pitch : l.m_pad;
+      p.so = l.m_pad * p.ldo;
+    };
+    for (int k = 0; k < n; ++k) fill(order[k], 0, items[k]);
+    {
+      Timed t(MUON_K_SYRK_XX, xx, s);
+      rc = muon_launch_products(MODE_SYRK, n, items.data(), 1.0f, 0.0f, first ? 2 : 0, nullptr, 0, 0, s);
+    }
+    if (rc != MUON_OK) return rc;
+    for (int k = 0; k < n; ++k) fill(order[k], 1, items[k]);
+    {
+      Timed t(MUON_K_SYRK_AA, aa, s);
+      if (c != 0.0f)
+        rc = muon_launch_products(MODE_SYRK, n, items.data(), c, pb, 0, nullptr, 0, 0, s);
+      else  // (the small tiles fold beta / alpha: a zero c goes bucket by bucket)
+        for (int k = 0; k < n && rc == MUON_OK; ++k) {
+          const MuonProduct& p = items[k];
+          const int64_t mp = p.N;
+          rc = muon_launch_gemm(MUON_DT_BF16, MODE_SYRK, false, p.batch, mp, mp, p.K, p.a, mp,
+                                mp * mp, p.a, mp, mp * mp, p.a, mp, mp * mp, p.out, mp, mp * mp,
+                                nullptr, 0, 0, p.m, p.m, c, pb, nullptr, 0, 0, s);
+        }
+    }
+    if (rc != MUON_OK) return rc;
+    // the last product: fused applies by orientation and parameter type, MUON_APPLY_MAX tensors
+    // per launch; the others store X'
+    std::vector<char> done(n, 0);
+    for (int k0 = 0; last && k0 < n; ++k0) {
+      const int i0 = order[k0];
+      if (done[i0] || !fuse[i0]) continue;
+      MuonApply ap;
+      memset(&ap, 0, sizeof(ap));
+      ap.nb = 1;
+      ap.wd = wd;
+      ap.cautious = cautious;
+      int cnt = 0, tensors = 0;
+      double work = 0.0;
+      for (int k = k0; k < n; ++k) {
+        const int i = order[k];
+        const MuonBucket& b = *own[i];
+        if (done[i] || !fuse[i] || L[i].tall != L[i0].tall || b.p_dtype != own[i0]->p_dtype ||
+            tensors + b.ntensors > MUON_APPLY_MAX)
+          continue;
+        fill(i, 2, items[cnt]);
+        items[cnt].t0 = tensors;
+        items[cnt].nb = (int)b.nb;
+        ++cnt;
+        for (int t = 0; t < b.ntensors; ++t) {
+          ap.params[tensors] = b.params[t];
+          ap.adj[tensors++] = b.adjusted_lrs[t];
+        }
+        work += (double)b.batch * 2.0 * L[i].m * L[i].m * L[i].n;
+        done[i] = 1;
+      }
+      Timed t(MUON_K_GEMM_BX_APPLY, work, s);
+      rc = muon_launch_products(MODE_GEMM, cnt, items.data(), 1.0f, a, first ? 1 : 0, &ap,
+                                own[i0]->p_dtype, L[i0].tall, s);
+      if (rc != MUON_OK) return rc;
+    }
+    int cnt = 0;
+    for (int k = 0; k < n; ++k)
+      if (!done[order[k]]) fill(order[k], 2, items[cnt++]);
+    if (cnt > 0) {
+      Timed t(MUON_K_GEMM_BX, last ? 0.0 : bx, s);
+      rc = muon_launch_products(MODE_GEMM, cnt, items.data(), 1.0f, a, first ? 1 : 0, nullptr, 0, 0, s);
+    }
+    if (rc != MUON_OK) return rc;
+  }
+  for (int i = 0; i < n; ++i) {
+    const MuonBucket& b = *own[i];
+    if (b.ntensors == 0 || fuse[i]) continue;
+    rc = muon_postpass(b.ntensors, b.params, b.p_dtype, nullptr, 0, b.ws, MUON_DT_BF16, b.ws_batch,
+                       steps, b.nb, b.rows, b.cols, b.adjusted_lrs, nullptr, wd, cautious, stream);
+    if (rc != MUON_OK) return rc;
+  }
+  return MUON_OK;
+}
+
+int muon_orth_run_group(int nbuckets, const MuonBucket* buckets, const double* coeffs, int steps,
+                        float prescale, float eps, float wd, int cautious, void* stream) {
+  try {
+    return orth_run_group(nbuckets, buckets, coeffs, steps, prescale, eps, wd, cautious, stream);
+  } catch (const std::bad_alloc&) {
+    muon_set_error("orth_run_group: out of host memory (%d buckets)", nbuckets);
+    return MUON_ERR_ARG;
+  }
 }
 
 int muon_orth_extract(const void* ws, int ws_dtype, int64_t ws_batch, int64_t batch,

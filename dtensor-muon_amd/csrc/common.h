@@ -296,6 +296,18 @@ struct MuonApply {
   int cautious;
 };
 
+// One bucket's share of a product launched over several buckets (muon_launch_products): `batch`
+// matrices of m rows, N columns (a SYRK: m) contracted over K; operands as muon_launch_gemm's.
+struct MuonProduct {
+  const void* a;
+  const void* b;
+  void* out;
+  int64_t lda, sa, ldb, sb, ldo, so;
+  int64_t batch, m, nv, N, K;
+  const float* scale;
+  int t0, nb;  // an apply's first tensor in the launch's table, matrices per tensor
+};
+
 static inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // Thread-local last-error text for muon_amd_last_error().

@@ -4,6 +4,8 @@
 // pre-pass can emit both the stored layout and its transpose (through LDS) in one
 // read of the gradient and momentum, and reduce the Frobenius-norm partials of each
 // tile in a fixed order (deterministic, no atomics).
+#include <algorithm>
+#include <cstring>
 #include <type_traits>
 
 #include "common.h"
@@ -334,15 +336,12 @@ __global__ __launch_bounds__(256) void momentum_kernel(PrepassArgs a, int64_t nu
   }
 }
 
-// scale[b] = 1 / (sqrt(sum of partials) * prescale + eps); one workgroup per matrix,
+// *scale = 1 / (sqrt(sum of partials) * prescale + eps); one workgroup per matrix,
 // fixed-order reduction in double.
-__global__ __launch_bounds__(256) void finalize_scale_kernel(const float* partials,
-                                                             int64_t parts, float* scale,
-                                                             float prescale, float eps) {
+MUON_DEVICE void finalize_scale(const float* p, int64_t parts, float* scale, float prescale,
+                                float eps) {
 #pragma clang fp contract(off)
   __shared__ double red[256];
-  const int64_t b = blockIdx.x;
-  const float* p = partials + b * parts;
   double s = 0.0;
   for (int64_t i = threadIdx.x; i < parts; i += 256) s += (double)p[i];
   red[threadIdx.x] = s;
@@ -355,8 +354,32 @@ __global__ __launch_bounds__(256) void finalize_scale_kernel(const float* partia
     float norm = (float)sqrt(red[0]);
     float denom = norm * prescale;
     denom = denom + eps;
-    scale[b] = 1.0f / denom;
+    *scale = 1.0f / denom;
   }
+}
+
+__global__ __launch_bounds__(256) void finalize_scale_kernel(const float* partials,
+                                                             int64_t parts, float* scale,
+                                                             float prescale, float eps) {
+  const int64_t b = blockIdx.x;
+  finalize_scale(partials + b * parts, parts, scale + b, prescale, eps);
+}
+
+// finalize_scale_kernel over the matrices of several buckets: bucket i's are b0[i] .. b0[i + 1] - 1
+// of the launch.
+constexpr int FINALIZE_MAX = 8;
+struct FinalizeTab {
+  int n, b0[FINALIZE_MAX + 1];
+  const float* partials[FINALIZE_MAX];
+  float* scale[FINALIZE_MAX];
+  int64_t parts[FINALIZE_MAX];
+};
+__global__ __launch_bounds__(256) void finalize_scale_group_kernel(FinalizeTab t, float prescale,
+                                                                   float eps) {
+  int i = 0;
+  while (i + 1 < t.n && (int)blockIdx.x >= t.b0[i + 1]) ++i;
+  const int64_t b = (int)blockIdx.x - t.b0[i];
+  finalize_scale(t.partials[i] + b * t.parts[i], t.parts[i], t.scale[i] + b, prescale, eps);
 }
 
 // x *= scale[b] over the padded stored-layout matrices (steps == 0 path).
@@ -1035,6 +1058,27 @@ int muon_launch_finalize(const OrthLayout& L, void* ws, int64_t batch, float pre
                      (const float*)(w + L.off_part), L.parts, (float*)(w + L.off_scale),
                      prescale, eps);
   MUON_CHECK_LAUNCH("finalize_scale");
+  return MUON_OK;
+}
+
+// muon_launch_finalize for n buckets of batch[i] matrices each.
+int muon_launch_finalize_group(int n, const OrthLayout* L, char* const* ws, const int64_t* batch,
+                               float prescale, float eps, hipStream_t s) {
+  for (int i0 = 0; i0 < n; i0 += FINALIZE_MAX) {
+    FinalizeTab t;
+    memset(&t, 0, sizeof(t));
+    t.n = std::min(FINALIZE_MAX, n - i0);
+    for (int i = 0; i < t.n; ++i) {
+      t.partials[i] = (const float*)(ws[i0 + i] + L[i0 + i].off_part);
+      t.scale[i] = (float*)(ws[i0 + i] + L[i0 + i].off_scale);
+      t.parts[i] = L[i0 + i].parts;
+      t.b0[i + 1] = t.b0[i] + (int)batch[i0 + i];
+    }
+    if (t.b0[t.n] == 0) continue;
+    hipLaunchKernelGGL(finalize_scale_group_kernel, dim3((unsigned)t.b0[t.n]), dim3(256), 0, s, t,
+                       prescale, eps);
+  }
+  MUON_CHECK_LAUNCH("finalize_scale_group");
   return MUON_OK;
 }
 

@@ -3325,3 +3325,121 @@ int muon_launch_gemm_apply(int64_t batch, int64_t M, int64_t N, int64_t K, const
   MUON_CHECK_LAUNCH("gemm_apply");
   return MUON_OK;
 }
+
+// A product of several buckets in launches of up to GROUP_MAX of them, on 128- or 64-row tiles
+// (mode 1: SYRK, 0: B X, with `ap` the apply of parameters of type pdt, tall as
+// muon_launch_gemm_apply's): the same bits as a launch per bucket. One launch per product
+// instead of one per bucket, for buckets so small that the host's launches take longer than the
+// kernels: 16 matrices of four shapes (512 x 512 to 512 x 2048) take 23 / 12 / 24 us for X X^T /
+// A A / B X in one launch each, against four launches of 5 to 17 us for each product.
+int muon_launch_products(int mode, int n, const MuonProduct* items, float alpha, float beta,
+                         int scale_mode, const MuonApply* ap, int pdt, int tall,
+                         hipStream_t stream) {
+  if (reserve_lds() != 0) {
+    muon_set_error("products: cannot reserve LDS");
+    return MUON_ERR_LAUNCH;
+  }
+  if (alpha == 0.0f) {
+    muon_set_error("products: alpha must be nonzero");
+    return MUON_ERR_ARG;
+  }
+  for (int i0 = 0; i0 < n; i0 += GROUP_MAX) {
+    const int cnt = std::min(GROUP_MAX, n - i0);
+    // tile size by the whole launch: its tiles, their K on average and the longest
+    int64_t n128 = 0;
+    double work = 0.0, kmax = 0.0;
+    for (int i = i0; i < i0 + cnt; ++i) {
+      const MuonProduct& p = items[i];
+      const int64_t t = round_up(p.m, 128) / 128;
+      const int64_t tiles = (mode == MODE_SYRK ? t * (t + 1) / 2 : t * (p.N / 128)) * p.batch;
+      if (p.K % 64 || p.N % 128 || p.lda * p.m * 2 >= (int64_t)0x7fffffff ||
+          (mode == MODE_GEMM && p.ldb * p.K * 2 >= (int64_t)0x7fffffff)) {
+        muon_set_error("products: unsupported extents (%lld, %lld, %lld)", (long long)p.m,
+                       (long long)p.N, (long long)p.K);
+        return MUON_ERR_SHAPE;
+      }
+      n128 += tiles;
+      work += (double)tiles * p.K;
+      kmax = std::max(kmax, (double)p.K);
+    }
+    if (n128 == 0) continue;
+    if (n128 > (1 << 24)) {
+      muon_set_error("products: grid too large (%lld tiles)", (long long)n128);
+      return MUON_ERR_SHAPE;
+    }
+    const double kavg = work / (double)n128;
+    const int64_t n64 = 4 * n128;
+    bool t64;
+    if (mode == MODE_SYRK) {
+      const double c128 = n128 <= device_cus() ? 9.0 + 0.0089 * kmax
+                                               : std::max(9.0 + 0.0089 * kmax, 9.0 + per_cu(n128) * (1.7 + 0.0092 * kavg));
+      const double c64 = std::max(5.0 + 0.0037 * kmax, 5.0 + per_cu(n64) * (0.6 + 0.0037 * kavg));
+      t64 = c64 < c128;
+    } else {
+      const double c128 = n128 <= device_cus() ? 5.5 + 0.0122 * kmax
+                                               : 6.0 + per_cu(n128) * (0.8 + 0.0098 * kavg);
+      const double c64 = n64 <= device_cus() ? 4.5 + 0.0078 * kmax
+                                             : 4.5 + per_cu(n64) * (0.5 + 0.0038 * kavg);
+      t64 = c64 < c128;
+    }
+    const int TM = t64 ? 64 : 128;
+    GemmTab tab;
+    memset(&tab, 0, sizeof(tab));
+    tab.n = cnt;
+    for (int i = 0; i < cnt; ++i) {
+      const MuonProduct& p = items[i0 + i];
+      GemmArgs g;
+      memset(&g, 0, sizeof(g));
+      g.a = p.a;
+      g.lda = p.lda;
+      g.sa = p.sa;
+      g.b = mode == MODE_SYRK ? p.a : p.b;
+      g.ldb = mode == MODE_SYRK ? p.lda : p.ldb;
+      g.sb = mode == MODE_SYRK ? p.sa : p.sb;
+      g.out = p.out;
+      g.ldo = p.ldo;
+      g.so = p.so;
+      g.K = p.K;
+      g.Mv = p.m;
+      g.Nv = mode == MODE_SYRK ? p.m : p.nv;
+      g.alpha = alpha;
+      g.beta = beta;
+      g.scale = p.scale;
+      g.scale_mode = scale_mode;
+      g.t0 = p.t0;
+      g.nb = p.nb;
+      tab.g[i] = on_tiles(g, mode, TM, p.m, p.N, p.batch);
+      tab.tile0[i + 1] = tab.tile0[i] + tab.g[i].tiles_total;
+    }
+    const dim3 grid((unsigned)tab.tile0[cnt]), block(256);
+    if (mode == MODE_SYRK) {
+      if (t64)
+        hipLaunchKernelGGL((tile_syrk_kernel<64, GemmTab>), grid, block, TileK<64>::SMEM, stream, tab);
+      else
+        hipLaunchKernelGGL((gemm_bf16_s16h_kernel<GemmTab>), grid, block, H_SMEM, stream, tab);
+    } else {
+      MuonApply none;
+      none.nb = 1;
+      const MuonApply& apv = ap ? *ap : none;
+#define LAUNCH_GROUP(P_, SW_)                                                                     \
+  do {                                                                                            \
+    if (t64)                                                                                      \
+      hipLaunchKernelGGL((tile_bx_kernel<64, P_, SW_, GemmTab>), grid, block, TileK<64>::SMEM,     \
+                         stream, tab, apv);                                                       \
+    else                                                                                          \
+      hipLaunchKernelGGL((tile_bx_kernel<128, P_, SW_, GemmTab>), grid, block, TileK<128>::SMEM,   \
+                         stream, tab, apv);                                                       \
+  } while (0)
+#define LAUNCH_GROUP_P(P_) \
+  do { if (tall) LAUNCH_GROUP(P_, true); else LAUNCH_GROUP(P_, false); } while (0)
+      if (!ap) LAUNCH_GROUP(-1, false);
+      else if (pdt == MUON_DT_BF16) LAUNCH_GROUP_P(MUON_DT_BF16);
+      else if (pdt == MUON_DT_F16) LAUNCH_GROUP_P(MUON_DT_F16);
+      else LAUNCH_GROUP_P(MUON_DT_F32);
+#undef LAUNCH_GROUP_P
+#undef LAUNCH_GROUP
+    }
+  }
+  MUON_CHECK_LAUNCH("products");
+  return MUON_OK;
+}

@@ -65,6 +65,11 @@ _SIGNATURES = {
          _c_f32, _c_f32, _c_int, _pp, _c_int, _c_i64, ctypes.POINTER(_c_f32), _c_f32, _c_int,
          _c_int, _vp],
     ),
+    "muon_orth_run_group": (
+        _c_int,
+        [_c_int, _vp, ctypes.POINTER(ctypes.c_double), _c_int, _c_f32, _c_f32, _c_f32, _c_int,
+         _vp],
+    ),
     "muon_orth_extract": (
         _c_int, [_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_int, _vp]
     ),
@@ -100,6 +105,15 @@ _SIGNATURES = {
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
+
+
+class Bucket(ctypes.Structure):
+    """MuonBucket of the header."""
+
+    _fields_ = [("ws", _vp), ("ws_batch", _c_i64), ("batch", _c_i64), ("rows", _c_i64),
+                ("cols", _c_i64), ("ntensors", _c_int), ("p_dtype", _c_int), ("nb", _c_i64),
+                ("params", _vp), ("adjusted_lrs", _vp)]
+
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -52,6 +52,10 @@ def workspace(device: torch.device, dtype: torch.dtype, batch: int, rows: int, c
     it reads later)."""
     m, n = _padded_extents(dtype, rows, cols)
     key = (device, _lib.stream(device), dtype, m, n)
+    group = _group()
+    if group is not None:  # each bucket of a group holds its workspace until the group has run
+        key = (*key, group.taken.setdefault(key, 0))
+        group.taken[key[:-1]] += 1
     with _ws_lock:
         hit = _ws_cache.get(key)
         if hit is not None and hit[0] >= batch:
@@ -96,6 +100,77 @@ class beside_others:
 
 def _beside() -> int:
     return int(getattr(_neighbours, "on", False))
+
+
+# ---------------------------------------------------------------------------------
+# Groups: the fused steps of several small buckets in common launches. Inside a ``grouped()`` context
+# a fused step runs its pre-pass and leaves its iteration to the end of the context, where all of
+# them run in one library call; what must follow a bucket's iteration (a NorMuon post-pass, the
+# copy back into a non-contiguous tensor) follows then, in order. Per thread.
+
+_grouping = threading.local()
+
+
+def _group():
+    return getattr(_grouping, "group", None)
+
+
+class grouped:
+    """Context collecting the iterations of the fused steps made in it (one device, stream and set
+    of hyperparameters)."""
+
+    def __enter__(self):
+        assert _group() is None
+        self.taken: dict[tuple, int] = {}  # workspaces of one key handed out so far
+        self.calls: list[tuple] = []       # (bucket, kept references, hyperparameters)
+        self.after: list = []
+        _grouping.group = self
+        return self
+
+    def __exit__(self, exc_type, *exc):
+        _grouping.group = None
+        if exc_type is None:
+            self._run()
+
+    def add(self, device, ws, cap, batch, rows, cols, hp, params=None, lrs=None, nb=1) -> None:
+        b = _lib.Bucket(ws.data_ptr(), cap, batch, rows, cols, 0, 0, nb, None, None)
+        kept = [ws]
+        if params is not None:
+            ptrs, adj = _lib.ptr_array(params), _lib.f32_array(lrs)
+            b.ntensors, b.p_dtype = len(params), _lib.dtype_code(params[0].dtype)
+            b.params, b.adjusted_lrs = ctypes.addressof(ptrs), ctypes.addressof(adj)
+            kept += [ptrs, adj, params]
+        self.calls.append((device, b, kept, hp))
+
+    def _run(self) -> None:
+        lib = _lib.load()
+        i = 0
+        while i < len(self.calls):
+            device, _, _, hp = self.calls[i]
+            j = i
+            while j < len(self.calls) and self.calls[j][0] == device and self.calls[j][3] == hp:
+                j += 1
+            buckets = (_lib.Bucket * (j - i))(*[c[1] for c in self.calls[i:j]])
+            coeffs, prescale, eps, wd, cautious = hp
+            _lib.check(
+                lib.muon_orth_run_group(j - i, ctypes.addressof(buckets), _flat_coeffs(coeffs),
+                                        len(coeffs) // 3, prescale, eps, wd, cautious,
+                                        _lib.stream(device)),
+                "muon_orth_run_group",
+            )
+            i = j
+        for fn in self.after:
+            fn()
+
+
+def when_done(fn) -> None:
+    """``fn()`` once the fused steps made so far have been launched: now, or at the end of the group
+    being collected."""
+    group = _group()
+    if group is None:
+        fn()
+    else:
+        group.after.append(fn)
 
 
 # ---------------------------------------------------------------------------------
@@ -337,7 +412,12 @@ def _fused_step_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Tenso
                          ws.data_ptr(), _lib.DT_BF16, cap, s),
         "muon_prepass",
     )
-    if u_scales is None:
+    group = _group()
+    hp = (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd))
+    if group is not None:
+        group.add(device, ws, cap, count * nb, rows, cols, hp,
+                  *((params, lrs, nb) if u_scales is None else ()))
+    elif u_scales is None:
         # the iteration and the apply in one call: the library fuses the apply into the last
         # X' = a X + B X where the shapes allow it, else runs the post-pass after it
         _lib.check(
@@ -348,19 +428,20 @@ def _fused_step_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Tenso
                 int(cautious_wd), _beside(), s),
             "muon_orth_run_apply",
         )
-        return
-    _lib.check(
-        lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                                 _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
-        "muon_orth_run",
-    )
-    _lib.check(
-        lib.muon_postpass(count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype), None,
-                          0, ws.data_ptr(), _lib.DT_BF16, cap, steps, nb, rows, cols,
-                          _lib.f32_array(lrs), _lib.f32_array(u_scales),
-                          float(weight_decay), int(cautious_wd), s),
-        "muon_postpass",
-    )
+    else:
+        _lib.check(
+            lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
+                                     _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
+            "muon_orth_run",
+        )
+    if u_scales is not None:
+        when_done(lambda: _lib.check(
+            lib.muon_postpass(count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype), None,
+                              0, ws.data_ptr(), _lib.DT_BF16, cap, steps, nb, rows, cols,
+                              _lib.f32_array(lrs), _lib.f32_array(u_scales),
+                              float(weight_decay), int(cautious_wd), s),
+            "muon_postpass",
+        ))
 
 
 def fused_step(
@@ -426,12 +507,17 @@ def _fused_normuon_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Te
                          ws.data_ptr(), _lib.DT_BF16, cap, s),
         "muon_prepass",
     )
-    _lib.check(
-        lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                                 _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
-        "muon_orth_run",
-    )
-    _lib.check(
+    group = _group()
+    if group is not None:
+        group.add(device, ws, cap, count * nb, rows, cols,
+                  (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd)))
+    else:
+        _lib.check(
+            lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
+                                     _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
+            "muon_orth_run",
+        )
+    when_done(lambda: _lib.check(
         lib.muon_normuon_postpass(
             count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype),
             _lib.ptr_array(variances), _lib.dtype_code(variances[0].dtype), None, 0,
@@ -440,7 +526,7 @@ def _fused_normuon_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Te
             float(weight_decay), int(cautious_wd), float(beta2), s,
         ),
         "muon_normuon_postpass",
-    )
+    ))
 
 
 def fused_normuon_step(
@@ -547,6 +633,12 @@ def _fused_lp_impl(params: list[Tensor], grads: list[Tensor], codes: list[Tensor
         "muon_lp_prepass",
     )
     # the iteration and the apply (fused into the last B X where the shapes allow)
+    group = _group()
+    if group is not None:
+        group.add(device, ws, cap, count * nb, rows, cols,
+                  (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd)), params,
+                  lrs, nb)
+        return
     _lib.check(
         lib.muon_orth_run_apply_beside(
             ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols, _flat_coeffs(coeffs), steps,

@@ -135,11 +135,11 @@ def muon_step(
                                        split_sizes=split_sizes) for g in gq]
         _ops.postpass(pview, [u.reshape(g.shape) for u, g in zip(us, G.work)], lr_ratios, lr,
                       weight_decay=weight_decay, cautious_wd=cautious_wd, shape=G.work[0].shape)
-    P.writeback()
+    _ops.when_done(P.writeback)
     if batched and nesterov and not maximize:
-        G.writeback()
+        _ops.when_done(G.writeback)
     if B is not None:
-        B.writeback()
+        _ops.when_done(B.writeback)
 
 
 def _fused_split_step(params, grads, bufs, lr_ratios, lr, split_sizes, **kw) -> None:

@@ -76,12 +76,12 @@ def _normuon_step(params, grads, bufs, variances, lr_ratios, *, lr, weight_decay
         _ops.normuon_postpass(pview, [u.reshape(g.shape) for u, g in zip(us, G.work)], V.work,
                               lr_ratios, lr, weight_decay=weight_decay, cautious_wd=cautious_wd,
                               beta2=muon_beta2, split_sizes=split_sizes, shape=G.work[0].shape)
-    P.writeback()
+    _ops.when_done(P.writeback)
     if batched and nesterov and not maximize:
-        G.writeback()
+        _ops.when_done(G.writeback)
     if B is not None:
-        B.writeback()
-    V.writeback()
+        _ops.when_done(B.writeback)
+    _ops.when_done(V.writeback)
 
 
 def _fused_normuon_split_step(params, grads, bufs, variances, lr_ratios, lr, split_sizes,

@@ -23,7 +23,7 @@ from torch.optim.optimizer import (
     _use_grad_for_differentiable,
 )
 
-from muonium_amd._ops import beside_others
+from muonium_amd._ops import beside_others, grouped
 from muonium_amd.orthogonalize import OrthogonalizationStrategy
 from muonium_amd.utils import group_tensors_by_shape, move_tensors_to_device
 from muonium_amd.utils.offload import pipeline_supported, run_offloaded
@@ -157,21 +157,56 @@ def _concurrent_plan(buckets, algorithm: MuonAlgorithm,
     return slots, side + [bi for bi in natural if bi not in slots]
 
 
-def _run_on_streams(slots: dict[int, int], order: list[int], device_of, run) -> None:
+# The most work of a step's buckets that goes in common launches: 128-row tiles of B X times their
+# K, per CU. With less the host's launches bound the step: 16 matrices of four shapes of a small
+# model (512 wide, 1536 per CU) took 0.67-0.74 ms on four streams and 0.40 ms in common launches,
+# eight matrices of three shapes (768 wide, 2160) 0.54 and 0.45 ms. With more the device does,
+# and the streams' 256-row tiles read half the operand bytes: six of 1024 wide (3072) took 0.53
+# and 0.55 ms, two dozen of 768 wide (7776) 0.97 and 1.12 ms.
+_GROUP_WORK_PER_CU = 2400
+
+
+def _grouped_plan(buckets, slots: dict[int, int]) -> bool:
+    """Whether the buckets, all of which `_concurrent_plan` would run side by side, run in common
+    launches instead: so little work that the host takes longer to launch it than the device to
+    run it, on one device and stream."""
+    if len(slots) + 1 != len(buckets):  # (all but one on side streams: every bucket is small)
+        return False
+    work = 0
+    for device, _, grads, _, _ in buckets:
+        rows, cols = grads[0].shape[-2:]
+        if device != buckets[0][0] or min(rows, cols) <= 64:
+            return False
+        tiles_m, tiles_n = -(-min(rows, cols) // 128), 2 * -(-max(rows, cols) // 256)
+        work += math.prod(grads[0].shape[:-2]) * len(grads) * tiles_m * tiles_n * tiles_m * 128
+    cus = torch.cuda.get_device_properties(buckets[0][0]).multi_processor_count
+    return work <= _GROUP_WORK_PER_CU * cus
+
+
+def _run_on_streams(buckets, slots: dict[int, int], order: list[int], run,
+                    whole: bool = True) -> None:
     """``run(i)`` for every i of ``order``; those with a slot on that side stream of their
-    device, forked from the caller's stream at first use and joined back into it at the end."""
+    device, forked from the caller's stream at first use and joined back into it at the end;
+    or all of them on the caller's stream, in common launches (``whole``: no bucket is cut into
+    batches, whose workspaces a group would hold at the same time). The plan's streams are made
+    either way: the gradients of a later step may need them."""
+    sides = {i: _side_stream(buckets[i][0], slot) for i, slot in slots.items()}
+    if slots and whole and _grouped_plan(buckets, slots):
+        with grouped():
+            for i in order:
+                run(i)
+        return
     forked: dict[tuple[torch.device, int], torch.cuda.Stream] = {}
     with beside_others(bool(slots)):
         for i in order:
             if i not in slots:
                 run(i)
                 continue
-            key = (device_of(i), slots[i])
-            side = _side_stream(*key)
+            key = (buckets[i][0], slots[i])
             if key not in forked:
-                _wait(side, torch.cuda.current_stream(key[0]), (*key, 0))
-                forked[key] = side
-            with torch.cuda.stream(side):
+                _wait(sides[i], torch.cuda.current_stream(key[0]), (*key, 0))
+                forked[key] = sides[i]
+            with torch.cuda.stream(sides[i]):
                 run(i)
     for key, side in forked.items():
         _wait(torch.cuda.current_stream(key[0]), side, (*key, 1))
@@ -540,9 +575,8 @@ class Muon(torch.optim.Optimizer):
                          for idx in runs]
                 slots, order = _concurrent_plan(views, algorithm, None)
             else:
-                slots, order = {}, list(range(len(runs)))
-            _run_on_streams(slots, order, lambda ri: params[runs[ri][0]].device,
-                            lambda ri: update(runs[ri]))
+                views, slots, order = [], {}, list(range(len(runs)))
+            _run_on_streams(views, slots, order, lambda ri: update(runs[ri]))
             return
 
         buckets = _group_muon_tensors(params, grads, state, lr_ratios)
@@ -553,7 +587,7 @@ class Muon(torch.optim.Optimizer):
             self._muon_bucket(algorithm, hp, nesterov, maximize, device, dev_p, dev_g,
                               dev_state, dev_lr)
 
-        _run_on_streams(slots, order, lambda bi: buckets[bi][0], bucket)
+        _run_on_streams(buckets, slots, order, bucket, whole=not self.batch_size)
 
     def _muon_bucket(self, algorithm, hp, nesterov, maximize, device, dev_p, dev_g, dev_state,
                      dev_lr) -> None:

@@ -143,6 +143,22 @@ int muon_orth_run_apply_beside(void* ws, int ws_dtype, int64_t ws_batch, int64_t
                                int p_dtype, int64_t nb, const float* adjusted_lrs, float wd,
                                int cautious, int beside, void* stream);
 
+/* The iteration of several buckets (different extents, each with a bf16 workspace of its own whose
+ * pre-pass has run) in common launches, and the apply of the buckets that name parameters
+ * (ntensors > 0): bit for bit what one muon_orth_run (ntensors == 0, U stays in the workspace) or
+ * muon_orth_run_apply per bucket gives. For buckets too small to fill the device: one launch
+ * per product of an iteration instead of one per bucket. */
+typedef struct MuonBucket {
+  void* ws;
+  int64_t ws_batch, batch, rows, cols;
+  int ntensors, p_dtype;
+  int64_t nb;
+  void* const* params;
+  const float* adjusted_lrs;
+} MuonBucket;
+int muon_orth_run_group(int nbuckets, const MuonBucket* buckets, const double* coeffs, int steps,
+                        float prescale, float eps, float wd, int cautious, void* stream);
+
 /* Copy U (first `batch` matrices, stored layout) out of the workspace into a
  * contiguous (batch, rows, cols) tensor of out_dtype. Replaces the return/unbind of
  * orthogonalize.py:101-102, :159-162. */
