@@ -2411,7 +2411,9 @@ MUON_DEVICE void f32_dma(int vo, u32x4 rs, int so, uint32_t m0) {
                : "m0", "memory");
 }
 
-template <int MODE>
+// OWN (SYRK): gram_ of caller-owned tensors with K a multiple of 4: rows past the last read the last
+// one, chunks past a row's end its first one and count as zero, no stores outside the output.
+template <int MODE, bool OWN = false>
 __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
   extern __shared__ __align__(16) uint8_t smem[];
   int bidx, tm, tn;
@@ -2420,29 +2422,38 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
   const int64_t row0 = (int64_t)tm * F_TM, col0 = (int64_t)tn * F_TM;
-  const float* A = (const float*)g.a + (int64_t)bidx * g.sa + row0 * g.lda;
-  const float* B = (const float*)g.b + (int64_t)bidx * g.sb + (MODE == MODE_GEMM ? col0 : col0 * g.ldb);
+  const float* A = (const float*)g.a + (int64_t)bidx * g.sa + (OWN ? 0 : row0 * g.lda);
+  const float* B = (const float*)g.b + (int64_t)bidx * g.sb +
+                   (OWN ? 0 : MODE == MODE_GEMM ? col0 : col0 * g.ldb);
   const u32x4 rsa = n4_rsrc(A, false), rsb = n4_rsrc(B, false), rs_none = n4_rsrc(A, true);
   const int lda_b = (int)(g.lda * 4), ldb_b = (int)(g.ldb * 4);
   // this wave's load of a panel fills 1 KB: 8 rows of 8 chunks (K-contiguous panels), or 4
   // rows k of 16 chunks (X panel)
   const int ra = wave * 8 + (lane >> 3);
-  const int voa = ra * lda_b + (((lane & 7) ^ kswz(ra)) << 4);
+  const int lch = (lane & 7) ^ kswz(ra);
+  const int voa = OWN ? min((int)row0 + ra, (int)g.Mt - 1) * lda_b : ra * lda_b + (lch << 4);
   int vob, kstep_b;
   if constexpr (MODE == MODE_GEMM) {
     const int rk = wave * 4 + (lane >> 4);
     vob = rk * ldb_b + (((lane & 15) ^ (((rk >> 2) & 1) << 3)) << 4);
     kstep_b = F_KT * ldb_b;
   } else {
-    vob = ra * ldb_b + (((lane & 7) ^ kswz(ra)) << 4);
+    vob = OWN ? min((int)col0 + ra, (int)g.Mt - 1) * ldb_b : ra * ldb_b + (lch << 4);
     kstep_b = F_KT * 4;
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  const int KT = (int)(g.K / F_KT);
+  // (OWN: K-tiles up to a pair of them)
+  const int KT = OWN ? (int)((g.Kt + 2 * F_KT - 1) / (2 * F_KT)) * 2 : (int)(g.K / F_KT);
   auto issue = [&](int kt, int st) {
     const bool on = kt < KT;  // past the last K-tile: the null descriptor reads no memory
     const int kk = on ? kt : 0;
     const uint32_t m0 = lds0 + st * F_STAGEB + wave * 1024;
+    if constexpr (OWN) {
+      const int co = kk * F_KT * 4 + lch * 16 < lda_b ? kk * F_KT * 4 + lch * 16 : 0;
+      f32_dma(voa + co, on ? rsa : rs_none, 0, m0);
+      f32_dma(vob + co, on ? rsb : rs_none, 0, m0 + F_PANELB);
+      return;
+    }
     f32_dma(voa, on ? rsa : rs_none, kk * F_KT * 4, m0);
     f32_dma(vob, on ? rsb : rs_none, kk * kstep_b, m0 + F_PANELB);
   };
@@ -2454,7 +2465,7 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
   struct Frags {
     float4 a[2], b[2];  // this group's two groups of 8 k
   };
-  auto load = [&](Frags& f, int st) {
+  auto load = [&](Frags& f, int kt, int st) {
     const uint8_t* pa = smem + st * F_STAGEB + (wm * 32 + fr) * (F_KT * 4);
     const uint8_t* pb = smem + st * F_STAGEB + F_PANELB;
 #pragma unroll
@@ -2468,6 +2479,8 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
       } else {
         f.b[q2] = *(const float4*)(pb + (wn * 32 + fr) * (F_KT * 4) + cpos);
       }
+      if (OWN && kt * F_KT + 8 * q + 4 * fh >= g.Kt)
+        f.a[q2] = f.b[q2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
   };
   auto mma = [&](const Frags& f) {
@@ -2489,13 +2502,13 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
     lds_barrier();
     issue(kt + F_NS - 1, st == 0 ? F_NS - 1 : st - 1);
     st = st + 1 == F_NS ? 0 : st + 1;
-    load(next, st);
+    load(next, kt + 1, st);
     mma(cur);
   };
   Frags f0, f1;
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * (F_NS - 2)) : "memory");
   lds_barrier();
-  load(f0, 0);
+  load(f0, 0, 0);
   for (int kt = 0; kt < KT; kt += 2) {  // (K is a multiple of 64)
     step(kt, f0, f1);
     step(kt + 1, f1, f0);
@@ -2513,7 +2526,7 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
   f32x16 accs[1][1];
 #pragma unroll
   for (int r = 0; r < 16; ++r) accs[0][0][r] = acc[r] + sum[r * 64];
-  epilogue<float, 1, 1, false>(g, MODE, bidx, row0 + wm * 32, col0 + wn * 32, accs, lane,
+  epilogue<float, 1, 1, OWN>(g, MODE, bidx, row0 + wm * 32, col0 + wn * 32, accs, lane,
                                MODE == MODE_SYRK && tm == tn);
 }
 
@@ -2554,7 +2567,11 @@ MUON_DEVICE void tile_dma(int vo, u32x4 rs, int so, uint32_t m0) {
 }
 
 // A = alpha X X^T (K = n) or B = alpha (A A + ratio A): upper-triangle tiles, mirrored.
-template <int TM, typename Args>
+// OWN: gram_ of caller-owned tensors, M and K any (rows a whole number of 16-byte chunks): rows past
+// the last read the last one, the chunks past a row's end its first one and count as zero, and
+// nothing is stored outside the M x M output. Eight matrices of 1000 x 1336 take 27 us, 166 on the
+// register-staged masked kernel with its element loads (fp32, four of them: 84 and 181 us).
+template <int TM, typename Args, bool OWN = false>
 __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
   typedef TileK<TM> C;
   constexpr int F = C::F, WM = TM / 2;
@@ -2567,15 +2584,24 @@ __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
   const int wm = wave >> 1, wn = wave & 1;
   const bool diag = tm == tn;  // one panel serves both operands
   const bf16_t* A = (const bf16_t*)g.a + (int64_t)bidx * g.sa;
-  const u32x4 rsa = n4_rsrc(A + (int64_t)row0 * g.lda, false);
-  const u32x4 rsb = n4_rsrc(A + (int64_t)col0 * g.lda, diag);
+  const u32x4 rsa = n4_rsrc(OWN ? A : A + (int64_t)row0 * g.lda, false);
+  const u32x4 rsb = n4_rsrc(OWN ? A : A + (int64_t)col0 * g.lda, diag);
   const u32x4 rs_none = n4_rsrc(A, true);
   const int lda_b = (int)(g.lda * 2);
   // load q of this wave: rows (4 q + wave) * 8 + lane / 8 of the panel, 16-byte chunk lane % 8
   const int r_in = wave * 8 + (lane >> 3);
-  const int vo = r_in * lda_b + (((lane & 7) ^ kswz(r_in)) << 4);
+  const int lch = (lane & 7) ^ kswz(r_in);
+  const int vo = r_in * lda_b + (lch << 4);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  const int KT = (int)(g.K / V2_BK);
+  const int KT = OWN ? (int)((g.Kt + V2_BK - 1) / V2_BK) : (int)(g.K / V2_BK);
+  int voa[C::LOADS], vob[C::LOADS];  // (OWN) byte offsets of the rows from the matrix
+  if constexpr (OWN) {
+#pragma unroll
+    for (int q = 0; q < C::LOADS; ++q) {
+      voa[q] = min(row0 + q * 32 + r_in, (int)g.Mt - 1) * lda_b;
+      vob[q] = min(col0 + q * 32 + r_in, (int)g.Mt - 1) * lda_b;
+    }
+  }
   auto issue = [&](int kt, int st) {
     const bool on = kt < KT;
     const int kb = on ? kt * V2_ROWB : 0;
@@ -2583,8 +2609,14 @@ __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
     const u32x4 pa = on ? rsa : rs_none, pb = on ? rsb : rs_none;
 #pragma unroll
     for (int q = 0; q < C::LOADS; ++q) {
-      tile_dma(vo, pa, kb + q * 32 * lda_b, m0 + q * 4096);
-      tile_dma(vo, pb, kb + q * 32 * lda_b, m0 + C::PANELB + q * 4096);
+      if constexpr (OWN) {
+        const int co = kb + lch * 16 < lda_b ? kb + lch * 16 : 0;
+        tile_dma(voa[q] + co, pa, 0, m0 + q * 4096);
+        tile_dma(vob[q] + co, pb, 0, m0 + C::PANELB + q * 4096);
+      } else {
+        tile_dma(vo, pa, kb + q * 32 * lda_b, m0 + q * 4096);
+        tile_dma(vo, pb, kb + q * 32 * lda_b, m0 + C::PANELB + q * 4096);
+      }
     }
   };
   float alpha = g.alpha, beta = g.beta;
@@ -2623,6 +2655,14 @@ __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
         a[ks][f] = __builtin_bit_cast(bf16x8_mfma, *(const uint4*)(sp + abase + f * 16 * V2_ROWB + off));
         b[ks][f] = __builtin_bit_cast(bf16x8_mfma, *(const uint4*)(sp + bbase + f * 16 * V2_ROWB + off));
       }
+    }
+    if (OWN && (kt + 1) * V2_BK > g.Kt) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        if (kt * V2_BK + ks * 32 + fg * 8 >= g.Kt) {
+#pragma unroll
+          for (int f = 0; f < F; ++f) a[ks][f] = b[ks][f] = __builtin_bit_cast(bf16x8_mfma, u32x4{0, 0, 0, 0});
+        }
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -2672,6 +2712,19 @@ __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
         hv[i][j][h] = w & ((c < mv && r < mv ? 0x0000ffffu : 0u) | (c < mv && r + 1 < mv ? 0xffff0000u : 0u));
       }
   constexpr int CH = TM / 8, ROWS = 256 / CH;  // 16-byte chunks per row, rows per store
+  // eight elements of output row r from column c on (OWN: those inside it)
+  const bool whole = !OWN || (g.ldo % 8 == 0 && !((uintptr_t)g.out & 15));
+  auto put = [&](int r, int c, uint4 w) {
+    bf16_t* o = out + (int64_t)r * g.ldo + c;
+    if (!OWN || (whole && r < mv && c + 8 <= mv)) {
+      *(uint4*)o = w;
+    } else if (r < mv) {
+      const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (c + e < mv) o[e] = (bf16_t)(u[e >> 1] >> (16 * (e & 1)));
+    }
+  };
 #pragma unroll
   for (int i = 0; i < F; ++i)
 #pragma unroll
@@ -2683,7 +2736,7 @@ __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
 #pragma unroll
     for (int it = 0; it < TM / ROWS; ++it) {
       const int jl = it * ROWS + tid / CH, c = tid % CH * 8;
-      *(uint4*)(out + (int64_t)(col0 + jl) * g.ldo + row0 + c) = *(const uint4*)(T + jl * C::PITCH + c);
+      put(col0 + jl, row0 + c, *(const uint4*)(T + jl * C::PITCH + c));
     }
     lds_barrier();
 #pragma unroll
@@ -2711,7 +2764,7 @@ __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
         e[q] = c + q > il ? T[(c + q) * C::PITCH + il] : T[il * C::PITCH + c + q];
       __builtin_memcpy(&w, e, 16);
     }
-    *(uint4*)(out + (int64_t)(row0 + il) * g.ldo + col0 + c) = w;
+    put(row0 + il, col0 + c, w);
   }
 }
 
@@ -2948,8 +3001,9 @@ int reserve_lds() {
       if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, N4_SMEM) !=
           hipSuccess)
         status = -1;
-    const void* f32[2] = {(const void*)gemm_f32_kernel<MODE_SYRK>,
-                          (const void*)gemm_f32_kernel<MODE_GEMM>};
+    const void* f32[3] = {(const void*)gemm_f32_kernel<MODE_SYRK>,
+                          (const void*)gemm_f32_kernel<MODE_GEMM>,
+                          (const void*)gemm_f32_kernel<MODE_SYRK, true>};
     for (const void* k : f32)
       if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, F_SMEM) !=
           hipSuccess)
@@ -3181,13 +3235,42 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
         // full tiles only: the 16 x 16 x 32 MFMA kernel
         hipLaunchKernelGGL(gemm_bf16_s16_kernel, grid, dim3(512), V2_SMEM, stream, g);
       }
+    } else if (masked && K % 8 == 0 && !((uintptr_t)a & 15)) {
+      // gram_ of any extents, rows of whole 16-byte chunks
+      const int TM = syrk_tile(batch, M, K, blocks, 0) == 64 ? 64 : 128;
+      GemmArgs gt = g;
+      gt.tiles_m = gt.tiles_n = (int)((M + TM - 1) / TM);
+      gt.tiles_per_batch = gt.tiles_m * (gt.tiles_m + 1) / 2;
+      const int64_t bt = (int64_t)gt.tiles_per_batch * batch;
+      if (bt > 0x7fffffffLL) {
+        muon_set_error("gemm: grid too large (%lld workgroups)", (long long)bt);
+        return MUON_ERR_SHAPE;
+      }
+      gt.tiles_total = (int)bt;
+      if (TM == 64)
+        hipLaunchKernelGGL((tile_syrk_kernel<64, GemmArgs, true>), dim3((unsigned)bt), dim3(256),
+                           TileK<64>::SMEM, stream, gt);
+      else
+        hipLaunchKernelGGL((tile_syrk_kernel<128, GemmArgs, true>), dim3((unsigned)bt), dim3(256),
+                           TileK<128>::SMEM, stream, gt);
     } else {
       if (masked) LAUNCH_BF(MODE_SYRK, true); else LAUNCH_BF(MODE_SYRK, false);
     }
 #undef LAUNCH_BF
   } else if (dtype == MUON_DT_F32) {
-    if (masked) {
+    if (masked && (K % 4 || ((uintptr_t)a & 15))) {
       hipLaunchKernelGGL(gemm_f32_masked_kernel, grid, block, 0, stream, g);
+    } else if (masked) {
+      GemmArgs gh = g;
+      gh.tiles_m = gh.tiles_n = (int)((M + F_TM - 1) / F_TM);
+      gh.tiles_per_batch = gh.tiles_m * (gh.tiles_m + 1) / 2;
+      const int64_t bh = (int64_t)gh.tiles_per_batch * batch;
+      if (bh > 0x7fffffffLL) {
+        muon_set_error("gemm: grid too large (%lld workgroups)", (long long)bh);
+        return MUON_ERR_SHAPE;
+      }
+      hipLaunchKernelGGL((gemm_f32_kernel<MODE_SYRK, true>), dim3((unsigned)bh), dim3(512), F_SMEM,
+                         stream, gh);
     } else {
       GemmArgs gh = g;  // 64-row tiles
       gh.tiles_m = (int)(M / F_TM);

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from helpers import rel_fro
-from muonium_amd.kernels.gram import gram
+from muonium_amd.kernels.gram import gram, gram_
 from muonium_amd.orthogonalize.newton_schulz import ns_loop
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +48,37 @@ def test_fp32_batch_equals_members():
     U = ns_loop(X, 5)
     for i in (0, 33, 69):
         assert torch.equal(U[i], ns_loop(X[i:i + 1], 5)[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B, M, K", [
+    (1, 1, 8), (2, 7, 16), (1, 63, 72), (3, 64, 64), (2, 65, 128), (1, 130, 1336), (4, 100, 40),
+    (1, 1000, 8), (40, 200, 136), (2, 1001, 264), (3, 17, 12), (3, 130, 70), (2, 33, 7)])
+def test_gram_of_any_extents(B, M, K, dtype):
+    """Tiles with partial rows, columns and K (whole 16-byte chunks per row, and rows that are not:
+    the element-load kernel), the output between canaries. bf16: one rounding of the fp32 sum."""
+    x = torch.randn(B, M, K, generator=torch.Generator().manual_seed(M * K)).to(dtype).cuda()
+    n = B * M * M
+    store = torch.full((n + 128,), 7.0, dtype=dtype, device="cuda")
+    y = store[64:64 + n].view(B, M, M)
+    gram_(x, y)
+    assert (store[:64] == 7).all() and (store[64 + n:] == 7).all()
+    assert torch.equal(y, y.mT)
+    xd = x.double()
+    exact, mag = xd @ xd.mT, xd.abs() @ xd.abs().mT
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    assert ((y.double() - exact).abs() <= ulp * exact.abs() + K * 2.0 ** -23 * mag).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gram_reads_nothing_past_its_rows(dtype):
+    """NaN right before and after the input, and in the rows' neighbours, stay out of the sums."""
+    B, M, K = 2, 70, 104
+    store = torch.full((B * M * K + 512,), float("nan"), dtype=dtype, device="cuda")
+    x = store[256:256 + B * M * K].view(B, M, K)
+    x.copy_(torch.randn(B, M, K, device="cuda"))
+    x[0, 3] = float("nan")
+    y = gram(x)
+    keep = torch.arange(M, device="cuda") != 3
+    assert y[1].isfinite().all() and y[0][keep][:, keep].isfinite().all()
+    assert y[0, 3].isnan().all()
