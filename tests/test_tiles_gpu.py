@@ -66,3 +66,15 @@ def test_update_matches_64_bits_at_tile_edges(shape, strategy):
     exact = muon_ref.polar_iteration(X.double(), coeffs, prescale=prescale, eps=1e-7)
     got = zeropower(X.to(DEV), strategy=strategy).cpu()
     assert rel_fro(got, exact) <= 1.25 * rel_fro(ref, exact) + 2e-3
+
+
+@pytest.mark.parametrize("m, n, count", [(2048, 2048, 8), (2048, 2304, 15), (1536, 4352, 13),
+                                         (4000, 4096, 2)])
+def test_gram_tail_in_small_tiles_has_the_same_bits(m, n, count):
+    """Launches of a little more than whole rounds of 256-row tiles (288, 540, 273 and 272 tiles on
+    256 compute units): the tiles left over are cut into small ones; each matrix as alone."""
+    gen = torch.Generator(device=DEV).manual_seed(m + n)
+    X = torch.randn(count, m, n, generator=gen, device=DEV).bfloat16()
+    U = zeropower(X, strategy="newton_schulz", steps=2)
+    for i in (0, count // 2, count - 1):
+        assert torch.equal(U[i], zeropower(X[i:i + 1], strategy="newton_schulz", steps=2)[0]), i
