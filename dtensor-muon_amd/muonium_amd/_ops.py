@@ -52,6 +52,9 @@ def workspace(device: torch.device, dtype: torch.dtype, batch: int, rows: int, c
     it reads later)."""
     m, n = _padded_extents(dtype, rows, cols)
     key = (device, _lib.stream(device), dtype, m, n)
+    owner = getattr(_neighbours, "owner", None)
+    if owner is not None:
+        key = (*key, ("thread", owner))
     group = _group()
     if group is not None:  # each bucket of a group holds its workspace until the group has run
         key = (*key, group.taken.setdefault(key, 0))
@@ -82,6 +85,27 @@ def release_workspaces() -> None:
 # weighs what a launch takes from its neighbours (the results are the same). Per thread.
 
 _neighbours = threading.local()
+
+
+class own_workspaces:
+    """Context of calls on a side stream of this thread: torch hands out a fixed set of streams, so
+    another thread's may be the same one, and two threads' launches on one stream interleave. The
+    calls take workspaces of this thread's own."""
+
+    def __enter__(self):
+        self.before = getattr(_neighbours, "owner", None)
+        _neighbours.owner = threading.get_ident()
+
+    def __exit__(self, *exc):
+        _neighbours.owner = self.before
+
+
+def release_workspaces_except(live: set[int]) -> None:
+    """Drop the side streams' workspaces of threads not among ``live``."""
+    with _ws_lock:
+        for key in list(_ws_cache):
+            if isinstance(key[-1], tuple) and key[-1][1] not in live:
+                del _ws_cache[key]
 
 
 class beside_others:
@@ -127,10 +151,9 @@ class grouped:
         _grouping.group = self
         return self
 
-    def __exit__(self, exc_type, *exc):
+    def __exit__(self, *exc):
         _grouping.group = None
-        if exc_type is None:
-            self._run()
+        self._run()  # (after an error too: the buckets before it are stepped, as one by one)
 
     def add(self, device, ws, cap, batch, rows, cols, hp, params=None, lrs=None, nb=1) -> None:
         b = _lib.Bucket(ws.data_ptr(), cap, batch, rows, cols, 0, 0, nb, None, None)

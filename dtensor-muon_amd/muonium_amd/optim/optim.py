@@ -23,7 +23,7 @@ from torch.optim.optimizer import (
     _use_grad_for_differentiable,
 )
 
-from muonium_amd._ops import beside_others, grouped
+from muonium_amd._ops import beside_others, grouped, own_workspaces, release_workspaces_except
 from muonium_amd.orthogonalize import OrthogonalizationStrategy
 from muonium_amd.utils import group_tensors_by_shape, move_tensors_to_device
 from muonium_amd.utils.offload import pipeline_supported, run_offloaded
@@ -86,8 +86,8 @@ def _per_tensor_runs(algorithm: MuonAlgorithm, params, grads, state, split_sizes
 # fourth side stream shared a queue with the third, which serialized their buckets)
 _MAX_SIDE_STREAMS = 3
 # Side streams, and the events of their forks and joins, each of one thread (its identifier is part
-# of the key): workspaces are cached by stream, so threads stepping at the same time must not
-# share a side stream, nor an event between one's record and its wait.
+# of the key): threads stepping at the same time must not share workspaces, nor an event between
+# one's record and its wait. Those of threads that have ended go when another makes its own.
 _side_streams: dict[tuple[int, int, int], torch.cuda.Stream] = {}
 
 
@@ -97,6 +97,11 @@ def _side_stream(device: torch.device, slot: int) -> torch.cuda.Stream:
     key = (threading.get_ident(), index, slot)
     stream = _side_streams.get(key)
     if stream is None:
+        live = {t.ident for t in threading.enumerate()} | {key[0]}
+        for made in (_side_streams, _sync_events):
+            for old in [k for k in list(made) if k[0] not in live]:
+                made.pop(old, None)
+        release_workspaces_except(live)
         stream = _side_streams[key] = torch.cuda.Stream(device=index)
     return stream
 
@@ -183,6 +188,20 @@ def _grouped_plan(buckets, slots: dict[int, int]) -> bool:
     return work <= _GROUP_WORK_PER_CU * cus
 
 
+def _share_memory(params) -> bool:
+    """Whether the address ranges of two of the tensors meet: a weight that is also a view of
+    another, whose updates must follow each other."""
+    end = 0
+    for lo, hi in sorted(
+            (p.data_ptr(), p.data_ptr() + p.element_size() *
+             (1 + sum((n - 1) * st for n, st in zip(p.shape, p.stride()))))
+            for p in params if type(p) in (Tensor, torch.nn.Parameter) and p.numel()):
+        if lo < end:
+            return True
+        end = hi
+    return False
+
+
 def _run_on_streams(buckets, slots: dict[int, int], order: list[int], run,
                     whole: bool = True) -> None:
     """``run(i)`` for every i of ``order``; those with a slot on that side stream of their
@@ -197,19 +216,21 @@ def _run_on_streams(buckets, slots: dict[int, int], order: list[int], run,
                 run(i)
         return
     forked: dict[tuple[torch.device, int], torch.cuda.Stream] = {}
-    with beside_others(bool(slots)):
-        for i in order:
-            if i not in slots:
-                run(i)
-                continue
-            key = (buckets[i][0], slots[i])
-            if key not in forked:
-                _wait(sides[i], torch.cuda.current_stream(key[0]), (*key, 0))
-                forked[key] = sides[i]
-            with torch.cuda.stream(sides[i]):
-                run(i)
-    for key, side in forked.items():
-        _wait(torch.cuda.current_stream(key[0]), side, (*key, 1))
+    try:
+        with beside_others(bool(slots)):
+            for i in order:
+                if i not in slots:
+                    run(i)
+                    continue
+                key = (buckets[i][0], slots[i])
+                if key not in forked:
+                    _wait(sides[i], torch.cuda.current_stream(key[0]), (*key, 0))
+                    forked[key] = sides[i]
+                with torch.cuda.stream(sides[i]), own_workspaces():
+                    run(i)
+    finally:  # (after an error too: what was launched is ordered before the caller's next work)
+        for key, side in forked.items():
+            _wait(torch.cuda.current_stream(key[0]), side, (*key, 1))
 
 
 class Muon(torch.optim.Optimizer):
@@ -574,6 +595,8 @@ class Muon(torch.optim.Optimizer):
                 views = [(params[idx[0]].device, None, [grads[i] for i in idx], None, None)
                          for idx in runs]
                 slots, order = _concurrent_plan(views, algorithm, None)
+                if slots and _share_memory(params):
+                    slots, order = {}, list(range(len(runs)))
             else:
                 views, slots, order = [], {}, list(range(len(runs)))
             _run_on_streams(views, slots, order, lambda ri: update(runs[ri]))
