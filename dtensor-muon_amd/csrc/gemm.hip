@@ -3087,7 +3087,11 @@ static int64_t rounds_of(int64_t blocks) { return (blocks + device_cus() - 1) / 
 // CUs idle for a round, cut into tm-row tiles in a second launch. Eight matrices of 4096 rows
 // are 4.25 rounds, four 2.125, two 1.06: the Gram launches of a step on four layers of a 4096-wide
 // model (28 matrices) went from 23.7 to 21.0 ms, the step from 51.7 to 50.1 ms, on one layer from
-// 13.5 to 12.5 ms. Launches of whole rounds (64 such matrices) keep one launch.
+// 13.5 to 12.5 ms; X X^T of 20 x 1280 x 5120 221 -> 202 us, of 8 x 2048 x 8192 321 -> 282.
+// Launches of whole rounds (64 such matrices) keep one launch, and so does K below 4096, where the
+// second launch's fill and drain take what the round saves (16 x 2048 x 2048: 152 us in one, 164
+// in two; 32 x 1024 x 1024 51 and 62; 100 x 512 x 2048 82 and 107), and a launch that 128-row tiles
+// fill evenly (30 x 1024 x 4096: 166 and 170; c128 is a fifth above the measured there, hence 0.78).
 struct SyrkPlan {
   int tm;
   int64_t head;
@@ -3106,10 +3110,10 @@ static SyrkPlan syrk_plan(int64_t batch, int64_t m, int64_t K, int64_t blocks256
   if (c64 < (beside ? 0.75 : 1.0) * c128 && c64 < c256) best.tm = 64;
   else if (c128 < c256) best.tm = 128;
   const int64_t head = blocks256 / cus * cus, rest = blocks256 - head;
-  if (!packed && head > 0 && rest > 0) {
+  if (!packed && head > 0 && rest > 0 && K >= 4096) {
     const double r128 = c128_of(4 * rest), r64 = c64_of(16 * rest);
     const double split = (double)(head / cus) * round + 4.0 + std::min(r128, r64);
-    if (split < 0.97 * (best.tm == 64 ? c64 : best.tm == 128 ? c128 : c256))
+    if (split < (best.tm == 64 ? 0.97 * c64 : best.tm == 128 ? 0.78 * c128 : 0.97 * c256))
       best = {r64 < r128 ? 64 : 128, head};
   }
   return best;
