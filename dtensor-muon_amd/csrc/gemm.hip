@@ -1359,6 +1359,7 @@ MUON_DEVICE void n16_beta_third(float ratio, int lane, bf16x8_mfma (&db)[2][2]) 
   M(P##0, x0, B) M(P##1, x1, B) M(P##2, x2, B) M(P##3, x3, B)                                 \
   M(P##4, x4, B) M(P##5, x5, B) M(P##6, x6, B) M(P##7, x7, B)
 #define NB_ALL(M) NB_ROW(M, a, FI, d0h) NB_ROW(M, b, FI + 1, d1h) NB_ROW(M, a, FI, d0l) NB_ROW(M, b, FI + 1, d1l)
+#define NB_HI(M) NB_ROW(M, a, FI, d0h) NB_ROW(M, b, FI + 1, d1h)
 #define NB_OUT                                                                               \
   [a0] "+a"(acc[FI][0]), [a1] "+a"(acc[FI][1]), [a2] "+a"(acc[FI][2]), [a3] "+a"(acc[FI][3]),   \
   [a4] "+a"(acc[FI][4]), [a5] "+a"(acc[FI][5]), [a6] "+a"(acc[FI][6]), [a7] "+a"(acc[FI][7]),   \
@@ -1371,16 +1372,22 @@ MUON_DEVICE void n16_beta_third(float ratio, int lane, bf16x8_mfma (&db)[2][2]) 
   [d1h] "v"(db[1][0]), [d1l] "v"(db[1][1])
 // ratio * X added to row blocks FI and FI + 1 (rows 32 ks .. 32 ks + 31 of the K-tile whose
 // X fragments cx are the substep's): 32 MFMAs, the hi parts of both row blocks first. The
-// diagonal fragment serves as srcA as well (SW): its per-lane layout is the same.
-template <int FI, bool SW = false>
+// diagonal fragment serves as srcA as well (SW): its per-lane layout is the same. HI: db holds one
+// part only (n16_beta_third), 16 MFMAs.
+template <int FI, bool SW = false, bool HI = false>
 MUON_DEVICE void n16_beta(f32x4 (&acc)[8][8], const bf16x8_mfma (&cx)[8],
                           const bf16x8_mfma (&db)[2][2]) {
-  if constexpr (SW)
+  if constexpr (HI && SW)
+    asm volatile(NB_HI(M16S) : NB_OUT : NB_IN);
+  else if constexpr (HI)
+    asm volatile(NB_HI(M16) : NB_OUT : NB_IN);
+  else if constexpr (SW)
     asm volatile(NB_ALL(M16S) : NB_OUT : NB_IN);
   else
     asm volatile(NB_ALL(M16) : NB_OUT : NB_IN);
 }
 #undef NB_ALL
+#undef NB_HI
 #undef NB_OUT
 #undef NB_IN
 #undef M16S
@@ -1517,7 +1524,7 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_nn16_kernel(GemmArgs g, Muon
         n16_beta<FB, SW>(acc, x0, db);
         if constexpr (B3) {
           n16_beta_third(ratio, lane, db);
-          n16_beta<FB, SW>(acc, x0, db);
+          n16_beta<FB, SW, true>(acc, x0, db);
         }
       }
       n16_join(x1, xl, xh);
@@ -1536,7 +1543,7 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_nn16_kernel(GemmArgs g, Muon
         n16_beta<FB + 2, SW>(acc, x1, db);
         if constexpr (B3) {
           n16_beta_third(ratio, lane, db);
-          n16_beta<FB + 2, SW>(acc, x1, db);
+          n16_beta<FB + 2, SW, true>(acc, x1, db);
         }
       }
       n16_join(x0, xl, xh);
