@@ -1373,7 +1373,8 @@ MUON_DEVICE void n16_beta_third(float ratio, int lane, bf16x8_mfma (&db)[2][2]) 
 // ratio * X added to row blocks FI and FI + 1 (rows 32 ks .. 32 ks + 31 of the K-tile whose
 // X fragments cx are the substep's): 32 MFMAs, the hi parts of both row blocks first. The
 // diagonal fragment serves as srcA as well (SW): its per-lane layout is the same. HI: db holds one
-// part only (n16_beta_third), 16 MFMAs.
+// part only (n16_beta_third), 16 MFMAs (B X of 100 x 512 x 2048 164 -> 156 us against 32 with a
+// zero part).
 template <int FI, bool SW = false, bool HI = false>
 MUON_DEVICE void n16_beta(f32x4 (&acc)[8][8], const bf16x8_mfma (&cx)[8],
                           const bf16x8_mfma (&db)[2][2]) {
