@@ -1557,7 +1557,7 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_nn16_kernel(GemmArgs g, Muon
     // Leaving a loop that the peeled beta K-tiles follow, the compiler may copy accumulators
     // between registers before any asm that follows the loop; it does not see the MFMAs in
     // the asm, so the last K-tile of such a loop ends with their latency.
-    if constexpr (APPLY == 0) {
+    if constexpr (APPLY == 0 && !B3) {
       // K-tile 0 peeled off every loop, so the loops carry no test for it (B X 1.6% faster on
       // the Llama set than with the test in the loops)
       int kt;
@@ -1580,7 +1580,10 @@ __global__ __launch_bounds__(256, 1) void gemm_bf16_nn16_kernel(GemmArgs g, Muon
       for (; kt < KT; ++kt) kstep(kt, no_beta{}, later);
     } else {
       // the apply kernels test for K-tile 0 in the loops: peeled, their larger epilogue spilled
-      // (their launches took 7% longer on the MoE experts)
+      // (their launches took 7% longer on the MoE experts), and so do those with the three-part
+      // beta term, whose peeled K-tiles hold 64 more MFMAs each (80 bytes of scratch a lane and
+      // 154 scalar registers spilled: 100 x 512 x 2048 154 -> 143 us, 200 x 640 x 640 223 -> 196,
+      // 300 x 256 x 3072 235 -> 208)
       int kt = 0;
       if (kd0 >= 0) {
         for (; kt < kd0; ++kt) {
