@@ -8,11 +8,13 @@ whole bucket.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 import threading
 
 import numpy as np
-from typing import Optional, Sequence
+from typing import NamedTuple, Optional, Sequence
 
 import torch
 from torch import Tensor
@@ -20,17 +22,22 @@ from torch import Tensor
 from . import _lib
 
 # ---------------------------------------------------------------------------------
-# workspace cache: one growable buffer per (device, stream, iteration dtype, padded m, n)
+# workspaces: kept per (device, stream, iteration dtype, padded m, n), each with one call at a time
 #
-# A buffer is only ever used on the stream that allocated it. Buckets running on
-# different streams (the foreach driver's side streams) therefore never share one,
-# and a capacity regrow frees the old buffer on the only stream that used it, which
-# the caching allocator orders behind that stream's earlier launches.
+# A call takes a buffer out of the cache and puts it back when its last launch has been
+# enqueued (a call in a group: when the group has run). A buffer is only ever used on the stream
+# that allocated it, so whoever takes it next is ordered behind those launches; and while a call
+# has it, no other does, also where two threads step on one stream and their launches interleave
+# (a library call releases the interpreter lock between a pre-pass and its iteration). The cache
+# holds as many buffers of a key as calls have had one at the same time. A regrow frees the old
+# buffer on the only stream that used it, which the caching allocator orders behind that stream's
+# earlier launches.
 
 _ws_lock = threading.Lock()
-_ws_cache: dict[tuple, tuple[int, Tensor]] = {}
+_ws_cache: dict[tuple, list[Workspace]] = {}
 
 
+@functools.lru_cache(maxsize=1024)
 def _padded_extents(dtype: torch.dtype, rows: int, cols: int) -> tuple[int, int]:
     """(m_pad, n_pad) of the library's workspace layout for one rows x cols matrix."""
     off, pitch, mst, trans = (ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64(),
@@ -43,8 +50,31 @@ def _padded_extents(dtype: torch.dtype, rows: int, cols: int) -> tuple[int, int]
     return mst.value // pitch.value, pitch.value
 
 
+class Workspace(NamedTuple):
+    """A buffer taken out of the cache; leaving its context puts it back."""
+
+    buf: Tensor
+    capacity: int
+    key: tuple
+
+    def __enter__(self):
+        return self.buf, self.capacity
+
+    def __exit__(self, *exc):
+        group = _group()
+        if group is not None:
+            group.taken.append(self)
+        else:
+            self.give_back()
+
+    def give_back(self) -> None:
+        with _ws_lock:
+            _ws_cache.setdefault(self.key, []).append(self)
+
+
 def workspace(device: torch.device, dtype: torch.dtype, batch: int, rows: int, cols: int):
-    """(buffer, capacity) with room for ``batch`` matrices of rows x cols.
+    """A buffer with room for ``batch`` matrices of rows x cols, as a context of the launches that
+    use it: ``with workspace(...) as (buffer, capacity)``.
 
     The layout only depends on the padded (min, max) extents and the capacity, so
     tall and wide matrices of the same extents share a buffer, on the current stream
@@ -52,26 +82,19 @@ def workspace(device: torch.device, dtype: torch.dtype, batch: int, rows: int, c
     it reads later)."""
     m, n = _padded_extents(dtype, rows, cols)
     key = (device, _lib.stream(device), dtype, m, n)
-    owner = getattr(_neighbours, "owner", None)
-    if owner is not None:
-        key = (*key, ("thread", owner))
-    group = _group()
-    if group is not None:  # each bucket of a group holds its workspace until the group has run
-        key = (*key, group.taken.setdefault(key, 0))
-        group.taken[key[:-1]] += 1
     with _ws_lock:
-        hit = _ws_cache.get(key)
-        if hit is not None and hit[0] >= batch:
-            return hit[1], hit[0]
-        nbytes = _lib.load().muon_orth_workspace_bytes(_lib.dtype_code(dtype), batch, rows, cols)
-        if nbytes < 0:
-            raise RuntimeError(f"muonium_amd: bad workspace request {batch}x{rows}x{cols}")
-        if hit is not None:
-            del _ws_cache[key]
-            del hit
-        buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        _ws_cache[key] = (batch, buf)
-        return buf, batch
+        free = _ws_cache.get(key)
+        if free:  # the smallest that is large enough, else the largest goes to make room
+            if len(free) > 1:
+                free.sort(key=lambda ws: ws.capacity)
+            ws = free.pop(next((i for i, w in enumerate(free) if w.capacity >= batch), -1))
+            if ws.capacity >= batch:
+                return ws
+            del ws
+    nbytes = _lib.load().muon_orth_workspace_bytes(_lib.dtype_code(dtype), batch, rows, cols)
+    if nbytes < 0:
+        raise RuntimeError(f"muonium_amd: bad workspace request {batch}x{rows}x{cols}")
+    return Workspace(torch.empty(nbytes, dtype=torch.uint8, device=device), batch, key)
 
 
 def release_workspaces() -> None:
@@ -85,27 +108,8 @@ def release_workspaces() -> None:
 # weighs what a launch takes from its neighbours (the results are the same). Per thread.
 
 _neighbours = threading.local()
-
-
-class own_workspaces:
-    """Context of calls on a side stream of this thread: torch hands out a fixed set of streams, so
-    another thread's may be the same one, and two threads' launches on one stream interleave. The
-    calls take workspaces of this thread's own."""
-
-    def __enter__(self):
-        self.before = getattr(_neighbours, "owner", None)
-        _neighbours.owner = threading.get_ident()
-
-    def __exit__(self, *exc):
-        _neighbours.owner = self.before
-
-
-def release_workspaces_except(live: set[int]) -> None:
-    """Drop the side streams' workspaces of threads not among ``live``."""
-    with _ws_lock:
-        for key in list(_ws_cache):
-            if isinstance(key[-1], tuple) and key[-1][1] not in live:
-                del _ws_cache[key]
+#: every call has its workspace to itself, on any stream
+own_workspaces = contextlib.nullcontext
 
 
 class beside_others:
@@ -145,7 +149,7 @@ class grouped:
 
     def __enter__(self):
         assert _group() is None
-        self.taken: dict[tuple, int] = {}  # workspaces of one key handed out so far
+        self.taken: list[Workspace] = []   # each bucket's, until the group has run
         self.calls: list[tuple] = []       # (bucket, kept references, hyperparameters)
         self.after: list = []
         _grouping.group = self
@@ -153,7 +157,11 @@ class grouped:
 
     def __exit__(self, *exc):
         _grouping.group = None
-        self._run()  # (after an error too: the buckets before it are stepped, as one by one)
+        try:
+            self._run()  # (after an error too: the buckets before it are stepped, as one by one)
+        finally:
+            for ws in self.taken:
+                ws.give_back()
 
     def add(self, device, ws, cap, batch, rows, cols, hp, params=None, lrs=None, nb=1) -> None:
         b = _lib.Bucket(ws.data_ptr(), cap, batch, rows, cols, 0, 0, nb, None, None)
@@ -293,27 +301,27 @@ def _orthogonalize_impl(tensors: list[Tensor], coeffs: list[float], prescale: fl
     out = torch.empty((count, *t0.shape), dtype=out_dtype, device=device)
     if out.numel() == 0:
         return out
-    ws, cap = workspace(device, iter_dtype, count * nb, rows, cols)
-    wdt = _lib.dtype_code(iter_dtype)
-    s = _lib.stream(device)
-    steps = len(coeffs) // 3
-    grads = _lib.ptr_array(tensors)
-    _lib.check(
-        lib.muon_prepass(count, grads, None, _lib.dtype_code(t0.dtype), 0, nb, rows, cols, 0.0,
-                         0, 0, 0, ws.data_ptr(), wdt, cap, s),
-        "muon_prepass",
-    )
-    _lib.check(
-        lib.muon_orth_run(ws.data_ptr(), wdt, cap, count * nb, rows, cols, _flat_coeffs(coeffs),
-                          steps, prescale, eps, s),
-        "muon_orth_run",
-    )
-    _lib.check(
-        lib.muon_orth_extract(ws.data_ptr(), wdt, cap, count * nb, rows, cols, steps,
-                              out.data_ptr(), _lib.dtype_code(out_dtype), s),
-        "muon_orth_extract",
-    )
-    return out
+    with workspace(device, iter_dtype, count * nb, rows, cols) as (ws, cap):
+        wdt = _lib.dtype_code(iter_dtype)
+        s = _lib.stream(device)
+        steps = len(coeffs) // 3
+        grads = _lib.ptr_array(tensors)
+        _lib.check(
+            lib.muon_prepass(count, grads, None, _lib.dtype_code(t0.dtype), 0, nb, rows, cols, 0.0,
+                             0, 0, 0, ws.data_ptr(), wdt, cap, s),
+            "muon_prepass",
+        )
+        _lib.check(
+            lib.muon_orth_run(ws.data_ptr(), wdt, cap, count * nb, rows, cols, _flat_coeffs(coeffs),
+                              steps, prescale, eps, s),
+            "muon_orth_run",
+        )
+        _lib.check(
+            lib.muon_orth_extract(ws.data_ptr(), wdt, cap, count * nb, rows, cols, steps,
+                                  out.data_ptr(), _lib.dtype_code(out_dtype), s),
+            "muon_orth_extract",
+        )
+        return out
 
 
 def orthogonalize(
@@ -425,46 +433,46 @@ def _fused_step_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Tenso
     lrs = adjusted_lrs(lr_ratios, lr)
     nb, rows, cols = matrix_view(g0)
     count = len(grads)
-    ws, cap = workspace(device, torch.bfloat16, count * nb, rows, cols)
-    s = _lib.stream(device)
-    steps = len(coeffs) // 3
-    _lib.check(
-        lib.muon_prepass(count, _lib.ptr_array(grads), _lib.ptr_array(bufs),
-                         _lib.dtype_code(g0.dtype), _lib.dtype_code(bufs[0].dtype), nb, rows, cols,
-                         momentum, int(nesterov), int(maximize), int(write_back_grad),
-                         ws.data_ptr(), _lib.DT_BF16, cap, s),
-        "muon_prepass",
-    )
-    group = _group()
-    hp = (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd))
-    if group is not None:
-        group.add(device, ws, cap, count * nb, rows, cols, hp,
-                  *((params, lrs, nb) if u_scales is None else ()))
-    elif u_scales is None:
-        # the iteration and the apply in one call: the library fuses the apply into the last
-        # X' = a X + B X where the shapes allow it, else runs the post-pass after it
+    with workspace(device, torch.bfloat16, count * nb, rows, cols) as (ws, cap):
+        s = _lib.stream(device)
+        steps = len(coeffs) // 3
         _lib.check(
-            lib.muon_orth_run_apply_beside(
-                ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols, _flat_coeffs(coeffs),
-                steps, prescale, eps, count, _lib.ptr_array(params),
-                _lib.dtype_code(params[0].dtype), nb, _lib.f32_array(lrs), float(weight_decay),
-                int(cautious_wd), _beside(), s),
-            "muon_orth_run_apply",
+            lib.muon_prepass(count, _lib.ptr_array(grads), _lib.ptr_array(bufs),
+                             _lib.dtype_code(g0.dtype), _lib.dtype_code(bufs[0].dtype), nb, rows,
+                             cols, momentum, int(nesterov), int(maximize), int(write_back_grad),
+                             ws.data_ptr(), _lib.DT_BF16, cap, s),
+            "muon_prepass",
         )
-    else:
-        _lib.check(
-            lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                                     _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
-            "muon_orth_run",
-        )
-    if u_scales is not None:
-        when_done(lambda: _lib.check(
-            lib.muon_postpass(count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype), None,
-                              0, ws.data_ptr(), _lib.DT_BF16, cap, steps, nb, rows, cols,
-                              _lib.f32_array(lrs), _lib.f32_array(u_scales),
-                              float(weight_decay), int(cautious_wd), s),
-            "muon_postpass",
-        ))
+        group = _group()
+        hp = (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd))
+        if group is not None:
+            group.add(device, ws, cap, count * nb, rows, cols, hp,
+                      *((params, lrs, nb) if u_scales is None else ()))
+        elif u_scales is None:
+            # the iteration and the apply in one call: the library fuses the apply into the last
+            # X' = a X + B X where the shapes allow it, else runs the post-pass after it
+            _lib.check(
+                lib.muon_orth_run_apply_beside(
+                    ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols, _flat_coeffs(coeffs),
+                    steps, prescale, eps, count, _lib.ptr_array(params),
+                    _lib.dtype_code(params[0].dtype), nb, _lib.f32_array(lrs), float(weight_decay),
+                    int(cautious_wd), _beside(), s),
+                "muon_orth_run_apply",
+            )
+        else:
+            _lib.check(
+                lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
+                                         _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
+                "muon_orth_run",
+            )
+        if u_scales is not None:
+            when_done(lambda: _lib.check(
+                lib.muon_postpass(count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype),
+                                  None, 0, ws.data_ptr(), _lib.DT_BF16, cap, steps, nb, rows, cols,
+                                  _lib.f32_array(lrs), _lib.f32_array(u_scales),
+                                  float(weight_decay), int(cautious_wd), s),
+                "muon_postpass",
+            ))
 
 
 def fused_step(
@@ -520,36 +528,36 @@ def _fused_normuon_impl(params: list[Tensor], grads: list[Tensor], bufs: list[Te
     lrs = adjusted_lrs(lr_ratios, lr)
     nb, rows, cols = matrix_view(g0)
     count = len(grads)
-    ws, cap = workspace(device, torch.bfloat16, count * nb, rows, cols)
-    s = _lib.stream(device)
-    steps = len(coeffs) // 3
-    _lib.check(
-        lib.muon_prepass(count, _lib.ptr_array(grads), _lib.ptr_array(bufs),
-                         _lib.dtype_code(g0.dtype), _lib.dtype_code(bufs[0].dtype), nb, rows, cols,
-                         momentum, int(nesterov), int(maximize), int(write_back_grad),
-                         ws.data_ptr(), _lib.DT_BF16, cap, s),
-        "muon_prepass",
-    )
-    group = _group()
-    if group is not None:
-        group.add(device, ws, cap, count * nb, rows, cols,
-                  (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd)))
-    else:
+    with workspace(device, torch.bfloat16, count * nb, rows, cols) as (ws, cap):
+        s = _lib.stream(device)
+        steps = len(coeffs) // 3
         _lib.check(
-            lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
-                                     _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
-            "muon_orth_run",
+            lib.muon_prepass(count, _lib.ptr_array(grads), _lib.ptr_array(bufs),
+                             _lib.dtype_code(g0.dtype), _lib.dtype_code(bufs[0].dtype), nb, rows,
+                             cols, momentum, int(nesterov), int(maximize), int(write_back_grad),
+                             ws.data_ptr(), _lib.DT_BF16, cap, s),
+            "muon_prepass",
         )
-    when_done(lambda: _lib.check(
-        lib.muon_normuon_postpass(
-            count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype),
-            _lib.ptr_array(variances), _lib.dtype_code(variances[0].dtype), None, 0,
-            ws.data_ptr(), _lib.DT_BF16, cap, steps, nb, rows, cols, None, 0,
-            _lib.f32_array(lrs), None if u_scales is None else _lib.f32_array(u_scales),
-            float(weight_decay), int(cautious_wd), float(beta2), s,
-        ),
-        "muon_normuon_postpass",
-    ))
+        group = _group()
+        if group is not None:
+            group.add(device, ws, cap, count * nb, rows, cols,
+                      (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd)))
+        else:
+            _lib.check(
+                lib.muon_orth_run_beside(ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols,
+                                         _flat_coeffs(coeffs), steps, prescale, eps, _beside(), s),
+                "muon_orth_run",
+            )
+        when_done(lambda: _lib.check(
+            lib.muon_normuon_postpass(
+                count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype),
+                _lib.ptr_array(variances), _lib.dtype_code(variances[0].dtype), None, 0,
+                ws.data_ptr(), _lib.DT_BF16, cap, steps, nb, rows, cols, None, 0,
+                _lib.f32_array(lrs), None if u_scales is None else _lib.f32_array(u_scales),
+                float(weight_decay), int(cautious_wd), float(beta2), s,
+            ),
+            "muon_normuon_postpass",
+        ))
 
 
 def fused_normuon_step(
@@ -597,20 +605,20 @@ def _normuon_postpass_impl(params: list[Tensor], us: list[Tensor], variances: li
     _check_cuda_contig(list(params) + list(variances), "NorMuon tensors")
     lrs = adjusted_lrs(lr_ratios, lr)
     nb, rows, cols = matrix_view(shape)
-    ws, cap = workspace(p0.device, torch.bfloat16, nb, rows, cols)
-    sp, nsp = _splits(split_sizes)
-    s = _lib.stream(p0.device)
-    for p, u, v, lr_t in zip(params, us, variances, lrs):
-        u = u.contiguous()
-        _lib.check(
-            lib.muon_normuon_postpass(
-                1, _lib.ptr_array([p]), _lib.dtype_code(p.dtype), _lib.ptr_array([v]),
-                _lib.dtype_code(v.dtype), u.data_ptr(), _lib.dtype_code(u.dtype), ws.data_ptr(),
-                _lib.DT_BF16, cap, 0, nb, rows, cols, sp, nsp, _lib.f32_array([lr_t]), None,
-                float(weight_decay), int(cautious_wd), float(beta2), s,
-            ),
-            "muon_normuon_postpass",
-        )
+    with workspace(p0.device, torch.bfloat16, nb, rows, cols) as (ws, cap):
+        sp, nsp = _splits(split_sizes)
+        s = _lib.stream(p0.device)
+        for p, u, v, lr_t in zip(params, us, variances, lrs):
+            u = u.contiguous()
+            _lib.check(
+                lib.muon_normuon_postpass(
+                    1, _lib.ptr_array([p]), _lib.dtype_code(p.dtype), _lib.ptr_array([v]),
+                    _lib.dtype_code(v.dtype), u.data_ptr(), _lib.dtype_code(u.dtype), ws.data_ptr(),
+                    _lib.DT_BF16, cap, 0, nb, rows, cols, sp, nsp, _lib.f32_array([lr_t]), None,
+                    float(weight_decay), int(cautious_wd), float(beta2), s,
+                ),
+                "muon_normuon_postpass",
+            )
 
 
 def normuon_postpass(
@@ -643,32 +651,33 @@ def _fused_lp_impl(params: list[Tensor], grads: list[Tensor], codes: list[Tensor
     lrs = adjusted_lrs(lr_ratios, lr)
     nb, rows, cols = matrix_view(g0)
     count = len(grads)
-    ws, cap = workspace(device, torch.bfloat16, count * nb, rows, cols)
-    s = _lib.stream(device)
-    steps = len(coeffs) // 3
-    _lib.check(
-        lib.muon_lp_prepass(
-            count, _lib.ptr_array(grads), _lib.dtype_code(g0.dtype), _lib.ptr_array(codes),
-            _lib.ptr_array(scales), qmap.data_ptr() if qmap is not None else None, qformat,
-            block, nb, rows, cols, momentum, int(nesterov), int(maximize), ws.data_ptr(),
-            _lib.DT_BF16, cap, s,
-        ),
-        "muon_lp_prepass",
-    )
-    # the iteration and the apply (fused into the last B X where the shapes allow)
-    group = _group()
-    if group is not None:
-        group.add(device, ws, cap, count * nb, rows, cols,
-                  (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd)), params,
-                  lrs, nb)
-        return
-    _lib.check(
-        lib.muon_orth_run_apply_beside(
-            ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols, _flat_coeffs(coeffs), steps,
-            prescale, eps, count, _lib.ptr_array(params), _lib.dtype_code(params[0].dtype), nb,
-            _lib.f32_array(lrs), float(weight_decay), int(cautious_wd), _beside(), s),
-        "muon_orth_run_apply",
-    )
+    with workspace(device, torch.bfloat16, count * nb, rows, cols) as (ws, cap):
+        s = _lib.stream(device)
+        steps = len(coeffs) // 3
+        _lib.check(
+            lib.muon_lp_prepass(
+                count, _lib.ptr_array(grads), _lib.dtype_code(g0.dtype), _lib.ptr_array(codes),
+                _lib.ptr_array(scales), qmap.data_ptr() if qmap is not None else None, qformat,
+                block, nb, rows, cols, momentum, int(nesterov), int(maximize), ws.data_ptr(),
+                _lib.DT_BF16, cap, s,
+            ),
+            "muon_lp_prepass",
+        )
+        # the iteration and the apply (fused into the last B X where the shapes allow)
+        group = _group()
+        if group is not None:
+            group.add(device, ws, cap, count * nb, rows, cols,
+                      (tuple(coeffs), prescale, eps, float(weight_decay), int(cautious_wd)), params,
+                      lrs, nb)
+            return
+        _lib.check(
+            lib.muon_orth_run_apply_beside(
+                ws.data_ptr(), _lib.DT_BF16, cap, count * nb, rows, cols, _flat_coeffs(coeffs),
+                steps, prescale, eps, count, _lib.ptr_array(params),
+                _lib.dtype_code(params[0].dtype), nb,
+                _lib.f32_array(lrs), float(weight_decay), int(cautious_wd), _beside(), s),
+            "muon_orth_run_apply",
+        )
 
 
 def fused_lp_step(

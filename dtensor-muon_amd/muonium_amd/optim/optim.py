@@ -23,7 +23,7 @@ from torch.optim.optimizer import (
     _use_grad_for_differentiable,
 )
 
-from muonium_amd._ops import beside_others, grouped, own_workspaces, release_workspaces_except
+from muonium_amd._ops import beside_others, grouped
 from muonium_amd.orthogonalize import OrthogonalizationStrategy
 from muonium_amd.utils import group_tensors_by_shape, move_tensors_to_device
 from muonium_amd.utils.offload import pipeline_supported, run_offloaded
@@ -86,8 +86,8 @@ def _per_tensor_runs(algorithm: MuonAlgorithm, params, grads, state, split_sizes
 # fourth side stream shared a queue with the third, which serialized their buckets)
 _MAX_SIDE_STREAMS = 3
 # Side streams, and the events of their forks and joins, each of one thread (its identifier is part
-# of the key): threads stepping at the same time must not share workspaces, nor an event between
-# one's record and its wait. Those of threads that have ended go when another makes its own.
+# of the key): threads stepping at the same time must not share an event between one's record and
+# its wait. Those of threads that have ended go when another makes its own.
 _side_streams: dict[tuple[int, int, int], torch.cuda.Stream] = {}
 
 
@@ -101,7 +101,6 @@ def _side_stream(device: torch.device, slot: int) -> torch.cuda.Stream:
         for made in (_side_streams, _sync_events):
             for old in [k for k in list(made) if k[0] not in live]:
                 made.pop(old, None)
-        release_workspaces_except(live)
         stream = _side_streams[key] = torch.cuda.Stream(device=index)
     return stream
 
@@ -134,7 +133,7 @@ def _concurrent_plan(buckets, algorithm: MuonAlgorithm,
     the caller's stream. Buckets on side streams are enqueued first, so each forks from the
     caller's stream as the step starts and the largest is not held back by the host time of
     enqueueing the others (about 15 us per launch, 17 launches per bucket). Workspaces are
-    cached per stream, so a side stream never touches the buffer of the current stream or of
+    kept per stream, so a side stream never touches the buffer of the current stream or of
     another side stream, also when two buckets pad to the same workspace shape (the GPT-2
     mlp c_fc and the transposed c_proj: on one stream they ran one after the other and made
     the step's critical path). Built-in algorithms only."""
@@ -226,7 +225,7 @@ def _run_on_streams(buckets, slots: dict[int, int], order: list[int], run,
                 if key not in forked:
                     _wait(sides[i], torch.cuda.current_stream(key[0]), (*key, 0))
                     forked[key] = sides[i]
-                with torch.cuda.stream(sides[i]), own_workspaces():
+                with torch.cuda.stream(sides[i]):
                     run(i)
     finally:  # (after an error too: what was launched is ordered before the caller's next work)
         for key, side in forked.items():
