@@ -60,17 +60,14 @@ def _group_muon_tensors(
     return buckets
 
 
-def _per_tensor_runs(algorithm: MuonAlgorithm, params, grads, state, split_sizes):
-    """Index lists for the per-parameter driver: singletons (one `update` call each, the
-    reference's loop, optim.py:511-531), except that same-shape device tensors of a
-    built-in algorithm whose per-tensor update runs entirely in this library's fused
-    kernels are grouped and handed to `update_same_shape` in one launch sequence. Each
+def _per_tensor_runs(params, grads, state):
+    """Index lists for the per-parameter driver, of an algorithm whose per-tensor update runs
+    entirely in this library's fused kernels: singletons (one `update` call each, the
+    reference's loop, optim.py:511-531), except that same-shape device tensors are grouped and
+    handed to `update_same_shape` in one launch sequence. Each
     tensor keeps the per-tensor semantics (its gradient is not rewritten) and gets bit
     for bit the result of its own `update` call: the kernels treat every matrix of a
     batch independently. Groups keep first-seen order; the updates are independent."""
-    if not getattr(algorithm, "batches_per_tensor", lambda s: False)(split_sizes) or \
-            torch.compiler.is_compiling():
-        return [[i] for i in range(len(params))]
     keyed: dict[tuple, list[int]] = {}
     for i, (p, g) in enumerate(zip(params, grads)):
         if not p.is_cuda:
@@ -187,18 +184,24 @@ def _grouped_plan(buckets, slots: dict[int, int]) -> bool:
     return work <= _GROUP_WORK_PER_CU * cus
 
 
-def _share_memory(params) -> bool:
+def _share_memory(tensors) -> bool:
     """Whether the address ranges of two of the tensors meet: a weight that is also a view of
-    another, whose updates must follow each other."""
-    end = 0
-    for lo, hi in sorted(
-            (p.data_ptr(), p.data_ptr() + p.element_size() *
-             (1 + sum((n - 1) * st for n, st in zip(p.shape, p.stride()))))
-            for p in params if type(p) in (Tensor, torch.nn.Parameter) and p.numel()):
-        if lo < end:
+    another, whose updates must follow each other. Tensors whose memory cannot be looked at (a
+    subclass without storage of its own) count as sharing."""
+    spans = []
+    for t in tensors:
+        try:
+            lo, size = t.data_ptr(), t.nbytes
+            if size and not t.is_contiguous():
+                size = t.itemsize * (1 + sum((n - 1) * st for n, st in zip(t.shape, t.stride())))
+        except RuntimeError:
             return True
-        end = hi
-    return False
+        if size:
+            if lo == 0:
+                return True
+            spans.append((lo, lo + size))
+    spans.sort()
+    return any(hi > lo for (_, hi), (lo, _) in zip(spans, spans[1:]))
 
 
 def _run_on_streams(buckets, slots: dict[int, int], order: list[int], run,
@@ -574,7 +577,14 @@ class Muon(torch.optim.Optimizer):
             **opts,
         )
         if not foreach:
-            runs = _per_tensor_runs(algorithm, params, grads, state, split_sizes)
+            # same-shape runs, which go side by side as the foreach driver's buckets do, where the
+            # whole update is in the fused kernels and no parameter is a view of another; else
+            # the reference's loop, one after the other
+            apart = (len(params) > 1 and not torch.compiler.is_compiling()
+                     and getattr(algorithm, "batches_per_tensor", lambda s: False)(split_sizes)
+                     and not _share_memory(params))
+            runs = (_per_tensor_runs(params, grads, state) if apart
+                    else [[i] for i in range(len(params))])
 
             def update(idx) -> None:
                 if len(idx) == 1:
@@ -587,22 +597,18 @@ class Muon(torch.optim.Optimizer):
                         {k: [b[i] for i in idx] for k, b in state.items()},
                         [lr_ratios[i] for i in idx], **hp)
 
-            # runs that are one fused launch sequence each go side by side as the foreach
-            # driver's buckets do; anything else in the reference's order, one after the other
-            if len(runs) > 1 and getattr(algorithm, "batches_per_tensor",
-                                         lambda s: False)(split_sizes):
+            views, slots, order = [], {}, list(range(len(runs)))
+            if apart and len(runs) > 1:
                 views = [(params[idx[0]].device, None, [grads[i] for i in idx], None, None)
                          for idx in runs]
                 slots, order = _concurrent_plan(views, algorithm, None)
-                if slots and _share_memory(params):
-                    slots, order = {}, list(range(len(runs)))
-            else:
-                views, slots, order = [], {}, list(range(len(runs)))
             _run_on_streams(views, slots, order, lambda ri: update(runs[ri]))
             return
 
         buckets = _group_muon_tensors(params, grads, state, lr_ratios)
         slots, order = _concurrent_plan(buckets, algorithm, self.batch_size)
+        if slots and (_share_memory(params) or _share_memory(grads)):  # (it writes both)
+            slots, order = {}, list(range(len(buckets)))
 
         def bucket(bi) -> None:
             device, dev_p, dev_g, dev_state, dev_lr = buckets[bi]
