@@ -3072,76 +3072,115 @@ static int persistent_wgs(int64_t blocks) {
 }
 
 // Tile size of a SYRK (256, 128 or 64 rows) and of a B X launch, by the time each would take: the
-// kernels give the same bits. Microseconds of one launch, fitted to launches of 1 to 1000 matrices of
-// 128 to 4096 rows (K from 128 to 14336; within about 20%, the choice within 10% of the best
-// of the three measured ones). A launch on 256-row tiles is rounds of one workgroup per CU, each
-// its prologue and epilogue plus a time per k; on 128-row tiles two workgroups share a CU, and
-// once the CUs are full the time goes by the operand bytes (half the reuse of 256-row tiles);
-// 64-row tiles have the shortest chain and again half the reuse. blocks: tiles of the size at
-// hand; the padding beyond round_up(m, 128) rows is only computed by 256-row tiles.
-// beside: the launch shares the device with other streams' (a step's small buckets). Near the lines
-// the larger tiles then win, since what the launch takes from its neighbours counts, not its own
-// time: 24 fp32 matrices of four shapes with 8-bit momentum, on four streams, took 0.95 ms a
-// step with the factors below and 1.11 without; a dozen matrices each of four shapes 0.5% more
-// with 0.8 in place of 0.6.
-// Measured (us, 256 / 128 / 64): X X^T of 1 x 256 x 512 12.4 / 13.3 / 7.7 and of 1 x 1024 x 4096 52.9 / 45.4
-// / 20.7, of 64 x 512 x 2048 65 / 80 / 79; A A of 1408 rows 45.5 / 22.0 / 11.5; B X of 4 x 512 x 512
-// 22.0 / 12.1 / 9.3, of 2 x 1024 x 4096 30.2 / 24.3 / 39.4, of 12 x 768 x 3072 47.5 / 56 / 99.
-static double per_cu(int64_t blocks) {
-  const double w = (double)blocks / device_cus();
-  return w <= 1.0 ? 1.0 : w + 0.5;
-}
-static int64_t rounds_of(int64_t blocks) { return (blocks + device_cus() - 1) / device_cus(); }
+// kernels give the same bits. TileCost holds what a launch of one kernel takes in microseconds: up
+// to one workgroup per CU `one` + `one_k` per k; beyond, `base` plus, for each round of
+// workgroups over the CUs, `wave` + `wave_k` per k, where a last round that is partly filled counts
+// the share `whole` as a full one (two workgroups share a CU on 128- and 64-row tiles, so there the
+// others go on meanwhile). 256-row tiles have a long prologue and epilogue and the most reuse, 64-row
+// tiles the shortest chain; the padding beyond round_up(m, 128) rows is only computed by 256-row tiles.
+// Fitted to launches as they follow each other in 1178 iterations (1 to 300 matrices of 65 to 4096
+// rows, up to 16384 columns) and 1978 Gram products (256 to 4096 rows, K from 128 to 8192), each on
+// all three sizes; a launch is 5 to 11% from its cost (root mean square), and the size chosen
+// is on average 0.6% (SYRK) and 0.4% (B X) slower than the best of the three.
+// Measured (us, 256 / 128 / 64, between events): X X^T of 1 x 128 x 256 27 / 11 / 7, of 16 x 768 x 768 38 /
+// 21 / 22, of 24 x 768 x 3072 82 / 53 / 88, of 4 x 4096 x 4096 276 / 294 / 587; B X of the same 15 / 8.9 / 7.4,
+// 26 / 29 / 36, 93 / 111 / 183 and 386 / 538 / 896.
+struct TileCost {
+  double one, one_k, base, wave, wave_k, whole;
+};
+constexpr TileCost SYRK_256 = {22.4, 0.0162, 7.4, 13.0, 0.0220, 0.5};
+constexpr TileCost SYRK_PACKED = {19.9, 0.0239, 20.0, 10.0, 0.0254, 0.5};  // gemm_bf16_v2_kernel
+constexpr TileCost SYRK_128 = {6.8, 0.0081, 5.8, 2.35, 0.0068, 0.5};
+constexpr TileCost SYRK_64 = {4.7, 0.0033, 3.5, 1.0, 0.0028, 0.7};
+constexpr TileCost BX_256 = {16.7, 0.0213, 14.5, 6.0, 0.0216, 0.6};
+constexpr TileCost BX_128 = {6.1, 0.0099, 3.1, 2.35, 0.0068, 0.8};
+constexpr TileCost BX_64 = {4.9, 0.0046, 3.6, 1.1, 0.0029, 1.0};
 
+static double tile_cost(const TileCost& c, int64_t tiles, double k) {
+  const int64_t cus = device_cus(), rounds = (tiles + cus - 1) / cus;
+  if (rounds <= 1) return c.one + c.one_k * k;
+  const double w = c.whole * (double)rounds + (1.0 - c.whole) * (double)tiles / (double)cus;
+  return c.base + w * (c.wave + c.wave_k * k);
+}
+
+// Tiles of k on average, kmax at most (several buckets in one launch): the longest takes its time.
+static double tile_cost(const TileCost& c, int64_t tiles, double k, double kmax) {
+  return std::max(c.one + c.one_k * kmax, tile_cost(c, tiles, k));
+}
+
+// Data beyond the 256 MB of the last cache: the smaller tiles' further reads of their operands then
+// compete with the result's way to memory. For a Gram product its operand and result count
+// (32 x 2048 x 1024 takes 180 us on 256-row tiles and 198 on 128-row ones, 9 x 2048 x 2048 96 and 78), in
+// an iteration X, X', A and B (24 x 2048 x 2048: 209 and 251).
+static bool past_cache(int64_t bytes) { return bytes > ((int64_t)256 << 20); }
+
+// B X on 256-row tiles is persistent: a workgroup count that is no multiple of the 8 XCDs spreads a
+// round's tiles unevenly over their L2s (two rounds of 130 to 250 workgroups take 1.3 times those of
+// a multiple of 8, three 1.2 times).
+static double bx256_cost(int64_t tiles, double k) {
+  const int64_t cus = device_cus(), rounds = (tiles + cus - 1) / cus;
+  const bool uneven = rounds > 1 && persistent_wgs(tiles) % 8 != 0;
+  return tile_cost(BX_256, tiles, k) * (uneven ? 1.0 + 0.6 / (double)rounds : 1.0);
+}
+
+// What a SYRK on 128- or 64-row tiles takes more where the L2s do not hold a matrix and its rows are
+// read again from the last cache: 2240 rows, K 8108 (36 MB) takes 150 / 85 / 114 us on 256- / 128- /
+// 64-row tiles, 4096 rows, K 4096 (32 MB) 78 / 93 / 159.
+static double far_rows(int tm, int64_t tiles, double k, int64_t rows) {
+  const double mb = (double)rows * k * 2.0 / (1 << 20);
+  if (mb <= 2.0 || (tm == 64 && tiles <= device_cus())) return 1.0;
+  return 1.0 + (tm == 64 ? 0.01 : 0.0025) * (mb - 2.0);
+}
+static double syrk_cost(int tm, int64_t tiles, double k, int64_t rows) {
+  return tile_cost(tm == 64 ? SYRK_64 : SYRK_128, tiles, k) * far_rows(tm, tiles, k, rows);
+}
+
+// Costs within 5 or 6% of each other are ties and go to the larger tiles, which read less; a cut of
+// long sums (K from 4096 on, where the two launches' ends weigh little) takes what it is thought to.
+// beside: the launch shares the device with other streams' (a step's small buckets). The larger
+// tiles then win over a wider range, since what the launch takes from its neighbours counts, not its
+// own time.
 //
 // head > 0: the first `head` tiles (whole rounds) on 256-row tiles, the rest, which would leave most
-// CUs idle for a round, cut into tm-row tiles in a second launch. Eight matrices of 4096 rows
-// are 4.25 rounds, four 2.125, two 1.06: the Gram launches of a step on four layers of a 4096-wide
-// model (28 matrices) went from 23.7 to 21.0 ms, the step from 51.7 to 50.1 ms, on one layer from
-// 13.5 to 12.5 ms; X X^T of 20 x 1280 x 5120 221 -> 202 us, of 8 x 2048 x 8192 321 -> 282.
-// Launches of whole rounds (64 such matrices) keep one launch, and so does K below 4096, where the
-// second launch's fill and drain take what the round saves (16 x 2048 x 2048: 152 us in one, 164
-// in two; 32 x 1024 x 1024 51 and 62; 100 x 512 x 2048 82 and 107), and a launch that 128-row tiles
-// fill evenly (30 x 1024 x 4096: 166 and 170; c128 is a fifth above the measured there, hence 0.78).
+// CUs idle for a round, cut into tm-row tiles in a second launch (8 us for its fill and the first
+// one's drain). Eight matrices of 4096 rows are 4.25 rounds, four 2.125, two 1.06: the Gram launches
+// of a step on four layers of a 4096-wide model (28 matrices) went from 23.7 to 21.0 ms, the step
+// from 51.7 to 50.1 ms, on one layer from 13.5 to 12.5 ms. Over 936 products of more than a round
+// the choice is 0.8% slower on average than the best form of each, and 1.4% if none is cut.
 struct SyrkPlan {
   int tm;
   int64_t head;
 };
 static SyrkPlan syrk_plan(int64_t batch, int64_t m, int64_t K, int64_t blocks256, bool packed,
-                          int beside) {
-  const int64_t t1 = round_up(m, 128) / 128, t2 = 2 * t1, cus = device_cus();
+                          bool past, int beside) {
+  const int64_t rows = round_up(m, 128), t1 = rows / 128, t2 = 2 * t1, cus = device_cus();
   const int64_t n128 = t1 * (t1 + 1) / 2 * batch, n64 = t2 * (t2 + 1) / 2 * batch;
-  const double k = (double)K, round = 17.0 + 0.0212 * k;
-  auto c128_of = [&](int64_t n) {
-    return n <= cus ? 9.0 + 0.0089 * k : 9.0 + per_cu(n) * (1.7 + 0.0092 * k);
-  };
-  auto c64_of = [&](int64_t n) { return 5.0 + rounds_of(n) * (0.6 + 0.0037 * k); };
-  const double c256 = rounds_of(blocks256) * round, c128 = c128_of(n128), c64 = c64_of(n64);
+  const double k = (double)K, far = past ? 1.07 : 1.0;
+  const double c256 = tile_cost(packed ? SYRK_PACKED : SYRK_256, blocks256, k);
+  const double c128 = far * syrk_cost(128, n128, k, rows), c64 = far * syrk_cost(64, n64, k, rows);
   SyrkPlan best = {256, 0};
-  if (c64 < (beside ? 0.75 : 1.0) * c128 && c64 < c256) best.tm = 64;
-  else if (c128 < c256) best.tm = 128;
+  double cost = c256;
+  const double tie = beside ? 0.65 : n64 > cus && K >= 2048 ? 0.95 : 1.0;
+  if (c64 < tie * c128 && c64 < c256) best.tm = 64, cost = c64;
+  else if (c128 < 0.94 * c256) best.tm = 128, cost = c128;
   const int64_t head = blocks256 / cus * cus, rest = blocks256 - head;
-  if (!packed && head > 0 && rest > 0 && K >= 4096) {
-    const double r128 = c128_of(4 * rest), r64 = c64_of(16 * rest);
-    const double split = (double)(head / cus) * round + 4.0 + std::min(r128, r64);
-    if (split < (best.tm == 64 ? 0.97 * c64 : best.tm == 128 ? 0.78 * c128 : 0.97 * c256))
+  if (!packed && head > 0 && rest > 0) {
+    const double r128 = tile_cost(SYRK_128, 4 * rest, k), r64 = tile_cost(SYRK_64, 16 * rest, k);
+    if (tile_cost(SYRK_256, head, k) + 8.0 + std::min(r128, r64) <
+        (K >= 4096 ? 0.98 : 0.94) * cost)
       best = {r64 < r128 ? 64 : 128, head};
   }
   return best;
 }
 
 static int bx_tile(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, int beside) {
-  const int64_t me = round_up(m, 128);
-  const int64_t n256 = (M / 256) * (N / 256) * batch, n128 = (me / 128) * (N / 128) * batch;
-  const int64_t n64 = 4 * n128;
-  const double k = (double)K;
-  const double c256 = rounds_of(n256) * (9.0 + 0.0215 * k);
-  const double c128 = n128 <= device_cus()       ? 5.5 + 0.0122 * k
-                      : n128 <= 2 * device_cus() ? 6.0 + 0.0185 * k
-                                                 : 6.0 + per_cu(n128) * (0.8 + 0.0098 * k);
-  const double c64 = n64 <= device_cus() ? 4.5 + 0.0078 * k : 4.5 + per_cu(n64) * (0.5 + 0.0038 * k);
-  if (c64 < c128 && c64 < c256) return 64;
-  return c128 < (beside ? 0.6 : 0.9) * c256 ? 128 : 256;
+  const int64_t rows = round_up(m, 128);
+  const int64_t n256 = (M / 256) * (N / 256) * batch, n128 = rows / 128 * (N / 128) * batch;
+  const double k = (double)K, far = past_cache(batch * rows * (N + rows) * 4) ? 1.08 : 1.0;
+  const double c256 = bx256_cost(n256, k), c128 = far * tile_cost(BX_128, n128, k),
+               c64 = far * tile_cost(BX_64, 4 * n128, k);
+  if (c64 < 0.95 * c128 && c64 < c256) return 64;
+  return c128 < (beside ? 0.5 : 1.0) * c256 ? 128 : 256;
 }
 
 // `g` on TM-row tiles covering round_up(m, 128) rows (of a SYRK, columns too).
@@ -3277,7 +3316,9 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
         gp.tiles_per_batch = (T - 1) * T / 2 + (2 * T - 1 + 3) / 4;
         gp.tiles_total = gp.tiles_per_batch * (int)batch;
       }
-      const SyrkPlan plan = syrk_plan(batch, Mv, K, gp.tiles_total, packed, beside);
+      // (A A's operands are a small part of an iteration's data)
+      const bool past = beta == 0.0f && past_cache(batch * M * (K + M) * (scale ? 4 : 2));
+      const SyrkPlan plan = syrk_plan(batch, Mv, K, gp.tiles_total, packed, past, beside);
       const int TM = plan.tm;
       if (plan.head > 0) {
         hipLaunchKernelGGL(gemm_bf16_s16_kernel, dim3((unsigned)plan.head), dim3(512), V2_SMEM,
@@ -3307,7 +3348,9 @@ int muon_launch_gemm(int dtype, int mode, bool masked, int64_t batch, int64_t M,
       }
     } else if (masked && K % 8 == 0 && !((uintptr_t)a & 15)) {
       // gram_ of any extents, rows of whole 16-byte chunks
-      const int TM = syrk_plan(batch, M, K, blocks, true, 0).tm == 64 ? 64 : 128;
+      const int64_t t1 = (M + 127) / 128, t2 = (M + 63) / 64;
+      const int TM = syrk_cost(64, t2 * (t2 + 1) / 2 * batch, (double)K, M) <
+                             syrk_cost(128, t1 * (t1 + 1) / 2 * batch, (double)K, M) ? 64 : 128;
       GemmArgs gt = g;
       gt.tiles_m = gt.tiles_n = (int)((M + TM - 1) / TM);
       gt.tiles_per_batch = gt.tiles_m * (gt.tiles_m + 1) / 2;
@@ -3378,8 +3421,7 @@ int muon_apply_fuses(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, 
   const int pes = pdt == MUON_DT_F32 ? 4 : 2;
   const double post = 6.0 + (double)batch * m * n * (2 + 2 * pes) / 5.0e6;
   const int64_t n256 = (M / 256) * (N / 256) * batch, n128 = round_up(m, 128) / 128 * (N / 128) * batch;
-  const double c256 = rounds_of(n256) * (9.0 + 0.0215 * (double)K);
-  const double c128 = 6.0 + per_cu(n128) * (0.8 + 0.0098 * (double)K);
+  const double c256 = bx256_cost(n256, (double)K), c128 = tile_cost(BX_128, n128, (double)K);
   return bx_tile(batch, M, N, K, m, beside) != 256 || c128 < c256 + 0.5 * post;
 }
 
@@ -3521,20 +3563,10 @@ int muon_launch_products(int mode, int n, const MuonProduct* items, float alpha,
       return MUON_ERR_SHAPE;
     }
     const double kavg = work / (double)n128;
-    const int64_t n64 = 4 * n128;
-    bool t64;
-    if (mode == MODE_SYRK) {
-      const double c128 = n128 <= device_cus() ? 9.0 + 0.0089 * kmax
-                                               : std::max(9.0 + 0.0089 * kmax, 9.0 + per_cu(n128) * (1.7 + 0.0092 * kavg));
-      const double c64 = std::max(5.0 + 0.0037 * kmax, 5.0 + per_cu(n64) * (0.6 + 0.0037 * kavg));
-      t64 = c64 < c128;
-    } else {
-      const double c128 = n128 <= device_cus() ? 5.5 + 0.0122 * kmax
-                                               : 6.0 + per_cu(n128) * (0.8 + 0.0098 * kavg);
-      const double c64 = n64 <= device_cus() ? 4.5 + 0.0078 * kmax
-                                             : 4.5 + per_cu(n64) * (0.5 + 0.0038 * kavg);
-      t64 = c64 < c128;
-    }
+    const bool t64 = mode == MODE_SYRK ? tile_cost(SYRK_64, 4 * n128, kavg, kmax) <
+                                             tile_cost(SYRK_128, n128, kavg, kmax)
+                                       : tile_cost(BX_64, 4 * n128, kavg, kmax) <
+                                             tile_cost(BX_128, n128, kavg, kmax);
     const int TM = t64 ? 64 : 128;
     GemmTab tab;
     memset(&tab, 0, sizeof(tab));
