@@ -634,12 +634,11 @@ static int orth_run_group(int nbuckets, const MuonBucket* buckets, const double*
   const int n = (int)own.size();
   if (n == 0) return MUON_OK;
   hipStream_t s = (hipStream_t)stream;
-  double xx = 0.0, aa = 0.0, bx = 0.0;
+  double xx = 0.0, aa = 0.0;
   for (int i = 0; i < n; ++i) {
     const double bm = (double)batch[i], md = (double)L[i].m, nd = (double)L[i].n;
     xx += bm * md * (md + 1) * nd;
     aa += bm * md * (md + 1) * md;
-    bx += bm * 2.0 * md * md * nd;
   }
   int rc;
   {
@@ -760,10 +759,15 @@ static int orth_run_group(int nbuckets, const MuonBucket* buckets, const double*
       if (rc != MUON_OK) return rc;
     }
     int cnt = 0;
-    for (int k = 0; k < n; ++k)
-      if (!done[order[k]]) fill(order[k], 2, items[cnt++]);
+    double bx = 0.0;
+    for (int k = 0; k < n; ++k) {
+      const int i = order[k];
+      if (done[i]) continue;
+      fill(i, 2, items[cnt++]);
+      bx += (double)batch[i] * 2.0 * L[i].m * L[i].m * L[i].n;
+    }
     if (cnt > 0) {
-      Timed t(MUON_K_GEMM_BX, last ? 0.0 : bx, s);
+      Timed t(MUON_K_GEMM_BX, bx, s);
       rc = muon_launch_products(MODE_GEMM, cnt, items.data(), 1.0f, a, first ? 1 : 0, nullptr, 0, 0, s);
     }
     if (rc != MUON_OK) return rc;
