@@ -1039,16 +1039,6 @@ constexpr int NN_STAGEB = NN_ATILEB + NN_XTILEB;
 
 typedef __attribute__((ext_vector_type(4))) short i16x4;
 
-MUON_DEVICE void nn_join(bf16x8_mfma (&cx)[4], const i16x4 (&lo)[4], const i16x4 (&hi)[4]) {
-#pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    const i16x4 l = lo[f], h = hi[f];
-    const __attribute__((ext_vector_type(8))) short v =
-        __builtin_shufflevector(l, h, 0, 1, 2, 3, 4, 5, 6, 7);
-    cx[f] = __builtin_bit_cast(bf16x8_mfma, v);
-  }
-}
-
 // ----------------------------------------------------------------------------------
 // Persistent bf16 X' = alpha * (B X + ratio * X): 4 wavefronts (2 x 2), each owning a
 // 128 x 128 block of the 256 x 256 tile, accumulators in AGPRs (256 per lane).
@@ -2433,7 +2423,8 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_s16h_kernel(Args args) {
 constexpr int F_TM = 64, F_KT = 32, F_NS = 5;
 constexpr int F_PANELB = F_TM * F_KT * 4, F_STAGEB = 2 * F_PANELB, F_SMEM = F_NS * F_STAGEB;
 
-MUON_DEVICE void f32_dma(int vo, u32x4 rs, int so, uint32_t m0) {
+// 16 bytes per lane from memory to LDS (1 KB per wave from byte m0 on).
+MUON_DEVICE void lds_dma(int vo, u32x4 rs, int so, uint32_t m0) {
   asm volatile("s_mov_b32 m0, %[mz]\n\ts_nop 0\n\tbuffer_load_dwordx4 %[vo], %[rs], %[so] offen lds\n\t"
                :
                : [vo] "v"(vo), [rs] "s"(rs), [so] "s"(so), [mz] "s"(m0)
@@ -2479,12 +2470,12 @@ __global__ __launch_bounds__(512, 4) void gemm_f32_kernel(GemmArgs g) {
     const uint32_t m0 = lds0 + st * F_STAGEB + wave * 1024;
     if constexpr (OWN) {
       const int co = kk * F_KT * 4 + lch * 16 < lda_b ? kk * F_KT * 4 + lch * 16 : 0;
-      f32_dma(voa + co, on ? rsa : rs_none, 0, m0);
-      f32_dma(vob + co, on ? rsb : rs_none, 0, m0 + F_PANELB);
+      lds_dma(voa + co, on ? rsa : rs_none, 0, m0);
+      lds_dma(vob + co, on ? rsb : rs_none, 0, m0 + F_PANELB);
       return;
     }
-    f32_dma(voa, on ? rsa : rs_none, kk * F_KT * 4, m0);
-    f32_dma(vob, on ? rsb : rs_none, kk * kstep_b, m0 + F_PANELB);
+    lds_dma(voa, on ? rsa : rs_none, kk * F_KT * 4, m0);
+    lds_dma(vob, on ? rsb : rs_none, kk * kstep_b, m0 + F_PANELB);
   };
 
   f32x16 acc;
@@ -2588,13 +2579,6 @@ struct TileK {
   static_assert(TM * PITCH * 2 <= SMEM, "the staging tile fits the stages");
 };
 
-MUON_DEVICE void tile_dma(int vo, u32x4 rs, int so, uint32_t m0) {
-  asm volatile("s_mov_b32 m0, %[mz]\n\ts_nop 0\n\tbuffer_load_dwordx4 %[vo], %[rs], %[so] offen lds\n\t"
-               :
-               : [vo] "v"(vo), [rs] "s"(rs), [so] "s"(so), [mz] "s"(m0)
-               : "m0", "memory");
-}
-
 // A = alpha X X^T (K = n) or B = alpha (A A + ratio A): upper-triangle tiles, mirrored.
 // OWN: gram_ of caller-owned tensors, M and K any (rows a whole number of 16-byte chunks): rows past
 // the last read the last one, the chunks past a row's end its first one and count as zero, and
@@ -2643,11 +2627,11 @@ __global__ __launch_bounds__(256, 2) void tile_syrk_kernel(Args args) {
     for (int q = 0; q < C::LOADS; ++q) {
       if constexpr (OWN) {
         const int co = kb + lch * 16 < lda_b ? kb + lch * 16 : 0;
-        tile_dma(voa[q] + co, pa, 0, m0 + q * 4096);
-        tile_dma(vob[q] + co, pb, 0, m0 + C::PANELB + q * 4096);
+        lds_dma(voa[q] + co, pa, 0, m0 + q * 4096);
+        lds_dma(vob[q] + co, pb, 0, m0 + C::PANELB + q * 4096);
       } else {
-        tile_dma(vo, pa, kb + q * 32 * lda_b, m0 + q * 4096);
-        tile_dma(vo, pb, kb + q * 32 * lda_b, m0 + C::PANELB + q * 4096);
+        lds_dma(vo, pa, kb + q * 32 * lda_b, m0 + q * 4096);
+        lds_dma(vo, pb, kb + q * 32 * lda_b, m0 + C::PANELB + q * 4096);
       }
     }
   };
@@ -2840,8 +2824,8 @@ __global__ __launch_bounds__(256, 2) void tile_bx_kernel(Args args, MuonApply ap
     const u32x4 pa = on ? rsa : rs_none, px = on ? rsx : rs_none;
 #pragma unroll
     for (int q = 0; q < C::LOADS; ++q) {
-      tile_dma(voa, pa, kk * V2_ROWB + q * 32 * lda_b, m0 + q * 4096);
-      tile_dma(vox, px, (kk * V2_BK + q * (4096 / XR)) * ldx_b, m0 + C::PANELB + q * 4096);
+      lds_dma(voa, pa, kk * V2_ROWB + q * 32 * lda_b, m0 + q * 4096);
+      lds_dma(vox, px, (kk * V2_BK + q * (4096 / XR)) * ldx_b, m0 + C::PANELB + q * 4096);
     }
   };
   float alpha = g.alpha, beta = g.beta;
@@ -3196,9 +3180,9 @@ static GemmArgs on_tiles(const GemmArgs& g, int mode, int TM, int64_t m, int64_t
 
 }  // namespace
 
-// Launch one batched product. `dtype` selects bf16 (256-tiles) or fp32 (128-tiles).
-// M/N are the (padded) output extents; they must be multiples of the tile unless
-// `masked`. SYRK: a and b are the same K-contiguous rows. GEMM (NN): b is the
+// Launch one batched product. `dtype` selects bf16 (256-, 128- or 64-row tiles) or fp32 (64-row
+// tiles; gram_ of rows that are no whole 16-byte chunks 128). M/N are the (padded) output extents;
+// they must be multiples of 256 (fp32: 128) unless `masked`. SYRK: a and b are the same K-contiguous rows. GEMM (NN): b is the
 // K x N row-major operand (row pitch ldb) and the beta term reads cin = b's first
 // M rows (cin(i, j) = b(i, j), true of X' = a X + B X); the bf16 kernels take it from
 // the staged operand panels. Masked (arbitrary-extent) launches exist for SYRK only.
