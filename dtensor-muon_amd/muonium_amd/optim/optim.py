@@ -117,6 +117,11 @@ def _wait(waiter: torch.cuda.Stream, producer: torch.cuda.Stream, key: tuple) ->
     waiter.wait_event(ev)
 
 
+@functools.lru_cache(maxsize=64)
+def _compute_units(device: torch.device) -> int:
+    return torch.cuda.get_device_properties(device).multi_processor_count
+
+
 def _concurrent_plan(buckets, algorithm: MuonAlgorithm,
                      batch_size: int | None) -> tuple[dict[int, int], list[int]]:
     """Side-stream slot per bucket index for buckets too small to fill the device, and the
@@ -138,17 +143,14 @@ def _concurrent_plan(buckets, algorithm: MuonAlgorithm,
     if not type(algorithm).__module__.startswith("muonium_amd.") or torch.compiler.is_compiling():
         return {}, natural  # (under an outer torch.compile the buckets run in the traced order)
 
-    cus: dict[torch.device, int] = {}
     work: dict[int, int] = {}
     for bi, (device, _, dev_g, _, _) in enumerate(buckets):
         if device.type != "cuda" or dev_g[0].dim() < 2:
             continue
-        if device not in cus:
-            cus[device] = torch.cuda.get_device_properties(device).multi_processor_count
         rows, cols = dev_g[0].shape[-2:]
         nmat = math.prod(dev_g[0].shape[:-2]) * min(len(dev_g), batch_size or len(dev_g))
         tiles = -(-min(rows, cols) // 256)
-        if tiles * (tiles + 1) // 2 * nmat < cus[device]:
+        if tiles * (tiles + 1) // 2 * nmat < _compute_units(device):
             work[bi] = min(rows, cols) ** 2 * max(rows, cols) * nmat
     if len(work) < 2:
         return {}, natural
@@ -158,30 +160,54 @@ def _concurrent_plan(buckets, algorithm: MuonAlgorithm,
     return slots, side + [bi for bi in natural if bi not in slots]
 
 
-# The most work of a step's buckets that goes in common launches: 128-row tiles of B X times their
-# K, per CU. With less the host's launches bound the step: 16 matrices of four shapes of a small
+# The most work of a step's buckets that the host bounds: 128-row tiles of B X times their K, per CU.
+# With less the launches bound the step and go in common ones: 16 matrices of four shapes of a small
 # model (512 wide, 1536 per CU) took 0.67-0.74 ms on four streams and 0.40 ms in common launches,
 # eight matrices of three shapes (768 wide, 2160) 0.54 and 0.45 ms. With more the device does,
 # and the streams' 256-row tiles read half the operand bytes: six of 1024 wide (3072) took 0.53
-# and 0.55 ms, two dozen of 768 wide (7776) 0.97 and 1.12 ms.
+# and 0.55 ms, two dozen of 768 wide (7776) 0.97 and 1.12 ms. One bucket of the set may be large
+# enough to fill the device by itself (us, streams and common launches): 300 matrices of 128 x 128
+# beside four small ones 460 and 246, 256 of 128 x 1024 656 and 583, 256 of 256 x 512 (2304) 631 and 640.
 _GROUP_WORK_PER_CU = 2400
+# Iterates of at most 64 rows have launches of their own; up to this many columns they overlap less on
+# streams than the forks and joins take (us on streams and in order, two boxes: 2 x 64 x 16384 and
+# 32 x 16384 253 and 281, 269 and 270; 64 x 32768, 64 x 16000, 128 x 1024 and 256 x 512 538 and 568, 477).
+_HOST_BOUND_SHORT_COLS = 32768
 
 
-def _grouped_plan(buckets, slots: dict[int, int]) -> bool:
-    """Whether the buckets, all of which `_concurrent_plan` would run side by side, run in common
-    launches instead: so little work that the host takes longer to launch it than the device to
-    run it, on one device and stream."""
-    if len(slots) + 1 != len(buckets):  # (all but one on side streams: every bucket is small)
-        return False
+def _host_bound(buckets) -> bool:
+    """Whether the buckets are so little work that the host takes longer to launch it than the device
+    to run it, on one device and stream."""
     work = 0
     for device, _, grads, _, _ in buckets:
         rows, cols = grads[0].shape[-2:]
-        if device != buckets[0][0] or min(rows, cols) <= 64:
+        if device != buckets[0][0]:
             return False
+        if min(rows, cols) <= 64:
+            if max(rows, cols) > _HOST_BOUND_SHORT_COLS:
+                return False
+            continue
         tiles_m, tiles_n = -(-min(rows, cols) // 128), 2 * -(-max(rows, cols) // 256)
         work += math.prod(grads[0].shape[:-2]) * len(grads) * tiles_m * tiles_n * tiles_m * 128
-    cus = torch.cuda.get_device_properties(buckets[0][0]).multi_processor_count
-    return work <= _GROUP_WORK_PER_CU * cus
+    return work <= _GROUP_WORK_PER_CU * _compute_units(buckets[0][0])
+
+
+def _has_short(buckets) -> bool:
+    return any(min(grads[0].shape[-2:]) <= 64 for _, _, grads, _, _ in buckets)
+
+
+def _grouped_plan(buckets, slots: dict[int, int]) -> bool:
+    """Whether the buckets, all but one of which `_concurrent_plan` has on side streams, run in common
+    launches instead."""
+    return (len(slots) + 1 == len(buckets) and not _has_short(buckets) and _host_bound(buckets))
+
+
+def _in_order(buckets) -> bool:
+    """Whether buckets that `_concurrent_plan` has on side streams run one after the other instead:
+    some are not for common launches, and the forks and joins take longer than what they
+    overlap (us on streams and in order: 64 x 128, 128 x 64 and 80 x 80 380-396 and 244-254, 64 x 1024,
+    128 x 512 and 256 x 256 383-411 and 270-278, eight of 64 x 1024, 16 x 4096 and 2048 x 64 393-404 and 360)."""
+    return _has_short(buckets) and _host_bound(buckets)
 
 
 def _share_memory(tensors) -> bool:
@@ -209,14 +235,16 @@ def _run_on_streams(buckets, slots: dict[int, int], order: list[int], run,
     """``run(i)`` for every i of ``order``; those with a slot on that side stream of their
     device, forked from the caller's stream at first use and joined back into it at the end;
     or all of them on the caller's stream, in common launches (``whole``: no bucket is cut into
-    batches, whose workspaces a group would hold at the same time). The plan's streams are made
-    either way: the gradients of a later step may need them."""
+    batches, whose workspaces a group would hold at the same time) or in order. The plan's streams
+    are made either way: the gradients of a later step may need them."""
     sides = {i: _side_stream(buckets[i][0], slot) for i, slot in slots.items()}
     if slots and whole and _grouped_plan(buckets, slots):
         with grouped():
             for i in order:
                 run(i)
         return
+    if slots and _in_order(buckets):
+        slots = {}
     forked: dict[tuple[torch.device, int], torch.cuda.Stream] = {}
     try:
         with beside_others(bool(slots)):
