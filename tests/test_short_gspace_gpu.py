@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from helpers import rel_fro
+from muonium_amd import _lib, _ops
 from muonium_amd.orthogonalize import foreach_zeropower, zeropower
 from muonium_amd.orthogonalize.newton_schulz import ns_loop
 from muonium_amd.orthogonalize.polar_express import pe_loop
@@ -63,14 +64,36 @@ def test_rank_deficient_zero_and_nan_matrices():
     assert out[2].isnan().all()
 
 
-def test_many_steps_and_large_coefficients_take_the_streaming_iteration():
-    """Six steps, and coefficients whose squares multiply past 2^18, stay on the iteration that
-    reads X each time (an error of the Gram matrix would grow too far)."""
-    X = _x((16, 65536))
-    coeffs = [(3.4445, -4.7750, 2.0315)] * 6
+NS = (3.4445, -4.7750, 2.0315)
+
+
+def _launches(X, coeffs):
+    """The update and the B X launches of its iteration: one on the Gram matrix, one per step where X is
+    read each time."""
+    x = X.to(DEV)
+    _lib.timing_enable(True)
+    u = _ops.orthogonalize([x], coeffs, prescale=1.0, eps=1e-7, iter_dtype=torch.bfloat16,
+                           out_dtype=torch.bfloat16)[0]
+    launches = _lib.timing_read()["gemm_bx"][1]
+    _lib.timing_enable(False)
     ref = muon_ref.polar_iteration_bf16(X.float(), coeffs, prescale=1.0, eps=1e-7)
-    assert rel_fro(ns_loop(X.to(DEV), 6).cpu(), ref) <= 1e-2
-    big = [(30.0, -50.0, 0.0)] * 5
-    got = ns_loop(X.to(DEV), 5, a=30.0, b=-50.0, c=0.0).cpu()
-    ref = muon_ref.polar_iteration_bf16(X.float(), big, prescale=1.0, eps=1e-7)
-    assert got.isfinite().equal(ref.isfinite())
+    assert u.isfinite().all()
+    assert rel_fro(u.cpu(), ref) <= 1e-2
+    return launches
+
+
+def _first(a, singular=0.25):
+    """Coefficients whose first step takes 16 equal singular values (of a unit-norm matrix) to 1."""
+    return [(a, (1.0 - a * singular) / singular ** 3, 0.0)] + [NS] * 4
+
+
+@pytest.mark.parametrize("shape, coeffs, gram", [
+    # up to five steps
+    ((16, 65536), [NS] * 5, True), ((16, 65536), [NS] * 6, False), ((16, 65536), [NS], False),
+    # the squares of all leading coefficients but the last multiply to 2^18 at a = 12.528
+    ((16, 65536), _first(12.4), True), ((16, 65536), _first(12.6), False),
+    ((16, 65535), [NS] * 5, False), ((65, 65536), [NS] * 2, False)])
+def test_many_steps_and_large_coefficients_take_the_streaming_iteration(shape, coeffs, gram):
+    """Six steps, and coefficients whose squares multiply past 2^18, stay on the iteration that
+    reads X each time (an error of the Gram matrix would grow too far), as do narrower and taller ones."""
+    assert _launches(_x(shape), coeffs) == (1 if gram else len(coeffs))
