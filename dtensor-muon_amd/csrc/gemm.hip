@@ -3092,11 +3092,11 @@ static double tile_cost(const TileCost& c, int64_t tiles, double k, double kmax)
   return std::max(c.one + c.one_k * kmax, tile_cost(c, tiles, k));
 }
 
-// Data beyond the 256 MB of the last cache: the smaller tiles' further reads of their operands then
+// Data beyond what the last cache (256 MB) keeps: the smaller tiles' further reads of their operands then
 // compete with the result's way to memory. For a Gram product its operand and result count
 // (32 x 2048 x 1024 takes 180 us on 256-row tiles and 198 on 128-row ones, 9 x 2048 x 2048 96 and 78), in
 // an iteration X, X', A and B (24 x 2048 x 2048: 209 and 251).
-static bool past_cache(int64_t bytes) { return bytes > ((int64_t)256 << 20); }
+static bool past_cache(int64_t bytes) { return bytes > ((int64_t)240 << 20); }
 
 // B X on 256-row tiles is persistent: a workgroup count that is no multiple of the 8 XCDs spreads a
 // round's tiles unevenly over their L2s (two rounds of 130 to 250 workgroups take 1.3 times those of
@@ -3124,7 +3124,8 @@ static double syrk_cost(int tm, int64_t tiles, double k, int64_t rows) {
 // beside: the launch shares the device with other streams' (a step's small buckets). The larger
 // tiles then win over a wider range, since what the launch takes from its neighbours counts, not its
 // own time (four matrices of 2048 x 2048 and two of 8192 x 2048, 128-row SYRK tiles for the former
-// 2% shorter alone: 1.95 ms a step with them, 1.87 without).
+// 2% shorter alone: 1.95 ms a step with them, 1.87 without; one fp32 matrix of 1022 x 1984 and one of
+// 1022 x 1022 beside nine of 1984 x 1022: 780 us with B X of the two on 64-row tiles, 772 on 128).
 //
 // head > 0: the first `head` tiles (whole rounds) on 256-row tiles, the rest, which would leave most
 // CUs idle for a round, cut into tm-row tiles in a second launch (8 us for its fill and the first
@@ -3164,7 +3165,7 @@ static int bx_tile(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t m, in
   const double k = (double)K, far = past_cache(batch * rows * (N + rows) * 4) ? 1.08 : 1.0;
   const double c256 = bx256_cost(n256, k), c128 = far * tile_cost(BX_128, n128, k),
                c64 = far * tile_cost(BX_64, 4 * n128, k);
-  if (c64 < 0.95 * c128 && c64 < c256) return 64;
+  if (c64 < (beside ? 0.65 : 0.95) * c128 && c64 < c256) return 64;
   return c128 < (beside ? 0.5 : 1.0) * c256 ? 128 : 256;
 }
 
