@@ -235,8 +235,8 @@ __global__ __launch_bounds__(256) void short_reduce_kernel(float* part, int P) {
 // 1.02e-2; 16 x 131072 with log-normal rows 2.99e-2 and 2.98e-2, 1.41e-2 and 1.43e-2; 64 x 65536 of rank
 // 8 and a tenth of noise 0.73e-2 and 2.98e-2, 0.29e-2 and 3.71e-2. Over 7 shapes of 8 to 64 rows, three
 // kinds of input and both strategies it is 0.08 to 1.009 times the streaming one's, above 1
-// in two of 42; single inputs differ by 0.7 to 1.4 either way. An error e of G grows by a^2 per iteration in the directions X does not
-// reach; the caller bounds that growth (muon_short_gspace_ok).
+// in two of 42; single inputs differ by 0.7 to 1.4 either way. An error e of G grows by a^2 per
+// iteration in the directions X does not reach; the caller bounds that growth (muon_short_gspace_ok).
 // Wave w owns the 16 x 16 tile (w / 4, w % 4) of every product (fp32 MFMA, 16 x 16 x 4).
 // The matrices live in LDS with a row pitch of 65 words. Q goes out as three bf16 parts
 // (24 significant bits) in the order of short_bx_kernel's fragments.
