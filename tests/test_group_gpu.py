@@ -64,8 +64,8 @@ def test_group_equals_one_bucket_at_a_time(monkeypatch, cls, shapes, kw):
 
 
 def test_large_and_short_buckets_stay_out():
-    """More tiles than the common launches take, and iterates of at most 64 rows, keep their
-    streams."""
+    """More tiles than the common launches take, and iterates of at most 64 rows, stay out of
+    them."""
     def plan(shapes):
         buckets = [(torch.device(DEV, 0), None, [torch.empty(s, device=DEV)], None, None)
                    for s in shapes]
